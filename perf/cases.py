@@ -9,8 +9,9 @@ GPU from a seed.  Kinds:
 - "euler":   the same with the Euler equations;
 - "solve":   a short adaptive advection solve: the tree goes back to its base
              level, the initial field is set, then regrid by the undivided
-             gradient and step, in turn, and the result is read back;
-- "esolve":  the same with the Euler equations and the density criterion;
+             gradient and step, in turn, and the result is read back to the host;
+- "esolve":  the same with the Euler equations and the density criterion, the
+  result left on the GPU;
 - "batch":   an ensemble of independent trees stepped as one batch;
 - "adjoint": a differentiable solve through torch.autograd, forward and
              backward, on a recorded solve.
@@ -321,7 +322,7 @@ def prepare(case, seed):
         else:
             crit = amr.make_criterion(amr.CRITERION_MAX_VALUE, 0.53, 0.49, case["base"], case["top"])
         back = amr.make_criterion(amr.CRITERION_MAX_VALUE, 1e300, 1e300, case["base"], case["top"])
-        state.update(u0=u0.cpu().numpy(), criterion=crit, back=back)
+        state.update(u0=u0.cpu().numpy(), criterion=crit, back=back, capacity=cap)
         return state
     if kind == "adjoint":
         crit = None
@@ -377,7 +378,8 @@ def run(state):
             solver.advance_batch_async(case["every"])
             dt, _ = solver.finish_advance_batch()
             time += dt
-        return {"keys": tree.keys().view(np.int64), "u": tree.get_interior(), "time": time}
+        u = tree.get_interior() if kind == "solve" else _device_view(tree, state["capacity"])
+        return {"keys": tree.keys().view(np.int64), "u": u, "time": time}
     if case["steps"] == 1:
         dt = solver.advance()
     else:
