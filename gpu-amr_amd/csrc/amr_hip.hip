@@ -737,7 +737,9 @@ struct amr_ctx
     // field-major (field v of slot s at u + v * fstride() + s * ni)
     int             nvar  = 1;
     double          gamma = 1.4;
-    euler_scalars*  esc   = nullptr; // device scalars of an Euler batch
+    euler_scalars*  esc   = nullptr; // the kEulerSlots device scalars of the dt logic
+    uint32_t        euler_last = 1;  // slot with the last batch's sums
+    bool            euler_cut  = false; // a launch of the last batch failed: slot 0 may not be empty
     size_t          fstride() const { return static_cast<size_t>(cap) * static_cast<size_t>(ni); }
     bool            euler() const { return nvar > 1; }
 
@@ -923,33 +925,57 @@ struct amr_ctx
         return prm;
     }
 
-    // advance_batch_async: the dt reduction of the batch's first state, then
-    // per step the dt logic and the update, which also folds the next
-    // step's dt minimum over the cells it writes (the values the reduction
-    // would read back, so the same minimum); dt never visits the host.
+    // advance_batch_async: the dt reduction of the batch's first state into
+    // slot 0, then one launch per step, which forms its dt itself
+    // (euler_step_dt) and folds the next step's dt minimum over the cells it
+    // writes (the values the reduction would read back, so the same
+    // minimum); dt never visits the host.  Every batch leaves slot 0 empty,
+    // so that a captured batch can be replayed.
     void euler_advance(uint64_t steps, double remaining)
     {
         ensure_usable();
-        euler_params prm = make_euler_params();
-        hipLaunchKernelGGL(k_euler_begin, dim3(1), dim3(1), 0, stream, esc, remaining);
-        check_launch("k_euler_begin");
-        const uint32_t nn = static_cast<uint32_t>(n);
-        if (steps > 0) op->euler_dt(*op, u[cur], fstride(), keys[kc], prm, esc, nn, stream);
+        if (steps == 0)
+        {
+            euler_clear(1);
+            euler_last = 1;
+            return;
+        }
+        euler_params   prm = make_euler_params();
+        const uint32_t nn  = static_cast<uint32_t>(n);
+        prm.cfl            = cfl;
+        prm.remaining      = remaining;
+        prm.next           = 0;
+        prm.clear          = 1;
+        if (euler_cut) euler_clear(0);
+        euler_cut = true;
+        op->euler_dt(*op, u[cur], fstride(), keys[kc], prm, esc, nn, stream);
         for (uint64_t s = 0; s < steps; ++s)
         {
-            hipLaunchKernelGGL(k_euler_finalize, dim3(1), dim3(1), 0, stream, esc, cfl);
-            check_launch("k_euler_finalize");
-            prm.reverse = static_cast<uint32_t>(sweeps++ & 1);
-            prm.next_dt = s + 1 < steps ? 1u : 0u;
+            prm.reverse  = static_cast<uint32_t>(sweeps++ & 1);
+            prm.next_dt  = s + 1 < steps ? 1u : 0u;
+            prm.now      = s == 0 ? 0u : 1u + static_cast<uint32_t>((s - 1) % 3);
+            prm.next     = 1u + static_cast<uint32_t>(s % 3);
+            prm.clear    = 1u + static_cast<uint32_t>((s + 1) % 3);
+            prm.first    = s == 0 ? 1u : 0u;
+            prm.clear_dt = s == 1 ? 1u : 0u;
             op->euler_step(*op, u[cur], u[1 - cur], fstride(), keys[kc], links, metas, prm, esc, nn, stream);
             cur = 1 - cur;
         }
+        euler_last = prm.next;
+        if (steps == 1) euler_clear(0);
+        euler_cut = false;
     }
 
-    // The Euler batch scalars once every queued operation has finished.
-    euler_scalars euler_read()
+    void euler_clear(uint32_t slot)
     {
-        publish_wait(nullptr, esc);
+        hipLaunchKernelGGL(k_euler_clear, dim3(1), dim3(1), 0, stream, esc + slot);
+        check_launch("k_euler_clear");
+    }
+
+    // The scalars of one slot once every queued operation has finished.
+    euler_scalars euler_read(uint32_t slot)
+    {
+        publish_wait(nullptr, esc + slot);
         return box->esc;
     }
 
@@ -957,11 +983,12 @@ struct amr_ctx
     double euler_dt_now()
     {
         ensure_usable();
-        const euler_params prm = make_euler_params();
-        hipLaunchKernelGGL(k_euler_begin, dim3(1), dim3(1), 0, stream, esc, 0.0);
-        check_launch("k_euler_begin");
+        euler_params prm = make_euler_params();
+        euler_clear(kEulerNowSlot);
+        prm.next = kEulerNowSlot;
+        prm.clear = 3; // free outside a batch's steps
         op->euler_dt(*op, u[cur], fstride(), keys[kc], prm, esc, static_cast<uint32_t>(n), stream);
-        const euler_scalars e = euler_read();
+        const euler_scalars e = euler_read(kEulerNowSlot);
         double raw;
         std::memcpy(&raw, &e.dtmin_bits, sizeof(raw));
         return cfl * raw;
@@ -1701,7 +1728,8 @@ int amr_euler_create(const amr_tree_config* cfg, double gamma, double cfl, amr_c
             auto c   = create_ctx(cfg, cfg->rank + 2);
             c->gamma = gamma;
             c->cfl   = cfl;
-            c->esc   = dev_alloc<euler_scalars>(1);
+            c->esc   = dev_alloc<euler_scalars>(kEulerSlots);
+            for (uint32_t k = 0; k < kEulerSlots; ++k) c->euler_clear(k);
             *out = c.release();
         }
     );
@@ -2171,7 +2199,7 @@ int amr_solver_finish_advance_batch(amr_ctx* ctx, double* dt_sum, uint64_t* exec
             if (!ctx) throw amr_error(AMR_ERR_ARGUMENT, "null argument");
             if (ctx->euler())
             {
-                const euler_scalars e = ctx->euler_read();
+                const euler_scalars e = ctx->euler_read(ctx->euler_last);
                 ctx->pending_dt       = e.acc;
                 ctx->pending_steps    = e.executed;
             }
