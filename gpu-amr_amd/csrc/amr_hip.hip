@@ -339,25 +339,67 @@ ops const* find_ops(int rank, int n, int h)
 // 64 threads for patches of up to 64 cells and 256 otherwise.  They read
 // neighbour cells from memory instead of LDS tiles; the arithmetic is the
 // fixed-shape kernels', so results are the same bits.
+constexpr size_t kBoxTileBytes = 64 * 1024; // largest LDS tile of the any-shape kernels
+
 template <int R>
 struct box_instance
 {
-    static box<R> shape(ops const& o) { return box<R>{ { o.ext[0], o.ext[1], o.ext[2] } }; }
-    static bool   small(ops const& o) { return o.ni() <= 64; }
+    static launch_box<R>       shape(ops const& o) { return launch_box<R>::of(o.ext); }
+    static launch_box<R, true> small_shape(ops const& o) { return launch_box<R, true>::of(o.ext); }
 
     static int         variant_count() { return 1; }
     static char const* variant_name(int) { return "box"; }
     static int         variant_needs(int) { return 0; }
+
+    // The walk of a patch (box_walk) and its workgroup size: the one of 64,
+    // 128, 256 (512 from 2048 cells on) threads that spends the fewest thread
+    // slots in at most four passes, the smaller one of equals, else the
+    // largest.  0 when a layer has more cells than the largest workgroup.
+    static int walk_for(ops const& o, box_walk& W)
+    {
+        const int cols = o.ni() / o.ext[0], most = o.ni() >= 2048 ? 512 : 256;
+        int       best = 0, slots = 0;
+        for (int nt = 64; nt <= most; nt *= 2)
+        {
+            if (cols > nt) continue;
+            const int layers = std::min(nt / cols, static_cast<int>(o.ext[0]));
+            const int passes = (o.ext[0] + layers - 1) / layers;
+            if (best && (passes * nt >= slots) && !(W.passes > 4)) continue;
+            best  = nt;
+            slots = passes * nt;
+            W     = box_walk{ layers, passes };
+        }
+        return best;
+    }
+
+    // LDS of one tile of nv fields
+    static size_t tile_bytes(ops const& o, int nv)
+    {
+        return static_cast<size_t>(nv) * box_tile<R>::cells(shape(o)) * sizeof(double);
+    }
 
     static void step(ops const& o, int, const double* u, double* un, const uint64_t* keys, const face_link* links,
                      const uint32_t* metas, step_params const& prm, const step_params* table, const uint16_t* inst,
                      uint32_t n, step_aux const&, hipStream_t s)
     {
         if (n == 0) return;
-        const dim3 grid(xcd_grid(n));
-        if (small(o))
-            hipLaunchKernelGGL((k_step_box<R, 64>), grid, dim3(64), 0, s, shape(o), u, un, keys, links, metas, prm,
-                               table, inst, n);
+        const dim3   grid(xcd_grid(n));
+        const size_t lds = tile_bytes(o, 1);
+        box_walk     W;
+        const int    nt  = lds <= kBoxTileBytes ? walk_for(o, W) : 0;
+        auto         go  = [&](auto threads) {
+            constexpr int NT = decltype(threads)::value;
+            hipLaunchKernelGGL((k_step_box_tile<R, NT, 4>), grid, dim3(NT), lds, s, small_shape(o), W, u, un, keys, links,
+                               metas, prm, table, inst, n);
+        };
+        if (nt == 64)
+            go(std::integral_constant<int, 64>{});
+        else if (nt == 128)
+            go(std::integral_constant<int, 128>{});
+        else if (nt == 256)
+            go(std::integral_constant<int, 256>{});
+        else if (nt == 512)
+            go(std::integral_constant<int, 512>{});
         else
             hipLaunchKernelGGL((k_step_box<R, 256>), grid, dim3(256), 0, s, shape(o), u, un, keys, links, metas, prm,
                                table, inst, n);

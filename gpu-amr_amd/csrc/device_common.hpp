@@ -28,7 +28,7 @@ enum : uint32_t
 //   ids[4]: same/coarser -> ids[0] = neighbour slot; finer -> the 2^(rank-1)
 //           fine slots little-endian over the non-normal layout dims.
 //   meta:   bits 0-1 relation, bit 2+d = contact quadrant of layout dim d.
-struct face_link
+struct alignas(16) face_link
 {
     int32_t ids[4];
 };
@@ -125,8 +125,20 @@ struct box
     __host__ __device__ constexpr int n(int d) const { return e[d]; }
     __host__ __device__ constexpr int half(int d) const { return e[d] / 2; }
     __host__ __device__ constexpr int ni() const { return (R == 2) ? e[0] * e[1] : e[0] * e[1] * e[2]; }
+    // the half of dim d that holds coordinate v in [0, n(d)), v's offset in
+    // it, and the first fine cell under v in a fine patch: (2 v) mod n(d)
+    __host__ __device__ constexpr int half_of(int v, int d) const { return v >= half(d) ? 1 : 0; }
+    __host__ __device__ constexpr int in_half(int v, int d) const { return v >= half(d) ? v - half(d) : v; }
+    __host__ __device__ constexpr int fine(int v, int d) const { return 2 * in_half(v, d); }
     // cells of a face normal to layout dim `dim`
-    __host__ __device__ constexpr int face(int dim) const { return ni() / e[dim]; }
+    __host__ __device__ constexpr int face(int dim) const
+    {
+        int f = 1;
+        for (int d = 0; d < R; ++d) f *= d == dim ? 1 : e[d];
+        return f;
+    }
+    // l / n(d) for 0 <= l < ni()
+    __host__ __device__ constexpr int quot(int l, int d) const { return l / e[d]; }
     // stride of layout dim d in the compact interior
     __host__ __device__ constexpr int stride(int d) const
     {
@@ -154,6 +166,44 @@ struct box
         int p = 1;
         for (int d = 0; d < R; ++d) p *= e[d] + 2 * h;
         return p;
+    }
+};
+
+// The box of a launch of the any-shape kernels: the extents with the
+// multipliers m[d] = ceil(2^32 / n(d)), so that a division by an extent is
+// one 32-bit multiply (an integer division by a launch argument takes some
+// twenty instructions).  l m = l 2^32 / n + l r / n with r < n, so the high
+// word is the quotient while l n < 2^32; larger patches keep m[d] = 0 and
+// divide.  SMALL: the multipliers are there (patches whose tile fits in LDS).
+template <int R, bool SMALL = false>
+struct launch_box : box<R>
+{
+    uint32_t m[3];
+
+    static launch_box of(const int32_t* ext)
+    {
+        launch_box b{};
+        for (int d = 0; d < 3; ++d) b.e[d] = ext[d];
+        for (int d = 0; d < R; ++d)
+        {
+            const uint64_t n = static_cast<uint64_t>(ext[d]);
+            const bool     fits = static_cast<uint64_t>(b.ni()) * n < (uint64_t{ 1 } << 32);
+            b.m[d]           = fits ? static_cast<uint32_t>(((uint64_t{ 1 } << 32) + n - 1) / n) : 0u;
+        }
+        return b;
+    }
+    __host__ __device__ int quot(int l, int d) const
+    {
+        return SMALL || m[d] ? static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(l)) * m[d]) >> 32) : l / this->e[d];
+    }
+    __host__ __device__ void coords(int l, int* c) const
+    {
+        for (int d = R - 1; d >= 0; --d)
+        {
+            const int q = quot(l, d);
+            c[d]        = l - q * this->e[d];
+            l           = q;
+        }
     }
 };
 

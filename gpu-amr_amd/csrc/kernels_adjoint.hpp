@@ -43,8 +43,8 @@ struct adjoint_params
 };
 
 // In-patch part of (A^T lambda')_c.
-template <int R>
-__host__ __device__ inline double adj_interior(box<R> const& B, const double* __restrict__ lam, int i,
+template <int R, class BX>
+__host__ __device__ inline double adj_interior(BX const& B, const double* __restrict__ lam, int i,
                                                const double* dtdx, const double* vp, const double* vm)
 {
     int c[R];
@@ -80,8 +80,8 @@ __host__ __device__ inline double adj_interior(const double* __restrict__ lam, i
 // The neighbour's boundary cell reads its ghost on side dir^1 with
 // coefficient dt/dx vp (ghost is its u_L, dir positive) or -dt/dx vm (ghost
 // is its u_R, dir negative), at the neighbour's own level.
-template <int R>
-__host__ __device__ inline double adj_face_term(box<R> const& B, const double* __restrict__ lam, const face_link& L,
+template <int R, class BX>
+__host__ __device__ inline double adj_face_term(BX const& B, const double* __restrict__ lam, const face_link& L,
                                                 uint32_t meta, int dir, const int* c, int level,
                                                 const adjoint_params& prm)
 {
@@ -108,9 +108,9 @@ __host__ __device__ inline double adj_face_term(box<R> const& B, const double* _
                     base[k] = nb;
                     continue;
                 }
-                kid |= (c[k] / B.half(k)) << bit;
+                kid |= B.half_of(c[k], k) << bit;
                 ++bit;
-                base[k] = (c[k] % B.half(k)) * 2;
+                base[k] = B.fine(c[k], k);
             }
             const double* q   = lam + static_cast<size_t>(L.ids[kid]) * B.ni();
             double        sum = 0.0;
@@ -183,8 +183,8 @@ __host__ __device__ inline void adj_velocity_cell(const double* tile, int i, dou
 }
 
 // adj_velocity_cell with the neighbours read from memory (any patch shape).
-template <int R>
-__host__ __device__ inline void adj_velocity_cell_direct(box<R> const& B, const double* __restrict__ u, uint32_t leaf,
+template <int R, class BX>
+__host__ __device__ inline void adj_velocity_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
                                                          const face_link* __restrict__ links,
                                                          const uint32_t* __restrict__ metas, int i, double lam_c,
                                                          const double* dtdx, const double* sgn, double* acc)
@@ -205,8 +205,8 @@ __host__ __device__ inline void adj_velocity_cell_direct(box<R> const& B, const 
 }
 
 // Face index of tangential coordinates c (dims other than dim), row-major.
-template <int R>
-__host__ __device__ inline int face_index(box<R> const& B, const int* c, int dim)
+template <int R, class BX>
+__host__ __device__ inline int face_index(BX const& B, const int* c, int dim)
 {
     int f = 0;
     for (int k = 0; k < R; ++k)
@@ -222,8 +222,8 @@ __host__ __device__ inline int face_index(const int* c, int dim)
 }
 
 // Tangential coordinates of face index f of direction dir (c[dim] = 0).
-template <int R>
-__host__ __device__ inline void face_coords(box<R> const& B, int f, int dir, int* c)
+template <int R, class BX>
+__host__ __device__ inline void face_coords(BX const& B, int f, int dir, int* c)
 {
     const int dim = dir >> 1;
     for (int k = R - 1; k >= 0; --k)
@@ -233,8 +233,9 @@ __host__ __device__ inline void face_coords(box<R> const& B, int f, int dir, int
             c[k] = 0;
             continue;
         }
-        c[k] = f % B.n(k);
-        f /= B.n(k);
+        const int q = B.quot(f, k);
+        c[k]        = f - q * B.n(k);
+        f           = q;
     }
 }
 
@@ -268,8 +269,8 @@ __host__ __device__ inline double adj_cell(const double* __restrict__ lam, const
 
 // adj_cell with lambda' and the transposed halo terms read from memory (any
 // patch shape; the terms are added in adj_cell's order, so the same bits).
-template <int R>
-__host__ __device__ inline double adj_cell_direct(box<R> const& B, const double* __restrict__ lam_next, uint32_t leaf,
+template <int R, class BX>
+__host__ __device__ inline double adj_cell_direct(BX const& B, const double* __restrict__ lam_next, uint32_t leaf,
                                                   const face_link* __restrict__ L, const uint32_t* __restrict__ M,
                                                   int i, int level, const adjoint_params& prm, const double* dtdx,
                                                   const double* vp, const double* vm)
@@ -289,16 +290,16 @@ __host__ __device__ inline double adj_cell_direct(box<R> const& B, const double*
 
 // Transposed regrid transfer, value of cell t of old leaf i.
 // Refined leaf: sum of lambda over the 2^R fine cells injected from t.
-template <int R>
-__host__ __device__ inline double adj_refine_value(box<R> const& B, const double* __restrict__ lam_new,
+template <int R, class BX>
+__host__ __device__ inline double adj_refine_value(BX const& B, const double* __restrict__ lam_new,
                                                    uint32_t first_child, int t)
 {
     int tc[R], base[R], kid = 0;
     B.coords(t, tc);
     for (int d = 0; d < R; ++d)
     {
-        kid |= (tc[d] / B.half(d)) << (R - 1 - d);
-        base[d] = (tc[d] % B.half(d)) * 2;
+        kid |= B.half_of(tc[d], d) << (R - 1 - d);
+        base[d] = B.fine(tc[d], d);
     }
     const double* q   = lam_new + static_cast<size_t>(first_child + kid) * B.ni();
     double        sum = 0.0;
@@ -313,8 +314,8 @@ __host__ __device__ inline double adj_refine_value(box<R> const& B, const double
 
 // Coarsened family: cell f of child kid receives lambda of the parent cell
 // that averaged it, divided by 2^R.
-template <int R>
-__host__ __device__ inline double adj_restrict_value(box<R> const& B, const double* __restrict__ lam_parent, int kid,
+template <int R, class BX>
+__host__ __device__ inline double adj_restrict_value(BX const& B, const double* __restrict__ lam_parent, int kid,
                                                      int f)
 {
     int fc[R], t[R];
@@ -417,8 +418,8 @@ __global__ __launch_bounds__(NT) void k_adj_step(const double* __restrict__ lam_
 
 // Transposed regrid transfer of old leaf i (one workgroup; mark / head /
 // counts / pos recorded by the forward regrid).
-template <int R, int NT>
-__device__ inline void adj_regrid_leaf(box<R> const& B, const double* __restrict__ lam_new,
+template <int R, int NT, class BX>
+__device__ inline void adj_regrid_leaf(BX const& B, const double* __restrict__ lam_new,
                                        const uint8_t* __restrict__ mark, const uint8_t* __restrict__ head,
                                        const uint32_t* __restrict__ counts, const uint32_t* __restrict__ pos,
                                        double* __restrict__ lam_old, uint32_t i)
@@ -461,7 +462,7 @@ __global__ __launch_bounds__(NT) void k_adj_regrid(const double* __restrict__ la
 
 // k_adj_regrid for patches of any shape.
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_adj_regrid_box(box<R> B, const double* __restrict__ lam_new,
+__global__ __launch_bounds__(NT) void k_adj_regrid_box(launch_box<R> B, const double* __restrict__ lam_new,
                                                        const uint8_t* __restrict__ mark,
                                                        const uint8_t* __restrict__ head,
                                                        const uint32_t* __restrict__ counts,
@@ -476,7 +477,7 @@ __global__ __launch_bounds__(NT) void k_adj_regrid_box(box<R> B, const double* _
 // k_adj_step for patches of any shape: lambda', u and the transposed halo
 // terms read from memory (the operands and sums of k_adj_step).
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_adj_step_box(box<R> B, const double* __restrict__ lam_next,
+__global__ __launch_bounds__(NT) void k_adj_step_box(launch_box<R> B, const double* __restrict__ lam_next,
                                                      const double* __restrict__ u, const uint64_t* __restrict__ keys,
                                                      const face_link* __restrict__ links,
                                                      const uint32_t* __restrict__ metas,

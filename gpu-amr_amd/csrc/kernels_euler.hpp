@@ -147,8 +147,8 @@ struct euler_flux
 // once and the source cells of every field are loaded together.  Each
 // field's arithmetic (the copy, the injection, the fine mean summed from 0.0
 // in row-major order) is ghost_value's, so the values are the same bits.
-template <int R, int NV>
-__device__ inline void ghost_values(box<R> const& B, const double* __restrict__ u, size_t fstride,
+template <int R, int NV, class BX>
+__device__ inline void ghost_values(BX const& B, const double* __restrict__ u, size_t fstride,
                                     const face_link& L, uint32_t meta, int dir, const int* c, double* out)
 {
     const uint32_t rel = rel_of(meta);
@@ -169,10 +169,10 @@ __device__ inline void ghost_values(box<R> const& B, const double* __restrict__ 
     for (int d = 0; d < R; ++d)
     {
         const int w = (d == dim) ? nrm : c[d];
-        base[d]     = (w * 2) % B.n(d);
+        base[d]     = B.fine(w, d);
         if (d != dim)
         {
-            k |= (c[d] / B.half(d)) << bit;
+            k |= B.half_of(c[d], d) << bit;
             ++bit;
         }
     }
@@ -200,8 +200,8 @@ __device__ inline void ghost_values(const double* __restrict__ u, size_t fstride
 // The NV values of the cell with layout coordinates c of `leaf`: interior
 // cells from the leaf, ghost cells (one coordinate just outside) through
 // the ghost rules.
-template <int R>
-__device__ inline void euler_cell(box<R> const& B, const double* __restrict__ u, size_t fstride, uint32_t leaf,
+template <int R, class BX>
+__device__ inline void euler_cell(BX const& B, const double* __restrict__ u, size_t fstride, uint32_t leaf,
                                   const face_link* __restrict__ links, const uint32_t* __restrict__ metas, const int* c,
                                   double* U)
 {
@@ -324,8 +324,8 @@ __device__ inline void fold_speed_max(double* smax, const double* cs, euler_scal
 // and dims of dx_d / speed (speed > 1e-12), folded into the launch-wide
 // minimum.  The minimum is exact and order-free, so any reduction order
 // gives the oracle's value.
-template <int R, int NT>
-__device__ inline void euler_dt_leaf(box<R> const& B, const double* __restrict__ u, size_t fstride,
+template <int R, int NT, class BX>
+__device__ inline void euler_dt_leaf(BX const& B, const double* __restrict__ u, size_t fstride,
                                      const uint64_t* __restrict__ keys, euler_params const& prm,
                                      euler_scalars* sc, uint32_t leaf)
 {
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(NT) void k_euler_dt(const double* __restrict__ u, s
 
 // k_euler_dt for patches of any shape.
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_euler_dt_box(box<R> B, const double* __restrict__ u, size_t fstride,
+__global__ __launch_bounds__(NT) void k_euler_dt_box(launch_box<R> B, const double* __restrict__ u, size_t fstride,
                                                      const uint64_t* __restrict__ keys, euler_params prm,
                                                      euler_scalars* sc, uint32_t nleaves)
 {
@@ -413,8 +413,8 @@ __global__ void k_euler_clear(euler_scalars* __restrict__ slot)
 // total[k] -= dt / dx_d * (fR[k] - fL[k]); out = U + total.  A step the dt
 // logic stopped copies the state (the CPU loop runs no step).  Neighbours
 // are read from memory.
-template <int R, int NT>
-__device__ inline void euler_step_leaf(box<R> const& B, const double* __restrict__ u, double* __restrict__ un,
+template <int R, int NT, class BX>
+__device__ inline void euler_step_leaf(BX const& B, const double* __restrict__ u, double* __restrict__ un,
                                        size_t fstride, const uint64_t* __restrict__ keys,
                                        const face_link* __restrict__ links, const uint32_t* __restrict__ metas,
                                        euler_params const& prm, euler_scalars* sc, double dt, uint32_t leaf)
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(NT) void k_euler_step(const double* __restrict__ u,
 
 // k_euler_step for patches of any shape.
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_euler_step_box(box<R> B, const double* __restrict__ u, double* __restrict__ un,
+__global__ __launch_bounds__(NT) void k_euler_step_box(launch_box<R> B, const double* __restrict__ u, double* __restrict__ un,
                                                        size_t fstride, const uint64_t* __restrict__ keys,
                                                        const face_link* __restrict__ links,
                                                        const uint32_t* __restrict__ metas, euler_params prm,

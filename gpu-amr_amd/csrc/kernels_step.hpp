@@ -13,6 +13,8 @@
 
 #include "device_common.hpp"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace amrhip
@@ -77,8 +79,8 @@ __device__ inline const step_params& params_for(const step_params& prm, const st
 // Its CPU rule reduces every dim mod n(dim) of the face normal
 // (patch_utils.hpp:358), the same for square patches only; for other shapes
 // that rule addresses cells outside the fine patch's interior.
-template <int R>
-__host__ __device__ inline double ghost_value(box<R> const& B, const double* __restrict__ u, const face_link& L,
+template <int R, class BX>
+__host__ __device__ inline double ghost_value(BX const& B, const double* __restrict__ u, const face_link& L,
                                               uint32_t meta, int dir, const int* c)
 {
     const int  dim = dir >> 1;
@@ -105,10 +107,10 @@ __host__ __device__ inline double ghost_value(box<R> const& B, const double* __r
             for (int d = 0; d < R; ++d)
             {
                 const int v = (d == dim) ? nrm : c[d];
-                base[d]     = (v * 2) % B.n(d);
+                base[d]     = B.fine(v, d);
                 if (d != dim)
                 {
-                    k |= (c[d] / B.half(d)) << bit;
+                    k |= B.half_of(c[d], d) << bit;
                     ++bit;
                 }
             }
@@ -195,8 +197,8 @@ __host__ __device__ inline void stage_ghost(double* tile, const double* __restri
 // Index into u of the one interior cell that gives the ghost value of cell c
 // when the direction-`dir` neighbour (slot nb) is same-level (copy) or
 // coarser (injection): ghost_value's single-cell rules.
-template <int R>
-__host__ __device__ inline size_t ghost_source(box<R> const& B, int32_t nb, uint32_t meta, int dir, const int* c)
+template <int R, class BX>
+__host__ __device__ inline size_t ghost_source(BX const& B, int32_t nb, uint32_t meta, int dir, const int* c)
 {
     const int  dim    = dir >> 1;
     const int  nrm    = (dir & 1) ? c[dim] - B.n(dim) : c[dim] + B.n(dim);
@@ -219,8 +221,8 @@ __host__ __device__ inline size_t ghost_source(int32_t nb, uint32_t meta, int di
 
 // Value of cell c of `leaf` (layout coordinates, at most one of them outside
 // the patch): the interior cell, or the ghost value by the face rules.
-template <int R>
-__host__ __device__ inline double cell_or_ghost(box<R> const& B, const double* __restrict__ u, uint32_t leaf,
+template <int R, class BX>
+__host__ __device__ inline double cell_or_ghost(BX const& B, const double* __restrict__ u, uint32_t leaf,
                                                 const face_link* __restrict__ links,
                                                 const uint32_t* __restrict__ metas, const int* c)
 {
@@ -466,8 +468,8 @@ __host__ __device__ inline double gradient_cell(const double* tile, int i)
 
 // Cell i of the padded view ((n(d) + 2h) per dim, row-major): interior copy,
 // face halo gathered; *kind = 0 interior, 1 face halo, 2 edge/corner (value 0).
-template <int R>
-__host__ __device__ inline double padded_value(box<R> const& B, int h, const double* __restrict__ u, uint32_t leaf,
+template <int R, class BX>
+__host__ __device__ inline double padded_value(BX const& B, int h, const double* __restrict__ u, uint32_t leaf,
                                                const face_link* __restrict__ links,
                                                const uint32_t* __restrict__ metas, int i, int* kind)
 {
@@ -506,8 +508,8 @@ __host__ __device__ inline double padded_value(const double* __restrict__ u, uin
 // The upwind update of interior cell i of `leaf` with its neighbours read
 // from memory (interior cells, or ghost values at the patch boundary): the
 // same operands as upwind_cell on a staged tile, for patches of any shape.
-template <int R>
-__host__ __device__ inline double upwind_cell_direct(box<R> const& B, const double* __restrict__ u, uint32_t leaf,
+template <int R, class BX>
+__host__ __device__ inline double upwind_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
                                                      const face_link* __restrict__ links,
                                                      const uint32_t* __restrict__ metas, int i, const double* dtdx,
                                                      const double* vel, const double* hs)
@@ -528,8 +530,8 @@ __host__ __device__ inline double upwind_cell_direct(box<R> const& B, const doub
 }
 
 // gradient_cell with the neighbours read from memory (any patch shape).
-template <int R>
-__host__ __device__ inline double gradient_cell_direct(box<R> const& B, const double* __restrict__ u, uint32_t leaf,
+template <int R, class BX>
+__host__ __device__ inline double gradient_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
                                                        const face_link* __restrict__ links,
                                                        const uint32_t* __restrict__ metas, int i)
 {
@@ -569,6 +571,294 @@ __device__ inline void stage_tile(double* tile, const double* __restrict__ u, ui
     const double* up = u + static_cast<size_t>(leaf) * S::NI;
     for (int i = threadIdx.x; i < S::NI; i += NT) stage_interior<R, N>(tile, up, i);
     for (int g = threadIdx.x; g < S::NDIR * S::FACE; g += NT) stage_ghost<R, N>(tile, u, leaf, links, metas, g);
+}
+
+// ---------------------------------------------------------------------------
+// LDS tiles of patches whose extents are launch arguments: the patch plus one
+// ghost layer, (n(d) + 2) cells per dim, row-major.
+// ---------------------------------------------------------------------------
+template <int R>
+struct box_tile
+{
+    int st[R]; // stride of layout dim d
+
+    template <class BX>
+    __host__ __device__ explicit box_tile(BX const& B)
+    {
+        st[R - 1] = 1;
+        for (int d = R - 1; d > 0; --d) st[d - 1] = st[d] * (B.n(d) + 2);
+    }
+    __host__ __device__ int idx(const int* c) const
+    {
+        int l = 0;
+        for (int d = 0; d < R; ++d) l += (c[d] + 1) * st[d];
+        return l;
+    }
+    template <class BX>
+    __host__ __device__ static int cells(BX const& B)
+    {
+        int l = 1;
+        for (int d = 0; d < R; ++d) l *= B.n(d) + 2;
+        return l;
+    }
+};
+
+// Ghost item g (0 <= g < 2 face(D)) of the two faces normal to layout dim D:
+// its cell c, and the side (0 negative, 1 positive).  D is a constant, so the
+// coordinates stay in registers.
+template <int R, int D, class BX>
+__host__ __device__ inline int face_pair_item(BX const& B, int g, int* c)
+{
+    const int fc = B.face(D), side = g >= fc ? 1 : 0, f = side ? g - fc : g;
+    if constexpr (R == 2)
+        c[1 - D] = f;
+    else
+    {
+        constexpr int hi = D == 0 ? 1 : 0, lo = D == 2 ? 1 : 2;
+        c[hi]            = B.quot(f, lo);
+        c[lo]            = f - c[hi] * B.n(lo);
+    }
+    c[D] = side ? B.n(D) : -1;
+    return side;
+}
+
+// ghost_source for a face normal to the constant dim D.
+template <int R, int D, class BX>
+__host__ __device__ inline size_t face_source(BX const& B, int32_t nb, uint32_t meta, int side, const int* c)
+{
+    const bool coarse = rel_of(meta) == REL_COARSER;
+    int        cc[R];
+    for (int d = 0; d < R; ++d)
+    {
+        const int v = (d == D) ? (side ? c[D] - B.n(D) : c[D] + B.n(D)) : c[d];
+        cc[d]       = coarse ? static_cast<int>(quad_of(meta, d)) * B.half(d) + v / 2 : v;
+    }
+    return static_cast<size_t>(nb) * B.ni() + B.lin(cc);
+}
+
+// First of the 2^R fine cells under ghost cell c of a face normal to D with
+// finer neighbours ids (a vector, whose elements a select picks: an array
+// indexed by a lane's value would live in scratch memory).
+template <int R, int D, class BX>
+__device__ inline size_t face_fine_source(BX const& B, int4 ids, int side, const int* c)
+{
+    int k = 0, bit = 0, cc[R];
+    for (int d = 0; d < R; ++d)
+    {
+        cc[d] = B.fine((d == D) ? (side ? c[D] - B.n(D) : c[D] + B.n(D)) : c[d], d);
+        if (d != D)
+        {
+            k |= B.half_of(c[d], d) << bit;
+            ++bit;
+        }
+    }
+    int32_t nb = (k & 1) ? ids.y : ids.x;
+    if constexpr (R == 3) nb = (k & 2) ? ((k & 1) ? ids.w : ids.z) : nb;
+    return static_cast<size_t>(nb) * B.ni() + B.lin(cc);
+}
+
+__device__ inline int4 link_ids(const face_link* __restrict__ L) { return *reinterpret_cast<const int4*>(L); }
+
+// Offset of the o-th of those cells (row-major) from the first.
+template <int R, class BX>
+__host__ __device__ inline int fine_offset(BX const& B, int o)
+{
+    int l = 0;
+    for (int d = 0; d < R; ++d) l += ((o >> (R - 1 - d)) & 1) * B.stride(d);
+    return l;
+}
+
+// The NV values of the face-ghost cell c (fields fstride apart) of a face with
+// record (L, meta) by ghost_value's rules.
+template <int R, int NV, int D, class BX>
+__device__ inline void face_values(BX const& B, const double* __restrict__ u, size_t fstride, int4 L, uint32_t meta,
+                                   int side, const int* c, double* out)
+{
+    if (rel_of(meta) != REL_FINER)
+    {
+        const size_t at = face_source<R, D>(B, L.x, meta, side, c);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) out[v] = u[v * fstride + at];
+        return;
+    }
+    const size_t first = face_fine_source<R, D>(B, L, side, c);
+    double       sum[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) sum[v] = 0.0;
+#pragma unroll
+    for (int o = 0; o < (1 << R); ++o)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sum[v] += u[v * fstride + first + fine_offset<R>(B, o)];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) out[v] = sum[v] / static_cast<double>(1 << R);
+}
+
+// How a workgroup of NT threads walks the cells of a patch: `layers` layers of
+// layout dim 0 at a time, one cell per thread, so that a thread keeps its
+// column (the other coordinates) and steps along dim 0 with two additions per
+// cell; `passes` times.  Chosen on the host (box_walk_for).
+struct box_walk
+{
+    int32_t layers, passes;
+};
+
+// One thread's walk: active while k < passes and cell(k) is in the patch.
+template <int R>
+struct box_column
+{
+    int  i0, di; // patch cell of pass 0, step per pass
+    int  t0, dt; // the same in the tile
+    int  z0, dz; // layer
+    bool on;
+
+    template <class BX>
+    __device__ box_column(BX const& B, box_tile<R> const& T, box_walk const& W)
+    {
+        const int cols = B.face(0), tid = threadIdx.x;
+        di             = W.layers * cols;
+        on             = tid < di;
+        i0             = on ? tid : 0;
+        dz             = W.layers;
+        dt             = dz * T.st[0];
+        int c[R];
+        B.coords(i0, c); // W.layers <= n(0): a cell of the patch
+        z0 = c[0];
+        t0 = T.idx(c);
+    }
+};
+
+// Stages every field's tile of `leaf` (field v at tile + v * cells): the
+// patch and its face ghosts, edges and corners untouched.  Bound by the two
+// dependent loads of a ghost (its face record, then its cell), so the first
+// NT items of each face pair and CH cells per thread are loaded before any is
+// stored, the face pairs starting on different waves.
+template <int R, int NT, int NV, int CH, class BX>
+__device__ inline void stage_box(BX const& B, box_tile<R> const& T, box_column<R> const& col, box_walk const& W,
+                                 double* tile, const double* __restrict__ u, size_t fstride, uint32_t leaf,
+                                 const face_link* __restrict__ links, const uint32_t* __restrict__ metas)
+{
+    const int        cells = box_tile<R>::cells(B), tid = threadIdx.x;
+    const double*    own   = u + static_cast<size_t>(leaf) * B.ni();
+    const face_link* L     = links + static_cast<size_t>(leaf) * box<R>::NDIR;
+    const uint32_t*  M     = metas + static_cast<size_t>(leaf) * box<R>::NDIR;
+    // this thread's first ghost item of each face pair and its record
+    int      gc[R][R], item[R], side[R];
+    uint32_t meta[R];
+    int4     link[R];
+    auto     first_item = [&](auto dim) {
+        constexpr int D     = decltype(dim)::value;
+        constexpr int shift = (D * NT / R) / 64 * 64;
+        item[D]             = (tid + NT - shift) % NT;
+        const bool on       = item[D] < 2 * B.face(D);
+        side[D]             = face_pair_item<R, D>(B, on ? item[D] : 0, gc[D]);
+        meta[D]             = M[2 * D + side[D]];
+        link[D]             = link_ids(L + 2 * D + side[D]);
+    };
+    first_item(std::integral_constant<int, 0>{});
+    first_item(std::integral_constant<int, 1>{});
+    if constexpr (R == 3) first_item(std::integral_constant<int, 2>{});
+    double r[CH][NV];
+    auto   load_cells = [&](int k0) {
+#pragma unroll
+        for (int k = 0; k < CH; ++k)
+        {
+            const int i = col.z0 + (k0 + k) * col.dz < B.n(0) ? col.i0 + (k0 + k) * col.di : col.i0;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) r[k][v] = own[v * fstride + i];
+        }
+    };
+    auto store_cells = [&](int k0) {
+#pragma unroll
+        for (int k = 0; k < CH; ++k)
+            if (col.on && col.z0 + (k0 + k) * col.dz < B.n(0))
+            {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) tile[v * cells + col.t0 + (k0 + k) * col.dt] = r[k][v];
+            }
+    };
+    load_cells(0);
+    // single-cell ghosts of every face pair at once, then, in a wave that
+    // has finer neighbours, the 2^R fine cells (the cells of all face pairs
+    // at once took 84 instead of 60 registers in 3D and was 4 % slower)
+    size_t at[R];
+    at[0] = face_source<R, 0>(B, link[0].x, meta[0], side[0], gc[0]);
+    at[1] = face_source<R, 1>(B, link[1].x, meta[1], side[1], gc[1]);
+    if constexpr (R == 3) at[2] = face_source<R, 2>(B, link[2].x, meta[2], side[2], gc[2]);
+    double g[R][NV];
+    bool   fine[R], any_fine = false;
+#pragma unroll
+    for (int d = 0; d < R; ++d)
+    {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) g[d][v] = u[v * fstride + at[d]];
+        fine[d]  = rel_of(meta[d]) == REL_FINER;
+        any_fine = any_fine || fine[d];
+    }
+    if (__any(any_fine))
+    {
+        at[0] = fine[0] ? face_fine_source<R, 0>(B, link[0], side[0], gc[0]) : at[0];
+        at[1] = fine[1] ? face_fine_source<R, 1>(B, link[1], side[1], gc[1]) : at[1];
+        if constexpr (R == 3) at[2] = fine[2] ? face_fine_source<R, 2>(B, link[2], side[2], gc[2]) : at[2];
+        constexpr int F = 1 << R;
+#pragma unroll
+        for (int d = 0; d < R; ++d)
+            if (fine[d])
+            {
+                double sum[NV];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) sum[v] = 0.0;
+#pragma unroll
+                for (int o = 0; o < F; ++o)
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) sum[v] += u[v * fstride + at[d] + fine_offset<R>(B, o)];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) g[d][v] = sum[v] / static_cast<double>(F);
+            }
+    }
+    store_cells(0);
+#pragma unroll
+    for (int d = 0; d < R; ++d)
+        if (item[d] < 2 * B.face(d))
+        {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) tile[v * cells + T.idx(gc[d])] = g[d][v];
+        }
+    // what is left of larger patches
+    for (int k = CH; k < W.passes; k += CH)
+    {
+        load_cells(k);
+        store_cells(k);
+    }
+    auto rest = [&](auto dim) {
+        constexpr int D = decltype(dim)::value;
+        for (int q = item[D] + NT; q < 2 * B.face(D); q += NT)
+        {
+            int       c[R];
+            const int sd = face_pair_item<R, D>(B, q, c);
+            double    w[NV];
+            face_values<R, NV, D>(B, u, fstride, link_ids(L + 2 * D + sd), M[2 * D + sd], sd, c, w);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) tile[v * cells + T.idx(c)] = w[v];
+        }
+    };
+    rest(std::integral_constant<int, 0>{});
+    rest(std::integral_constant<int, 1>{});
+    if constexpr (R == 3) rest(std::integral_constant<int, 2>{});
+}
+
+// Upwind update of tile cell t from a staged tile.
+template <int R>
+__device__ inline double upwind_tile_cell(const double* tile, box_tile<R> const& T, int t, const double* dtdx,
+                                          const double* vel, const double* hs)
+{
+    double lo[R], hi[R];
+#pragma unroll
+    for (int d = 0; d < R; ++d)
+    {
+        lo[d] = tile[t - T.st[R - 1 - d]];
+        hi[d] = tile[t + T.st[R - 1 - d]];
+    }
+    return upwind_update<R>(tile[t], lo, hi, dtdx, vel, hs);
 }
 
 // One time step for every leaf; one workgroup per leaf patch
@@ -955,8 +1245,8 @@ __global__ __launch_bounds__(NT) void k_criterion_gradient(const double* __restr
 
 // Face-halo cells of a patch with h ghost layers: h * face(dim) items per
 // direction, direction after direction.
-template <int R>
-__host__ __device__ inline int halo_items(box<R> const& B, int h)
+template <int R, class BX>
+__host__ __device__ inline int halo_items(BX const& B, int h)
 {
     int items = 0;
     for (int dir = 0; dir < box<R>::NDIR; ++dir) items += h * B.face(dir >> 1);
@@ -966,8 +1256,8 @@ __host__ __device__ inline int halo_items(box<R> const& B, int h)
 // Halo item g (0 <= g < halo_items): its direction (returned) and its cell c
 // in compact coordinates (layer `layer` beyond the face, tangential cells in
 // row-major order).
-template <int R>
-__host__ __device__ inline int halo_item(box<R> const& B, int h, int g, int* c)
+template <int R, class BX>
+__host__ __device__ inline int halo_item(BX const& B, int h, int g, int* c)
 {
     int dir = 0, r = g;
     while (r >= h * B.face(dir >> 1))
@@ -975,13 +1265,19 @@ __host__ __device__ inline int halo_item(box<R> const& B, int h, int g, int* c)
         r -= h * B.face(dir >> 1);
         ++dir;
     }
-    const int dim = dir >> 1, fc = B.face(dim), layer = r / fc;
-    r %= fc;
+    const int dim = dir >> 1, fc = B.face(dim);
+    int       layer = 0; // < h <= 8
+    while (r >= fc)
+    {
+        r -= fc;
+        ++layer;
+    }
     for (int d = R - 1; d >= 0; --d)
     {
         if (d == dim) continue;
-        c[d] = r % B.n(d);
-        r /= B.n(d);
+        const int q = B.quot(r, d);
+        c[d]        = r - q * B.n(d);
+        r           = q;
     }
     c[dim] = (dir & 1) ? B.n(dim) + layer : -1 - layer;
     return dir;
@@ -991,8 +1287,8 @@ __host__ __device__ inline int halo_item(box<R> const& B, int h, int g, int* c)
 // 0, reduced over the workgroup (every thread must call it): the interior
 // with coalesced loads, then the face halos by the ghost rules (padded_value's
 // cells of kind 0 and 1; the maximum is order-free).
-template <int R, int NT>
-__device__ inline double leaf_max_value(box<R> const& B, int h, const double* __restrict__ u, uint32_t leaf,
+template <int R, int NT, class BX>
+__device__ inline double leaf_max_value(BX const& B, int h, const double* __restrict__ u, uint32_t leaf,
                                         const face_link* __restrict__ links, const uint32_t* __restrict__ metas,
                                         double* red)
 {
@@ -1035,8 +1331,46 @@ __global__ __launch_bounds__(NT) void k_criterion_max(const double* __restrict__
 // expressions of the fixed-shape kernels, so the results are the same bits.
 // ---------------------------------------------------------------------------
 
+// One time step of patches of any shape whose tile fits in LDS, one workgroup
+// per leaf.  Bound by the latency of its two dependent ghost loads and the
+// index arithmetic of runtime extents, hence the column walk (one coordinate
+// decomposition per thread) and the divisions by multiplication.  us per step
+// against k_step_box on adapted trees: 2200 leaves of 12x10x6 12.9 for 26.6,
+// 990 of 16^3 28 for 93, 10000 of 6^3 21 for 54, 2200 of 32^2 12.4 for 20.4.
+template <int R, int NT, int CH>
+__global__ __launch_bounds__(NT) void k_step_box_tile(launch_box<R, true> B, box_walk W, const double* __restrict__ u,
+                                                      double* __restrict__ un, const uint64_t* __restrict__ keys,
+                                                      const face_link* __restrict__ links,
+                                                      const uint32_t* __restrict__ metas, step_params prm,
+                                                      const step_params* __restrict__ table,
+                                                      const uint16_t* __restrict__ inst, uint32_t nleaves)
+{
+    extern __shared__ double box_lds[];
+    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    if (leaf >= nleaves) return;
+    const step_params&  P  = params_for(prm, table, inst, leaf);
+    const int           lv = key_level(keys[leaf]);
+    const box_tile<R>   T(B);
+    const box_column<R> col(B, T, W);
+    stage_box<R, NT, 1, CH>(B, T, col, W, box_lds, u, 0, leaf, links, metas);
+    double dtdx[R], vel[R], hs[R];
+#pragma unroll
+    for (int d = 0; d < R; ++d)
+    {
+        dtdx[d] = P.dtdx[lv][d];
+        vel[d]  = P.vel[d];
+        hs[d]   = P.hs[d];
+    }
+    __syncthreads();
+    if (!col.on) return;
+    double* out = un + static_cast<size_t>(leaf) * B.ni();
+    for (int k = 0; col.z0 + k * col.dz < B.n(0); ++k)
+        out[col.i0 + k * col.di] = upwind_tile_cell<R>(box_lds, T, col.t0 + k * col.dt, dtdx, vel, hs);
+}
+
+// Patches whose tile does not fit: neighbours from memory.
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_step_box(box<R> B, const double* __restrict__ u, double* __restrict__ un,
+__global__ __launch_bounds__(NT) void k_step_box(launch_box<R> B, const double* __restrict__ u, double* __restrict__ un,
                                                  const uint64_t* __restrict__ keys,
                                                  const face_link* __restrict__ links,
                                                  const uint32_t* __restrict__ metas, step_params prm,
@@ -1061,7 +1395,7 @@ __global__ __launch_bounds__(NT) void k_step_box(box<R> B, const double* __restr
 }
 
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_padded_box(box<R> B, int h, const double* __restrict__ u,
+__global__ __launch_bounds__(NT) void k_padded_box(launch_box<R> B, int h, const double* __restrict__ u,
                                                    double* __restrict__ pad, const face_link* __restrict__ links,
                                                    const uint32_t* __restrict__ metas, uint32_t nleaves)
 {
@@ -1076,7 +1410,7 @@ __global__ __launch_bounds__(NT) void k_padded_box(box<R> B, int h, const double
 }
 
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_criterion_gradient_box(box<R> B, const double* __restrict__ u,
+__global__ __launch_bounds__(NT) void k_criterion_gradient_box(launch_box<R> B, const double* __restrict__ u,
                                                                const uint64_t* __restrict__ keys,
                                                                const face_link* __restrict__ links,
                                                                const uint32_t* __restrict__ metas, double rthr,
@@ -1094,7 +1428,7 @@ __global__ __launch_bounds__(NT) void k_criterion_gradient_box(box<R> B, const d
 }
 
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_criterion_max_box(box<R> B, int h, const double* __restrict__ u,
+__global__ __launch_bounds__(NT) void k_criterion_max_box(launch_box<R> B, int h, const double* __restrict__ u,
                                                           const uint64_t* __restrict__ keys,
                                                           const face_link* __restrict__ links,
                                                           const uint32_t* __restrict__ metas, double rthr, double cthr,

@@ -260,8 +260,8 @@ __host__ __device__ inline uint64_t emit_key(uint64_t key, int depth, bool refin
 
 // Cell t of child o of a refined leaf: injection (ndtree.hpp:1463-1497,
 // 1528-1555).
-template <int R>
-__host__ __device__ inline double refine_value(box<R> const& B, const double* __restrict__ src, int o, int t)
+template <int R, class BX>
+__host__ __device__ inline double refine_value(BX const& B, const double* __restrict__ src, int o, int t)
 {
     int tc[R], sc[R];
     B.coords(t, tc);
@@ -279,15 +279,15 @@ __host__ __device__ inline double refine_value(const double* __restrict__ src, i
 // Cell t of the parent of the family whose first child is slot i: mean of
 // 2^R child cells summed from 0.0 in row-major order (ndtree.hpp:1499-1526,
 // intergrid_operator.hpp:91-106).
-template <int R>
-__host__ __device__ inline double restrict_value(box<R> const& B, const double* __restrict__ u, uint32_t i, int t)
+template <int R, class BX>
+__host__ __device__ inline double restrict_value(BX const& B, const double* __restrict__ u, uint32_t i, int t)
 {
     int tc[R], base[R], kid = 0;
     B.coords(t, tc);
     for (int d = 0; d < R; ++d)
     {
-        kid |= (tc[d] / B.half(d)) << (R - 1 - d);
-        base[d] = (tc[d] % B.half(d)) * 2;
+        kid |= B.half_of(tc[d], d) << (R - 1 - d);
+        base[d] = B.fine(tc[d], d);
     }
     const double* q   = u + static_cast<size_t>(i + kid) * B.ni();
     double        sum = 0.0;
@@ -561,8 +561,8 @@ __global__ void k_scan_add(uint32_t* __restrict__ out, uint32_t n, const uint32_
 
 // New keys and interiors of old leaf i (one workgroup; every thread calls
 // it): its copy, its 2^R injected children or its family's restriction.
-template <int R, int NT>
-__device__ inline void emit_leaf(box<R> const& B, const uint64_t* __restrict__ keys, const double* __restrict__ u,
+template <int R, int NT, class BX>
+__device__ inline void emit_leaf(BX const& B, const uint64_t* __restrict__ keys, const double* __restrict__ u,
                                  uint32_t i, int depth, const uint8_t* __restrict__ mark,
                                  const uint8_t* __restrict__ head, const uint32_t* __restrict__ counts,
                                  const uint32_t* __restrict__ pos, uint64_t* __restrict__ keys_out,
@@ -628,7 +628,7 @@ __global__ __launch_bounds__(NT) void k_emit(const uint64_t* __restrict__ keys, 
 
 // k_emit for patches of any shape.
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_emit_box(box<R> B, const uint64_t* __restrict__ keys,
+__global__ __launch_bounds__(NT) void k_emit_box(launch_box<R> B, const uint64_t* __restrict__ keys,
                                                  const double* __restrict__ u, uint32_t n, int depth,
                                                  const uint8_t* __restrict__ mark, const uint8_t* __restrict__ head,
                                                  const uint32_t* __restrict__ counts,
