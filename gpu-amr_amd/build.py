@@ -38,6 +38,10 @@ def flags():
         "-target-feature",
         "-Xclang",
         "-packed-fp32-ops",
+        # the leading pointer and integer arguments of every kernel arrive in
+        # scalar registers instead of being loaded by its first instructions
+        "-mllvm",
+        "-amdgpu-kernarg-preload-count=14",
         "-Wall",
         "-Wno-unused-function",
         f"-I{ROOT / 'include'}",

@@ -90,7 +90,7 @@ struct ops
     int     rank, n, h; // n: the extent of every dim of a fixed cubic shape, 0 for the any-shape instance
     int32_t ext[3];     // interior cells per layout dim
     void (*step)(ops const&, int variant, const double*, double*, const uint64_t*, const face_link*, const uint32_t*,
-                 step_params const&, const step_params*, const uint16_t*, uint32_t, step_aux const&, hipStream_t);
+                 step_params const&, const step_params*, const uint32_t*, uint32_t, step_aux const&, hipStream_t);
     int (*variant_count)();
     char const* (*variant_name)(int);
     int (*variant_needs)(int);
@@ -107,12 +107,12 @@ struct ops
     void (*adj_regrid)(ops const&, const double*, const uint8_t*, const uint8_t*, const uint32_t*, const uint32_t*,
                        double*, uint32_t, hipStream_t);
     // two fused steps of a single-level tree (null: not built for the shape)
-    void (*step2)(const double*, double*, step2_params const&, uint32_t, hipStream_t);
+    void (*step2)(const double*, double*, step2_params const&, uint32_t level, uint32_t reverse, uint32_t, hipStream_t);
     // Euler fields (field-major, stride fstride doubles between fields)
     void (*euler_dt)(ops const&, const double*, size_t, const uint64_t*, euler_params const&, euler_scalars*, uint32_t,
                      hipStream_t);
     void (*euler_step)(ops const&, const double*, double*, size_t, const uint64_t*, const face_link*, const uint32_t*,
-                       euler_params const&, euler_scalars*, uint32_t, hipStream_t);
+                       euler_params const&, euler_scalars*, uint32_t reverse, uint32_t, hipStream_t);
 
     int ni() const { return (rank == 2) ? ext[0] * ext[1] : ext[0] * ext[1] * ext[2]; }
     int padded_cells() const
@@ -128,6 +128,19 @@ struct ops
                ext[2] == o.ext[2];
     }
 };
+
+// Calls f with where a step launch's constants come from (step_consts), as a
+// constant.
+template <typename Fn>
+void for_source(const step_params* table, const uint32_t* inst, Fn&& f)
+{
+    if (!table)
+        f(std::integral_constant<int, FROM_LAUNCH>{});
+    else if (!inst)
+        f(std::integral_constant<int, FROM_TABLE>{});
+    else
+        f(std::integral_constant<int, PER_LEAF>{});
+}
 
 template <int R, int N, int H>
 struct instance
@@ -148,53 +161,56 @@ struct instance
     static char const*           variant_name(int v) { return kWave ? kVariantsWave[v] : kVariantsAny[v]; }
     static int                   variant_needs(int v) { return (kWave && (v == 4 || v == 5)) ? NEEDS_RUNS : 0; }
 
-    template <bool NTS>
-    static void launch_wave(dim3 grid, unsigned lds, const double* u, double* un, const uint64_t* keys,
-                            const face_link* links, const uint32_t* metas, step_params const& prm,
-                            const step_params* table, const uint16_t* inst, uint32_t n, hipStream_t s)
-    {
-        if constexpr (R == 3 && N == 8)
-            hipLaunchKernelGGL(k_step_3d8<NTS>, grid, dim3(64), lds, s, u, un, keys, links, metas, prm, table, inst, n);
-        else if constexpr (R == 2 && N == 16)
-            hipLaunchKernelGGL(k_step_2d16<NTS>, grid, dim3(64), lds, s, u, un, keys, links, metas, prm, table, inst, n);
-    }
-
     static void step(ops const&, int variant, const double* u, double* un, const uint64_t* keys, const face_link* links,
                      const uint32_t* metas, step_params const& prm, const step_params* table,
-                     const uint16_t* inst, uint32_t n, step_aux const& aux, hipStream_t s)
+                     const uint32_t* inst, uint32_t n, step_aux const& aux, hipStream_t s)
     {
         if (n == 0) return;
-        const dim3 per_leaf(xcd_grid(n));
-        if constexpr (kWave)
-        {
-            const int rk = (variant == 4 || variant == 5) ? variant - 4 : -1; // run list of the run variants
-            if (rk >= 0 && !aux.list[rk]) variant = 0; // no run list: wave-per-leaf kernel
-            switch (variant)
+        for_source(table, inst, [&](auto source) {
+            constexpr int FROM = decltype(source)::value;
+            const dim3    per_leaf(xcd_grid(n));
+            const auto    walk = walk_of(n, prm.reverse);
+            auto          wave = [&](auto nts, unsigned lds) {
+                constexpr bool NTS = decltype(nts)::value;
+                if constexpr (R == 3 && N == 8)
+                    hipLaunchKernelGGL((k_step_3d8<NTS, FROM>), per_leaf, dim3(64), lds, s, u, un, keys, links, metas,
+                                       n, walk, prm, table, inst);
+                else if constexpr (R == 2 && N == 16)
+                    hipLaunchKernelGGL((k_step_2d16<NTS, FROM>), per_leaf, dim3(64), lds, s, u, un, keys, links, metas,
+                                       n, walk, prm, table, inst);
+            };
+            auto tile = [&] {
+                hipLaunchKernelGGL((k_step<R, N, NT, FROM>), per_leaf, dim3(NT), 0, s, u, un, keys, links, metas, n,
+                                   walk, prm, table, inst);
+            };
+            if constexpr (kWave)
             {
-                case 1: launch_wave<true>(per_leaf, 0, u, un, keys, links, metas, prm, table, inst, n, s); break;
-                case 2: launch_wave<false>(per_leaf, 10 << 10, u, un, keys, links, metas, prm, table, inst, n, s); break;
-                case 3:
-                    hipLaunchKernelGGL((k_step<R, N, NT>), per_leaf, dim3(NT), 0, s, u, un, keys, links, metas, prm,
-                                       table, inst, n);
-                    break;
-                case 4:
-                case 5:
+                const int rk = (variant == 4 || variant == 5) ? variant - 4 : -1; // run list of the run variants
+                if (rk >= 0 && !aux.list[rk]) variant = 0; // no run list: wave-per-leaf kernel
+                switch (variant)
                 {
-                    const dim3 per_run(xcd_grid(aux.count[rk]));
-                    if constexpr (R == 3)
-                        hipLaunchKernelGGL(k_step_3d8_run<false>, per_run, dim3(64), 0, s, u, un, keys, links, metas,
-                                           prm, table, inst, aux.list[rk], aux.count[rk]);
-                    else
-                        hipLaunchKernelGGL(k_step_2d16_run<false>, per_run, dim3(64), 0, s, u, un, keys, links,
-                                           metas, prm, table, inst, aux.list[rk], aux.count[rk]);
-                    break;
+                    case 1: wave(std::true_type{}, 0); break;
+                    case 2: wave(std::false_type{}, 10 << 10); break;
+                    case 3: tile(); break;
+                    case 4:
+                    case 5:
+                    {
+                        const uint32_t runs = aux.count[rk], rw = walk_of(runs, prm.reverse);
+                        const dim3     per_run(xcd_grid(runs));
+                        if constexpr (R == 3)
+                            hipLaunchKernelGGL((k_step_3d8_run<false, FROM>), per_run, dim3(64), 0, s, u, un, keys,
+                                               links, metas, runs, rw, prm, table, inst, aux.list[rk]);
+                        else
+                            hipLaunchKernelGGL((k_step_2d16_run<false, FROM>), per_run, dim3(64), 0, s, u, un, keys,
+                                               links, metas, runs, rw, prm, table, inst, aux.list[rk]);
+                        break;
+                    }
+                    default: wave(std::false_type{}, 0);
                 }
-                default: launch_wave<false>(per_leaf, 0, u, un, keys, links, metas, prm, table, inst, n, s);
             }
-        }
-        else
-            hipLaunchKernelGGL((k_step<R, N, NT>), per_leaf, dim3(NT), 0, s, u, un, keys, links, metas, prm, table,
-                               inst, n);
+            else
+                tile();
+        });
         check_launch("k_step");
     }
     static void padded(ops const&, const double* u, double* pad, const face_link* links, const uint32_t* metas, uint32_t n,
@@ -244,7 +260,8 @@ struct instance
                            lam_old, n_old);
         check_launch("k_adj_regrid");
     }
-    static void step2(const double* u, double* un, step2_params const& prm, uint32_t n, hipStream_t s)
+    static void step2(const double* u, double* un, step2_params const& prm, uint32_t level, uint32_t reverse,
+                      uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
         if constexpr (R == 3 && N == 8)
@@ -253,10 +270,11 @@ struct instance
             // (n = 8^level, so the blocks tile the slots); the root alone:
             // one wave
             if (n % 4 == 0)
-                hipLaunchKernelGGL((k_step2_3d8_uniform<false, 4>), dim3(xcd_grid(n / 4)), dim3(256), 0, s, u, un, prm,
-                                   n);
+                hipLaunchKernelGGL((k_step2_3d8_uniform<false, 4>), dim3(xcd_grid(n / 4)), dim3(256), 0, s, u, un, n,
+                                   walk_of(n / 4, reverse), level, prm);
             else
-                hipLaunchKernelGGL((k_step2_3d8_uniform<false, 1>), dim3(xcd_grid(n)), dim3(64), 0, s, u, un, prm, n);
+                hipLaunchKernelGGL((k_step2_3d8_uniform<false, 1>), dim3(xcd_grid(n)), dim3(64), 0, s, u, un, n,
+                                   walk_of(n, reverse), level, prm);
         }
         check_launch("k_step2");
     }
@@ -268,8 +286,8 @@ struct instance
         check_launch("k_euler_dt");
     }
     static void euler_step(ops const&, const double* u, double* un, size_t fs, const uint64_t* keys, const face_link* links,
-                           const uint32_t* metas, euler_params const& prm, euler_scalars* sc, uint32_t n,
-                           hipStream_t s)
+                           const uint32_t* metas, euler_params const& prm, euler_scalars* sc, uint32_t reverse,
+                           uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
         // 3D 8^3: one wave per leaf with the column in registers; other
@@ -277,21 +295,25 @@ struct instance
         // the patch, else neighbours from memory
         constexpr size_t tile_bytes = (R + 2) * tile_shape<R, N>::TS * sizeof(double);
         constexpr int    B          = euler_strip_depth<R, N>(40 * 1024);
+        const uint32_t   walk       = walk_of(n, reverse);
+        (void)walk;
         if constexpr (R == 3 && N == 8)
-            hipLaunchKernelGGL((k_euler_step_3d8<false>), dim3(xcd_grid(n)), dim3(64), 0, s, u, un, fs, keys, links,
-                               metas, prm, sc, n);
+            hipLaunchKernelGGL((k_euler_step_3d8<false>), dim3(xcd_grid(n)), dim3(64), 0, s, u, un, fs, keys, links, metas,
+                               n, walk, prm, sc);
         else if constexpr (R == 2 && N == 64)
             hipLaunchKernelGGL((k_euler_step_2d64<kEuler2d64Rows>), dim3(xcd_grid(static_cast<uint64_t>(n) * (64 / kEuler2d64Rows))),
-                               dim3(64), 0, s, u, un, fs, keys, links, metas, prm, sc, n);
+                               dim3(64), 0, s, u, un, fs, keys, links, metas,
+                               n, walk_of(static_cast<uint64_t>(n) * (64 / kEuler2d64Rows), reverse), prm, sc);
         else if constexpr (tile_bytes <= 48 * 1024)
-            hipLaunchKernelGGL((k_euler_step_tile<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, un, fs, keys, links,
-                               metas, prm, sc, n);
+            hipLaunchKernelGGL((k_euler_step_tile<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, un, fs, keys, links, metas,
+                               n, walk, prm, sc);
         else if constexpr (B > 0)
             hipLaunchKernelGGL((k_euler_step_strip<R, N, B, NT>), dim3(xcd_grid(static_cast<uint64_t>(n) * (N / B))),
-                               dim3(NT), 0, s, u, un, fs, keys, links, metas, prm, sc, n);
+                               dim3(NT), 0, s, u, un, fs, keys, links, metas,
+                               n, walk_of(static_cast<uint64_t>(n) * (N / B), reverse), prm, sc);
         else
-            hipLaunchKernelGGL((k_euler_step<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, un, fs, keys, links,
-                               metas, prm, sc, n);
+            hipLaunchKernelGGL((k_euler_step<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, un, fs, keys, links, metas,
+                               n, walk, prm, sc);
         check_launch("k_euler_step");
     }
     static constexpr ops table()
@@ -379,7 +401,7 @@ struct box_instance
     }
 
     static void step(ops const& o, int, const double* u, double* un, const uint64_t* keys, const face_link* links,
-                     const uint32_t* metas, step_params const& prm, const step_params* table, const uint16_t* inst,
+                     const uint32_t* metas, step_params const& prm, const step_params* table, const uint32_t* inst,
                      uint32_t n, step_aux const&, hipStream_t s)
     {
         if (n == 0) return;
@@ -387,22 +409,25 @@ struct box_instance
         const size_t lds = tile_bytes(o, 1);
         box_walk     W;
         const int    nt  = lds <= kBoxTileBytes ? walk_for(o, W) : 0;
-        auto         go  = [&](auto threads) {
-            constexpr int NT = decltype(threads)::value;
-            hipLaunchKernelGGL((k_step_box_tile<R, NT, 4>), grid, dim3(NT), lds, s, small_shape(o), W, u, un, keys, links,
-                               metas, prm, table, inst, n);
-        };
-        if (nt == 64)
-            go(std::integral_constant<int, 64>{});
-        else if (nt == 128)
-            go(std::integral_constant<int, 128>{});
-        else if (nt == 256)
-            go(std::integral_constant<int, 256>{});
-        else if (nt == 512)
-            go(std::integral_constant<int, 512>{});
-        else
-            hipLaunchKernelGGL((k_step_box<R, 256>), grid, dim3(256), 0, s, shape(o), u, un, keys, links, metas, prm,
-                               table, inst, n);
+        for_source(table, inst, [&](auto source) {
+            constexpr int FROM = decltype(source)::value;
+            auto          go   = [&](auto threads) {
+                constexpr int NT = decltype(threads)::value;
+                hipLaunchKernelGGL((k_step_box_tile<R, NT, 4, FROM>), grid, dim3(NT), lds, s, u, un, keys,
+                                   links, metas, n, walk_of(n, prm.reverse), small_shape(o), W, prm, table, inst);
+            };
+            if (nt == 64)
+                go(std::integral_constant<int, 64>{});
+            else if (nt == 128)
+                go(std::integral_constant<int, 128>{});
+            else if (nt == 256)
+                go(std::integral_constant<int, 256>{});
+            else if (nt == 512)
+                go(std::integral_constant<int, 512>{});
+            else
+                hipLaunchKernelGGL((k_step_box<R, 256, FROM>), grid, dim3(256), 0, s, u, un, keys, links, metas, n,
+                                   walk_of(n, prm.reverse), shape(o), prm, table, inst);
+        });
         check_launch("k_step_box");
     }
     static void padded(ops const& o, const double* u, double* pad, const face_link* links, const uint32_t* metas,
@@ -462,11 +487,11 @@ struct box_instance
     }
     static void euler_step(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys,
                            const face_link* links, const uint32_t* metas, euler_params const& prm, euler_scalars* sc,
-                           uint32_t n, hipStream_t s)
+                           uint32_t reverse, uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
-        hipLaunchKernelGGL((k_euler_step_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, shape(o), u, un, fs, keys,
-                           links, metas, prm, sc, n);
+        hipLaunchKernelGGL((k_euler_step_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, u, un, fs, keys, links, metas, n,
+                           walk_of(n, reverse), shape(o), prm, sc);
         check_launch("k_euler_step_box");
     }
     static ops table(int h, const int32_t* ext)
@@ -696,7 +721,7 @@ __global__ void k_offset_links(face_link* __restrict__ links, uint64_t count, in
         if (links[i].ids[j] >= 0) links[i].ids[j] += offset;
 }
 
-__global__ void k_fill_instance(uint16_t* __restrict__ inst, uint64_t count, uint16_t value)
+__global__ void k_fill_instance(uint32_t* __restrict__ inst, uint64_t count, uint32_t value)
 {
     const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
     if (i < count) inst[i] = value;
@@ -921,9 +946,8 @@ struct amr_ctx
             prm.dtdx[0][d] = dt1 / cell_size(max_level, d);
             prm.dtdx[1][d] = dt2 / cell_size(max_level, d);
         }
-        prm.level   = static_cast<uint32_t>(max_level);
-        prm.reverse = static_cast<uint32_t>(sweeps++ & 1);
-        op->step2(u[cur], u[1 - cur], prm, static_cast<uint32_t>(n), stream);
+        op->step2(u[cur], u[1 - cur], prm, static_cast<uint32_t>(max_level), static_cast<uint32_t>(sweeps++ & 1),
+                  static_cast<uint32_t>(n), stream);
         cur = 1 - cur;
     }
 
@@ -993,14 +1017,14 @@ struct amr_ctx
         op->euler_dt(*op, u[cur], fstride(), keys[kc], prm, esc, nn, stream);
         for (uint64_t s = 0; s < steps; ++s)
         {
-            prm.reverse  = static_cast<uint32_t>(sweeps++ & 1);
             prm.next_dt  = s + 1 < steps ? 1u : 0u;
             prm.now      = s == 0 ? 0u : 1u + static_cast<uint32_t>((s - 1) % 3);
             prm.next     = 1u + static_cast<uint32_t>(s % 3);
             prm.clear    = 1u + static_cast<uint32_t>((s + 1) % 3);
             prm.first    = s == 0 ? 1u : 0u;
             prm.clear_dt = s == 1 ? 1u : 0u;
-            op->euler_step(*op, u[cur], u[1 - cur], fstride(), keys[kc], links, metas, prm, esc, nn, stream);
+            op->euler_step(*op, u[cur], u[1 - cur], fstride(), keys[kc], links, metas, prm, esc,
+                           static_cast<uint32_t>(sweeps++ & 1), nn, stream);
             cur = 1 - cur;
         }
         euler_last = prm.next;
@@ -1156,7 +1180,7 @@ struct amr_batch
     uint64_t*                keys    = nullptr;
     face_link*               links   = nullptr;
     uint32_t*                metas   = nullptr;
-    uint16_t*                inst    = nullptr;
+    uint32_t*                inst    = nullptr;
     step_params*             table   = nullptr;
     run_lists                runs;
     struct graph_entry
@@ -1329,11 +1353,9 @@ struct amr_tape
     double*                    acc       = nullptr;
     // Per-step constants in device memory, written before every pass: the
     // velocity-dependent ones change between calls while the captured
-    // launches stay the same.  inst0: instance 0 for every leaf (the step
-    // kernels' per-leaf table lookup).
+    // launches stay the same.
     step_params*               step_tab = nullptr;
     adjoint_params*            adj_tab  = nullptr;
-    uint16_t*                  inst0    = nullptr;
     std::vector<step_params>   h_step_tab;
     std::vector<adjoint_params> h_adj_tab;
     std::vector<uint32_t>      h_leaves;
@@ -1358,7 +1380,7 @@ struct amr_tape
         for (pass_graph* g : { &g_forward, &g_adjoint })
             if (g->exec) (void)hipGraphExecDestroy(g->exec);
         std::vector<void*> ptrs = { lam[0], lam[1], work, vpart, step_sums, step_leaves, chunk, acc, scratch_keys,
-                                    scratch_summary, step_tab, adj_tab, inst0 };
+                                    scratch_summary, step_tab, adj_tab };
         for (auto& t : topos) ptrs.insert(ptrs.end(), { t.keys, t.links, t.metas });
         for (auto& r : regrids) ptrs.insert(ptrs.end(), { r.mark, r.head, r.counts, r.pos });
         for (double* c : ckpts) ptrs.push_back(c);
@@ -1486,8 +1508,6 @@ struct amr_tape
         scratch_summary = dev_alloc<regrid_summary>(1);
         step_tab        = dev_alloc<step_params>(steps);
         adj_tab         = dev_alloc<adjoint_params>(steps);
-        inst0           = dev_alloc<uint16_t>(max_n);
-        AMR_HIP_CHECK(hipMemsetAsync(inst0, 0, max_n * sizeof(uint16_t), stream));
         h_leaves.resize(steps);
         for (uint64_t k = 0; k < steps; ++k) h_leaves[k] = static_cast<uint32_t>(topo(k).n);
         AMR_HIP_CHECK(hipMemcpyAsync(step_leaves, h_leaves.data(), steps * sizeof(uint32_t), hipMemcpyHostToDevice,
@@ -1538,7 +1558,7 @@ struct amr_tape
         topology const& t = topo(k);
         step_params     prm{}; // the sweep direction; the constants come from step_tab[k]
         prm.reverse = static_cast<uint32_t>(k & 1);
-        op->step(*op, variant, src, dst, t.keys, t.links, t.metas, prm, step_tab + k, inst0, static_cast<uint32_t>(t.n),
+        op->step(*op, variant, src, dst, t.keys, t.links, t.metas, prm, step_tab + k, nullptr, static_cast<uint32_t>(t.n),
                  step_aux{}, stream);
     }
 
@@ -2429,7 +2449,7 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
             b->keys  = dev_alloc<uint64_t>(b->total);
             b->links = dev_alloc<face_link>(b->total * b->ndir);
             b->metas = dev_alloc<uint32_t>(b->total * b->ndir);
-            b->inst  = dev_alloc<uint16_t>(b->total);
+            b->inst  = dev_alloc<uint32_t>(b->total);
             b->table = dev_alloc<step_params>(count);
             for (uint32_t i = 0; i < count; ++i)
             {
@@ -2447,7 +2467,7 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
                 hipLaunchKernelGGL(k_offset_links, dim3(grid1d(nl, 256)), dim3(256), 0, b->stream, b->links + o * b->ndir,
                                    nl, static_cast<int32_t>(o));
                 hipLaunchKernelGGL(k_fill_instance, dim3(grid1d(t->n, 256)), dim3(256), 0, b->stream, b->inst + o, t->n,
-                                   static_cast<uint16_t>(i));
+                                   i);
                 check_launch("batch packing");
                 b->host_table.push_back(t->make_params(t->compute_dt()));
             }

@@ -45,15 +45,14 @@ constexpr uint32_t kEulerNowSlot = 4; // amr_solver_compute_dt's minimum
 constexpr uint32_t kEulerSlots   = 5;
 
 // Per-launch constants of the Euler kernels: gamma, the cell sizes of every
-// level (physics_system::cell_sizes, formed on the host), the sweep
-// direction, and the step's place in its batch.
+// level (physics_system::cell_sizes, formed on the host) and the step's place
+// in its batch.
 struct euler_params
 {
     double   gamma;
     double   cs[kMaxLevels][3];
     double   cfl;
     double   remaining;  // time left at the batch's start (read by its first step)
-    uint32_t reverse;
     uint32_t next_dt;    // step kernels: fold the next step's dt minimum over their output
     uint32_t now, next;  // slots: this launch's, the one it folds into
     uint32_t clear;      // slot whose minimum it empties
@@ -472,11 +471,11 @@ template <int R, int N, int NT>
 __global__ __launch_bounds__(NT) void k_euler_step(const double* __restrict__ u, double* __restrict__ un,
                                                    size_t fstride, const uint64_t* __restrict__ keys,
                                                    const face_link* __restrict__ links,
-                                                   const uint32_t* __restrict__ metas, euler_params prm,
-                                                   euler_scalars* sc, uint32_t nleaves)
+                                                   const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    euler_params prm, euler_scalars* sc)
 {
     constexpr box<R> B    = box<R>::cube(N);
-    const uint32_t   leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t   leaf = sweep_item(blockIdx.x, walk);
     const double   dt   = euler_step_dt(prm, sc);
     if (leaf >= nleaves) return;
     euler_step_leaf<R, NT>(B, u, un, fstride, keys, links, metas, prm, sc, dt, leaf);
@@ -484,13 +483,13 @@ __global__ __launch_bounds__(NT) void k_euler_step(const double* __restrict__ u,
 
 // k_euler_step for patches of any shape.
 template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_euler_step_box(launch_box<R> B, const double* __restrict__ u, double* __restrict__ un,
+__global__ __launch_bounds__(NT) void k_euler_step_box(const double* __restrict__ u, double* __restrict__ un,
                                                        size_t fstride, const uint64_t* __restrict__ keys,
                                                        const face_link* __restrict__ links,
-                                                       const uint32_t* __restrict__ metas, euler_params prm,
-                                                       euler_scalars* sc, uint32_t nleaves)
+                                                       const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    launch_box<R> B, euler_params prm, euler_scalars* sc)
 {
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     const double   dt   = euler_step_dt(prm, sc);
     if (leaf >= nleaves) return;
     euler_step_leaf<R, NT>(B, u, un, fstride, keys, links, metas, prm, sc, dt, leaf);
@@ -504,14 +503,14 @@ template <int R, int N, int NT>
 __global__ __launch_bounds__(NT) void k_euler_step_tile(const double* __restrict__ u, double* __restrict__ un,
                                                         size_t fstride, const uint64_t* __restrict__ keys,
                                                         const face_link* __restrict__ links,
-                                                        const uint32_t* __restrict__ metas, euler_params prm,
-                                                        euler_scalars* sc, uint32_t nleaves)
+                                                        const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    euler_params prm, euler_scalars* sc)
 {
     using S          = patch_shape<R, N>;
     using T          = tile_shape<R, N>;
     constexpr int NV = R + 2;
     __shared__ double tile[NV][T::TS];
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     const double dt = euler_step_dt(prm, sc);
     if (leaf >= nleaves) return;
     const size_t base = static_cast<size_t>(leaf) * S::NI;
@@ -629,14 +628,14 @@ __device__ inline euler_cell3 cell_lane_down8(euler_cell3 const& c)
 template <bool NTS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_euler_step_3d8(
     const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
-    const face_link* __restrict__ links, const uint32_t* __restrict__ metas, euler_params prm,
-    euler_scalars* sc, uint32_t nleaves)
+    const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    euler_params prm, euler_scalars* sc)
 {
     using F            = euler_flux<3>;
     constexpr int NV   = 5;
     constexpr int NI   = 512;
     __shared__ double fb[4][NV][64]; // boundary fluxes -y, +y (index z*8+x), -x, +x (index z*8+y)
-    const uint32_t    leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t    leaf = sweep_item(blockIdx.x, walk);
     const double dt = euler_step_dt(prm, sc);
     if (leaf >= nleaves) return;
     const int    lane = threadIdx.x, y = lane >> 3, x = lane & 7;
@@ -881,8 +880,8 @@ struct euler_cell2
 template <int B>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_euler_step_2d64(
     const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
-    const face_link* __restrict__ links, const uint32_t* __restrict__ metas, euler_params prm,
-    euler_scalars* sc, uint32_t nleaves)
+    const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    euler_params prm, euler_scalars* sc)
 {
     static_assert(B >= 2 && 64 % B == 0 && 2 * B <= 64, "strips of at least two rows");
     using F           = euler_flux<2>;
@@ -892,7 +891,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_
     constexpr int NS  = N / B;
     __shared__ double xg[NV + 3][B]; // +x ghost cell of each strip row: values, 1/rho, p, a
     __shared__ double xf[NV][B];     // -x boundary flux of each strip row
-    const uint32_t    item = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t    item = sweep_item(blockIdx.x, walk);
     const uint32_t    leaf = item / NS;
     const double dt = euler_step_dt(prm, sc);
     if (leaf >= nleaves) return;
@@ -1179,15 +1178,15 @@ template <int R, int N, int B, int NT>
 __global__ __launch_bounds__(NT) void k_euler_step_strip(const double* __restrict__ u, double* __restrict__ un,
                                                          size_t fstride, const uint64_t* __restrict__ keys,
                                                          const face_link* __restrict__ links,
-                                                         const uint32_t* __restrict__ metas, euler_params prm,
-                                                         euler_scalars* sc, uint32_t nleaves)
+                                                         const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    euler_params prm, euler_scalars* sc)
 {
     using S          = patch_shape<R, N>;
     using T          = strip_shape<R, N, B>;
     constexpr int NV = R + 2;
     __shared__ double tile[NV][T::TS];
     __shared__ double st_inv[T::TS], st_p[T::TS], st_a[T::TS];
-    const uint32_t item = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t item = sweep_item(blockIdx.x, walk);
     const uint32_t leaf = item / T::NS;
     const double dt = euler_step_dt(prm, sc);
     if (leaf >= nleaves) return;

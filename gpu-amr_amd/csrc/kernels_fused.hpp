@@ -25,11 +25,9 @@ namespace amrhip
 // for step s = 0, 1 (the second step can be clamped to the remaining time).
 struct step2_params
 {
-    double   vel[3];
-    double   hs[3];
-    double   dtdx[2][3];
-    uint32_t level;   // the level of every leaf
-    uint32_t reverse; // sweep direction (sweep_item)
+    double vel[3];
+    double hs[3];
+    double dtdx[2][3];
 };
 
 // Morton slot m moved by delta in {-1, 0, +1} along the axis whose bits are
@@ -110,14 +108,15 @@ __device__ inline void leaf_sync()
 // would have computed.  Every value is therefore the same bits as with W = 1.
 template <bool NT, int W = 1>
 __global__ __launch_bounds__(64 * W) void k_step2_3d8_uniform(const double* __restrict__ u, double* __restrict__ un,
-                                                              step2_params prm, uint32_t nleaves)
+                                                              uint32_t nleaves, uint32_t walk, uint32_t level,
+                                                              step2_params prm)
 {
     static_assert(W == 1 || W == 4, "one leaf or a 2 x 2 x 1 block per workgroup");
     constexpr int NI = 512;
     __shared__ double fbound_w[W][4][64]; // core boundary-face fluxes -y, +y, -x, +x (face layout)
     __shared__ double bring_w[W][4][64];  // u^{n+1} of the ghost ring (face layout)
     __shared__ double bcore_w[W][4][64];  // u^{n+1} of the core's boundary layers (face layout)
-    const uint32_t item = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t item = sweep_item(blockIdx.x, walk);
     if (item * W >= nleaves) return;
     // wave within the workgroup, as a wave-uniform (scalar) value
     const int      wv   = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -130,7 +129,7 @@ __global__ __launch_bounds__(64 * W) void k_step2_3d8_uniform(const double* __re
     const int           fyi  = (W == 4) ? ((wv & 2) ? 0 : 1) : -1;
     const int           lane = threadIdx.x & 63, hi = lane >> 3, lo = lane & 7;
     const bool          hlo = hi < 4, llo = lo < 4;
-    const morton_masks3 mk(prm.level);
+    const morton_masks3 mk(level);
     auto                P = [&](uint32_t slot) { return u + static_cast<size_t>(slot) * NI; };
     const double*       own = P(leaf);
 

@@ -32,19 +32,24 @@ struct step_params
     uint32_t reverse; // walk this launch's leaves backwards (sweep_item)
 };
 
-// Leaf (or run) of workgroup b in a launch over nblocks items: each XCD owns
-// the same contiguous range in every launch (xcd_item), walked backwards
-// when `reverse` is set.  Consecutive steps alternate the direction, so that
-// a step starts on the leaves the previous one wrote last -- the lines most
-// likely still in the memory-side cache (8^3 step, 32768 leaves: 57 us
-// alternating against 65 us always forward) -- while a tree small enough for
-// the XCDs' L2s keeps finding its leaves in the L2 that wrote them.  Items
-// >= count are skipped by the caller.
-__device__ inline uint32_t sweep_item(uint32_t b, uint32_t nblocks, uint32_t reverse)
+// Leaf (or run) of workgroup b: each XCD owns the same contiguous range in
+// every launch (xcd_item), walked backwards when `reverse` is set.
+// Consecutive steps alternate the direction, so that a step starts on the
+// leaves the previous one wrote last -- the lines most likely still in the
+// memory-side cache (8^3 step, 32768 leaves: 57 us alternating against 65 us
+// always forward) -- while a tree small enough for the XCDs' L2s keeps finding
+// its leaves in the L2 that wrote them.  Items >= count are skipped by the
+// caller.  `walk` is walk_of(items, reverse): an argument of its own ahead of
+// the constants, so that the hardware hands it to the wave with the pointers
+// (kernel arguments up to the first structure arrive in scalar registers; a
+// load of them would stand before the kernel's first load of data).
+__device__ inline uint32_t sweep_item(uint32_t b, uint32_t walk)
 {
-    const uint32_t per = nblocks / kXcds, j = b / kXcds;
-    return (b % kXcds) * per + (reverse ? per - 1 - j : j);
+    const uint32_t per = walk >> 1, j = b / kXcds;
+    return (b % kXcds) * per + ((walk & 1) ? per - 1 - j : j);
 }
+
+inline uint32_t walk_of(uint64_t items, uint32_t reverse) { return xcd_grid(items) / kXcds * 2 + (reverse & 1u); }
 
 // Output store of a step kernel.  The non-temporal form streams the new
 // state past L2 so that L2 keeps the input lines that neighbouring leaves'
@@ -58,12 +63,55 @@ __device__ inline void store_cell(double* p, double v)
         *p = v;
 }
 
-// Step constants of a leaf: the launch's own, or, for a batch of
-// concatenated trees, those of the leaf's instance.
-__device__ inline const step_params& params_for(const step_params& prm, const step_params* __restrict__ table,
-                                                const uint16_t* __restrict__ inst, uint32_t leaf)
+// Where a launch's step constants come from: its own argument, one entry of a
+// table in device memory (a captured launch, whose constants change between
+// replays) or, for a batch of concatenated trees, the entry of the leaf's
+// instance.
+enum : int
 {
-    return table ? table[inst[leaf]] : prm;
+    FROM_LAUNCH = 0,
+    FROM_TABLE  = 1,
+    PER_LEAF    = 2,
+};
+
+// A leaf's step constants.  Its key and instance are read at the top of a
+// kernel, next to the leaf's face records, and the constants they select
+// before the ghosts arrive: read after them they were two or three more round
+// trips to memory, one behind the other, in kernels bound by such chains (8^3
+// step of 22500 adapted leaves 39.4 -> 35.3 us, 16^2 step of a batch of 74000
+// leaves 82 -> 79 us).
+template <int R>
+struct step_consts
+{
+    double dtdx[R], vel[R], hs[R];
+};
+
+template <int FROM>
+__device__ inline uint32_t leaf_instance(const uint32_t* __restrict__ inst, uint32_t leaf)
+{
+    if constexpr (FROM == PER_LEAF) return inst[leaf];
+    return 0;
+}
+
+template <int FROM, int R>
+__device__ inline step_consts<R> leaf_consts(step_params const& prm, const step_params* __restrict__ table,
+                                             uint32_t who, int lv)
+{
+    step_consts<R> c;
+    auto           take = [&](step_params const& P) {
+#pragma unroll
+        for (int d = 0; d < R; ++d)
+        {
+            c.dtdx[d] = P.dtdx[lv][d];
+            c.vel[d]  = P.vel[d];
+            c.hs[d]   = P.hs[d];
+        }
+    };
+    if constexpr (FROM == FROM_LAUNCH)
+        take(prm);
+    else
+        take(table[who]);
+    return c;
 }
 
 // Ghost value of the cell with layout coordinates c (c[dim] lies outside
@@ -236,17 +284,17 @@ __host__ __device__ inline double cell_or_ghost(BX const& B, const double* __res
     return u[static_cast<size_t>(leaf) * B.ni() + B.lin(c)];
 }
 
-// A leaf's face records: relation/quadrant word and first neighbour slot per
+// A leaf's face records: relation/quadrant word and neighbour slots per
 // direction, read with one batch of scalar loads.
 template <int R>
 __device__ inline void load_faces(const face_link* __restrict__ L, const uint32_t* __restrict__ M, uint32_t* m,
-                                  int32_t* nb)
+                                  int4* nb)
 {
 #pragma unroll
     for (int k = 0; k < 2 * R; ++k)
     {
         m[k]  = M[k];
-        nb[k] = L[k].ids[0];
+        nb[k] = int4{ L[k].ids[0], L[k].ids[1], L[k].ids[2], L[k].ids[3] };
     }
 }
 
@@ -261,33 +309,61 @@ __device__ inline bool single_cell_ghosts(const uint32_t* m)
     return finer == 0;
 }
 
+// Ghost cell c of direction DIR with finer neighbours nb: ghost_value's
+// finer rule, the fine slot picked by selects.
+template <int DIR>
+__device__ inline double fine_mean_3d8(const double* __restrict__ u, int4 nb, const int* c)
+{
+    constexpr box<3> B   = box<3>::cube(8);
+    constexpr int    dim = DIR >> 1;
+    int              k = 0, bit = 0, cc[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+        cc[d] = (d == dim) ? ((DIR & 1) ? 0 : 6) : B.fine(c[d], d);
+        if (d != dim)
+        {
+            k |= B.half_of(c[d], d) << bit;
+            ++bit;
+        }
+    }
+    const int32_t slot = (k & 2) ? ((k & 1) ? nb.w : nb.z) : ((k & 1) ? nb.y : nb.x);
+    const double* q    = u + static_cast<size_t>(slot) * B.ni() + B.lin(cc);
+    double        f[8];
+#pragma unroll
+    for (int o = 0; o < 8; ++o) f[o] = q[((o >> 2) & 1) * 64 + ((o >> 1) & 1) * 8 + (o & 1)];
+    double sum = 0.0;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) sum += f[o];
+    return sum / 8.0;
+}
+
 // The six ghost values of a lane of the 3D wave layout (lane = 8 hi + lo),
-// from the leaf's face records (m, nb; L, M for the finer-neighbour path):
-// g[0], g[1] = -z / +z of the column (y, x) = (hi, lo); g[2], g[3] = the
-// (z, x) = (hi, lo) cell of the -y / +y face; g[4], g[5] = the (z, y) =
-// (hi, lo) cell of the -x / +x face (skipped unless wanted).  Unless a face
-// has finer neighbours, all loads are issued back to back: a per-face switch
-// on the relation makes the compiler wait for every outstanding load before
-// each face.
-__device__ inline void gather_ghosts_3d8(const double* __restrict__ u, const uint32_t* m, const int32_t* nb,
-                                         const face_link* __restrict__ L, const uint32_t* __restrict__ M, int hi,
+// from the leaf's face records (m, nb): g[0], g[1] = -z / +z of the column
+// (y, x) = (hi, lo); g[2], g[3] = the (z, x) = (hi, lo) cell of the -y / +y
+// face; g[4], g[5] = the (z, y) = (hi, lo) cell of the -x / +x face (skipped
+// unless wanted).  The single-cell ghosts are loaded back to back for all
+// faces (a face with finer neighbours reads a cell it then drops): a
+// per-face switch on the relation makes the compiler wait for every
+// outstanding load before each face.
+__device__ inline void gather_ghosts_3d8(const double* __restrict__ u, const uint32_t* m, const int4* nb, int hi,
                                          int lo, bool want_xm, bool want_xp, double* g)
 {
     const int c[6][3] = { { -1, hi, lo }, { 8, hi, lo }, { hi, -1, lo }, { hi, 8, lo }, { hi, lo, -1 }, { hi, lo, 8 } };
-    if (single_cell_ghosts<3>(m))
-    {
-        size_t src[6];
+    size_t src[6];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) src[k] = ghost_source<3, 8>(nb[k], m[k], k, c[k]);
+    for (int k = 0; k < 6; ++k) src[k] = ghost_source<3, 8>(nb[k].x, m[k], k, c[k]);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) g[k] = u[src[k]];
-        g[4] = want_xm ? u[src[4]] : 0.0;
-        g[5] = want_xp ? u[src[5]] : 0.0;
-        return;
-    }
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-        g[k] = ((k == 4 && !want_xm) || (k == 5 && !want_xp)) ? 0.0 : ghost_value<3, 8>(u, L[k], M[k], k, c[k]);
+    for (int k = 0; k < 4; ++k) g[k] = u[src[k]];
+    g[4] = want_xm ? u[src[4]] : 0.0;
+    g[5] = want_xp ? u[src[5]] : 0.0;
+    if (single_cell_ghosts<3>(m)) return;
+    if (rel_of(m[0]) == REL_FINER) g[0] = fine_mean_3d8<0>(u, nb[0], c[0]);
+    if (rel_of(m[1]) == REL_FINER) g[1] = fine_mean_3d8<1>(u, nb[1], c[1]);
+    if (rel_of(m[2]) == REL_FINER) g[2] = fine_mean_3d8<2>(u, nb[2], c[2]);
+    if (rel_of(m[3]) == REL_FINER) g[3] = fine_mean_3d8<3>(u, nb[3], c[3]);
+    if (rel_of(m[4]) == REL_FINER && want_xm) g[4] = fine_mean_3d8<4>(u, nb[4], c[4]);
+    if (rel_of(m[5]) == REL_FINER && want_xp) g[5] = fine_mean_3d8<5>(u, nb[5], c[5]);
 }
 
 // The ghost value a lane of the 2D wave layout gathers: cell t of face q
@@ -296,23 +372,24 @@ __device__ inline void gather_ghosts_3d8(const double* __restrict__ u, const uin
 // neighbour's mean needs -- a same-level or coarser neighbour's single cell
 // four times -- and keeps the mean (summed from 0.0 in row-major order, as
 // ghost_value) or the first value.
-__device__ inline double gather_ghost_2d16(const double* __restrict__ u, const uint32_t* ms, const int32_t* nbs,
-                                           const face_link* __restrict__ L, int q, int t)
+__device__ inline double gather_ghost_2d16(const double* __restrict__ u, const uint32_t* ms, const int4* nbs, int q,
+                                           int t)
 {
     using S = patch_shape<2, 16>;
     int c[2];
     c[0] = (q == 0) ? -1 : (q == 1) ? 16 : t;
     c[1] = (q == 2) ? -1 : (q == 3) ? 16 : t;
     // the lane's own face record, selected from the four uniform ones
-    uint32_t m  = ms[0];
-    int32_t  nb = nbs[0];
+    uint32_t m   = ms[0];
+    int32_t  nb  = nbs[0].x;
+    int32_t  id1 = nbs[0].y; // second fine slot of a face with finer neighbours
 #pragma unroll
     for (int k = 1; k < 4; ++k)
-        if (q == k)
-        {
-            m  = ms[k];
-            nb = nbs[k];
-        }
+    {
+        m   = q == k ? ms[k] : m;
+        nb  = q == k ? nbs[k].x : nb;
+        id1 = q == k ? nbs[k].y : id1;
+    }
     size_t src[4];
     if (single_cell_ghosts<2>(ms))
         return u[ghost_source<2, 16>(nb, m, q, c)];
@@ -324,14 +401,6 @@ __device__ inline double gather_ghost_2d16(const double* __restrict__ u, const u
         const int dim = q >> 1, nrm = (q & 1) ? c[dim] - 16 : c[dim] + 16;
         int       base[2];
         for (int d = 0; d < 2; ++d) base[d] = (((d == dim) ? nrm : c[d]) * 2) % 16;
-        // second fine slot of each face, read as uniform values and selected
-        int32_t id1s[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) id1s[k] = L[k].ids[1];
-        int32_t id1 = id1s[0];
-#pragma unroll
-        for (int k = 1; k < 4; ++k)
-            if (q == k) id1 = id1s[k];
         const int32_t fine = (t / S::HALF) ? id1 : nb;
 #pragma unroll
         for (int o = 0; o < 4; ++o)
@@ -863,31 +932,24 @@ __device__ inline double upwind_tile_cell(const double* tile, box_tile<R> const&
 
 // One time step for every leaf; one workgroup per leaf patch
 // (XCD-contiguous ranges).
-template <int R, int N, int NT>
+template <int R, int N, int NT, int FROM>
 __global__ __launch_bounds__(NT) void k_step(const double* __restrict__ u, double* __restrict__ un,
                                              const uint64_t* __restrict__ keys,
                                              const face_link* __restrict__ links,
-                                             const uint32_t* __restrict__ metas, step_params prm,
-                                             const step_params* __restrict__ table,
-                                             const uint16_t* __restrict__ inst, uint32_t nleaves)
+                                             const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
     using S = patch_shape<R, N>;
     __shared__ double tile[tile_shape<R, N>::TS];
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
+    const uint32_t who = leaf_instance<FROM>(inst, leaf);
+    const int      lv  = key_level(keys[leaf]);
     stage_tile<R, N, NT>(tile, u, leaf, links, metas);
+    const step_consts<R> C = leaf_consts<FROM, R>(prm, table, who, lv);
     __syncthreads();
-    const step_params& P  = params_for(prm, table, inst, leaf);
-    const int          lv = key_level(keys[leaf]);
-    double             dtdx[R], vel[R], hs[R];
-    for (int d = 0; d < R; ++d)
-    {
-        dtdx[d] = P.dtdx[lv][d];
-        vel[d]  = P.vel[d];
-        hs[d]   = P.hs[d];
-    }
     double* out = un + static_cast<size_t>(leaf) * S::NI;
-    for (int i = threadIdx.x; i < S::NI; i += NT) out[i] = upwind_cell<R, N>(tile, i, dtdx, vel, hs);
+    for (int i = threadIdx.x; i < S::NI; i += NT) out[i] = upwind_cell<R, N>(tile, i, C.dtdx, C.vel, C.hs);
 }
 
 // 3D 8^3 patches, one wave (64 lanes) per leaf.  Lane l owns the z-column at
@@ -896,41 +958,38 @@ __global__ __launch_bounds__(NT) void k_step(const double* __restrict__ u, doubl
 // ghost faces are gathered one face cell per lane; the -+z faces land in the
 // lane that needs them, the -+y / -+x faces go through 2 KiB of LDS.  With
 // no interior tile in LDS, 32 leaves are in flight per CU.
-template <bool NT>
+template <bool NT, int FROM>
 __global__ __launch_bounds__(64) void k_step_3d8(const double* __restrict__ u, double* __restrict__ un,
                                                  const uint64_t* __restrict__ keys,
                                                  const face_link* __restrict__ links,
-                                                 const uint32_t* __restrict__ metas, step_params prm,
-                                                 const step_params* __restrict__ table,
-                                                 const uint16_t* __restrict__ inst, uint32_t nleaves)
+                                                 const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
     constexpr int NI = 512;
     __shared__ double gface[4][64]; // -y, +y (index z*8+x), -x, +x (index z*8+y)
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
-    const int     lane = threadIdx.x, hi3 = lane >> 3, lo3 = lane & 7;
-    const double* up   = u + static_cast<size_t>(leaf) * NI;
+    const int      lane = threadIdx.x, hi3 = lane >> 3, lo3 = lane & 7;
+    const uint32_t who  = leaf_instance<FROM>(inst, leaf);
+    const int      lv   = key_level(keys[leaf]);
+    uint32_t       m[6];
+    int4           nb[6];
+    load_faces<3>(links + static_cast<size_t>(leaf) * 6, metas + static_cast<size_t>(leaf) * 6, m, nb);
+    const double* up = u + static_cast<size_t>(leaf) * NI;
     double        r[8];
 #pragma unroll
     for (int z = 0; z < 8; ++z) r[z] = up[z * 64 + lane];
-    const face_link* L = links + static_cast<size_t>(leaf) * 6;
-    const uint32_t*  M = metas + static_cast<size_t>(leaf) * 6;
-    uint32_t         m[6];
-    int32_t          nb[6];
-    load_faces<3>(L, M, m, nb);
-    double g[6];
-    gather_ghosts_3d8(u, m, nb, L, M, hi3, lo3, true, true, g);
+    const step_consts<3> C = leaf_consts<FROM, 3>(prm, table, who, lv);
+    double               g[6];
+    gather_ghosts_3d8(u, m, nb, hi3, lo3, true, true, g);
     const double gzm = g[0], gzp = g[1];
 #pragma unroll
     for (int k = 0; k < 4; ++k) gface[k][lane] = g[2 + k];
     __syncthreads();
-    const step_params& P       = params_for(prm, table, inst, leaf);
-    const int          lv      = key_level(keys[leaf]);
-    const double       dtdx[3] = { P.dtdx[lv][0], P.dtdx[lv][1], P.dtdx[lv][2] };
-    const int    y = hi3, x = lo3;
-    double*      out = un + static_cast<size_t>(leaf) * NI;
+    const int y = hi3, x = lo3;
+    double*   out = un + static_cast<size_t>(leaf) * NI;
     // z faces are evaluated once: the +z flux of cell z is the -z flux of z+1
-    double fz = upwind_flux(gzm, r[0], P.vel[2], P.hs[2]);
+    double fz = upwind_flux(gzm, r[0], C.vel[2], C.hs[2]);
 #pragma unroll
     for (int z = 0; z < 8; ++z)
     {
@@ -944,10 +1003,10 @@ __global__ __launch_bounds__(64) void k_step_3d8(const double* __restrict__ u, d
         const double ly = (y == 0) ? gface[0][z * 8 + x] : yl;
         const double hy = (y == 7) ? gface[1][z * 8 + x] : yr;
         const double hz = (z == 7) ? gzp : r[z < 7 ? z + 1 : 7];
-        const double fzr = upwind_flux(uc, hz, P.vel[2], P.hs[2]);
-        const double fL[3] = { upwind_flux(lx, uc, P.vel[0], P.hs[0]), upwind_flux(ly, uc, P.vel[1], P.hs[1]), fz };
-        const double fR[3] = { upwind_flux(uc, hx, P.vel[0], P.hs[0]), upwind_flux(uc, hy, P.vel[1], P.hs[1]), fzr };
-        store_cell<NT>(out + z * 64 + lane, update_from_fluxes<3>(uc, fL, fR, dtdx));
+        const double fzr = upwind_flux(uc, hz, C.vel[2], C.hs[2]);
+        const double fL[3] = { upwind_flux(lx, uc, C.vel[0], C.hs[0]), upwind_flux(ly, uc, C.vel[1], C.hs[1]), fz };
+        const double fR[3] = { upwind_flux(uc, hx, C.vel[0], C.hs[0]), upwind_flux(uc, hy, C.vel[1], C.hs[1]), fzr };
+        store_cell<NT>(out + z * 64 + lane, update_from_fluxes<3>(uc, fL, fR, C.dtdx));
         fz = fzr;
     }
 }
@@ -960,18 +1019,16 @@ __global__ __launch_bounds__(64) void k_step_3d8(const double* __restrict__ u, d
 // update); only the run's two end faces are gathered from memory.  An x face
 // touches every 64 B row of the neighbour patch, so this removes most of the
 // ghost traffic that does not hit in L2.
-template <bool NT>
+template <bool NT, int FROM>
 __global__ __launch_bounds__(64) void k_step_3d8_run(const double* __restrict__ u, double* __restrict__ un,
                                                      const uint64_t* __restrict__ keys,
                                                      const face_link* __restrict__ links,
-                                                     const uint32_t* __restrict__ metas, step_params prm,
-                                                     const step_params* __restrict__ table,
-                                                     const uint16_t* __restrict__ inst,
-                                                     const leaf_run* __restrict__ runs, uint32_t nruns)
+                                                     const uint32_t* __restrict__ metas, uint32_t nruns, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst, const leaf_run* __restrict__ runs)
 {
     constexpr int NI = 512;
     __shared__ double gface[4][64]; // -y, +y (index z*8+x), -x, +x (index z*8+y)
-    const uint32_t r = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t r = sweep_item(blockIdx.x, walk);
     if (r >= nruns) return;
     const int      lane = threadIdx.x, hi3 = lane >> 3, lo3 = lane & 7;
     const int      y = hi3, x = lo3;
@@ -994,11 +1051,14 @@ __global__ __launch_bounds__(64) void k_step_3d8_run(const double* __restrict__ 
         const bool       more = i + 1 < run.len;
         // ghosts of this leaf first, then the next leaf's interior, so that
         // the update below waits only for the ghosts
-        uint32_t m[6];
-        int32_t  nb[6];
+        const uint32_t who = leaf_instance<FROM>(inst, leaf);
+        const int      lv  = key_level(keys[leaf]);
+        uint32_t       m[6];
+        int4           nb[6];
         load_faces<3>(L, M, m, nb);
-        double g[6];
-        gather_ghosts_3d8(u, m, nb, L, M, hi3, lo3, i == 0, !more, g);
+        const step_consts<3> C = leaf_consts<FROM, 3>(prm, table, who, lv);
+        double               g[6];
+        gather_ghosts_3d8(u, m, nb, hi3, lo3, i == 0, !more, g);
         const double gzm = g[0], gzp = g[1];
         gface[0][lane]   = g[2];
         gface[1][lane]   = g[3];
@@ -1012,11 +1072,8 @@ __global__ __launch_bounds__(64) void k_step_3d8_run(const double* __restrict__ 
             for (int z = 0; z < 8; ++z) nxt[z] = np[z * 64 + lane];
         }
         __syncthreads();
-        const step_params& P       = params_for(prm, table, inst, leaf);
-        const int          lv      = key_level(keys[leaf]);
-        const double       dtdx[3] = { P.dtdx[lv][0], P.dtdx[lv][1], P.dtdx[lv][2] };
-        double*            out     = un + static_cast<size_t>(leaf) * NI;
-        double             fz      = upwind_flux(gzm, cur[0], P.vel[2], P.hs[2]); // z faces once
+        double* out = un + static_cast<size_t>(leaf) * NI;
+        double  fz  = upwind_flux(gzm, cur[0], C.vel[2], C.hs[2]); // z faces once
 #pragma unroll
         for (int z = 0; z < 8; ++z)
         {
@@ -1031,10 +1088,10 @@ __global__ __launch_bounds__(64) void k_step_3d8_run(const double* __restrict__ 
             const double ly = (y == 0) ? gface[0][z * 8 + x] : yl;
             const double hy = (y == 7) ? gface[1][z * 8 + x] : yr;
             const double hz = (z == 7) ? gzp : cur[z < 7 ? z + 1 : 7];
-            const double fzr = upwind_flux(uc, hz, P.vel[2], P.hs[2]);
-            const double fL[3] = { upwind_flux(lx, uc, P.vel[0], P.hs[0]), upwind_flux(ly, uc, P.vel[1], P.hs[1]), fz };
-            const double fR[3] = { upwind_flux(uc, hx, P.vel[0], P.hs[0]), upwind_flux(uc, hy, P.vel[1], P.hs[1]), fzr };
-            store_cell<NT>(out + z * 64 + lane, update_from_fluxes<3>(uc, fL, fR, dtdx));
+            const double fzr = upwind_flux(uc, hz, C.vel[2], C.hs[2]);
+            const double fL[3] = { upwind_flux(lx, uc, C.vel[0], C.hs[0]), upwind_flux(ly, uc, C.vel[1], C.hs[1]), fz };
+            const double fR[3] = { upwind_flux(uc, hx, C.vel[0], C.hs[0]), upwind_flux(uc, hy, C.vel[1], C.hs[1]), fzr };
+            store_cell<NT>(out + z * 64 + lane, update_from_fluxes<3>(uc, fL, fR, C.dtdx));
             fz = fzr;
         }
         __syncthreads();
@@ -1054,39 +1111,36 @@ __global__ __launch_bounds__(64) void k_step_3d8_run(const double* __restrict__ 
 // y = 4 (l / 16) .. 4 (l / 16) + 3; x-neighbours from lanes l -+ 1, the row
 // above / below a lane's four from lanes l -+ 16; the four ghost faces are
 // gathered one face cell per lane into 512 B of LDS.
-template <bool NT>
+template <bool NT, int FROM>
 __global__ __launch_bounds__(64) void k_step_2d16(const double* __restrict__ u, double* __restrict__ un,
                                                   const uint64_t* __restrict__ keys,
                                                   const face_link* __restrict__ links,
-                                                  const uint32_t* __restrict__ metas, step_params prm,
-                                                  const step_params* __restrict__ table,
-                                                  const uint16_t* __restrict__ inst, uint32_t nleaves)
+                                                  const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
     constexpr int NI = 256;
     __shared__ double gface[4][16]; // -y, +y (index x), -x, +x (index y)
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
-    const int     lane = threadIdx.x, x = lane & 15, q = lane >> 4;
-    const double* up   = u + static_cast<size_t>(leaf) * NI;
+    const int      lane = threadIdx.x, x = lane & 15, q = lane >> 4;
+    const uint32_t who  = leaf_instance<FROM>(inst, leaf);
+    const int      lv   = key_level(keys[leaf]);
+    uint32_t       m[4];
+    int4           nb[4];
+    load_faces<2>(links + static_cast<size_t>(leaf) * 4, metas + static_cast<size_t>(leaf) * 4, m, nb);
+    const double* up = u + static_cast<size_t>(leaf) * NI;
     double        r[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) r[j] = up[(4 * q + j) * 16 + x];
-    const face_link* L = links + static_cast<size_t>(leaf) * 4;
-    const uint32_t*  M = metas + static_cast<size_t>(leaf) * 4;
-    uint32_t         m[4];
-    int32_t          nb[4];
-    load_faces<2>(L, M, m, nb);
+    const step_consts<2> C = leaf_consts<FROM, 2>(prm, table, who, lv);
     // lane (q, x) gathers cell x of face q
-    gface[q][x] = gather_ghost_2d16(u, m, nb, L, q, x);
+    gface[q][x] = gather_ghost_2d16(u, m, nb, q, x);
     __syncthreads();
-    const step_params& P       = params_for(prm, table, inst, leaf);
-    const int          lv      = key_level(keys[leaf]);
-    const double       dtdx[2] = { P.dtdx[lv][0], P.dtdx[lv][1] };
     const double above   = __shfl_up(r[3], 16, 64);  // row 4q - 1
     const double below   = __shfl_down(r[0], 16, 64); // row 4q + 4
     double*      out     = un + static_cast<size_t>(leaf) * NI;
     // y faces are evaluated once: the +y flux of row j is the -y flux of j+1
-    double fy = upwind_flux((q == 0) ? gface[0][x] : above, r[0], P.vel[1], P.hs[1]);
+    double fy = upwind_flux((q == 0) ? gface[0][x] : above, r[0], C.vel[1], C.hs[1]);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
     {
@@ -1097,10 +1151,10 @@ __global__ __launch_bounds__(64) void k_step_2d16(const double* __restrict__ u, 
         const double lx = (x == 0) ? gface[2][y] : xl;
         const double hx = (x == 15) ? gface[3][y] : xr;
         const double hy = (j < 3) ? r[j < 3 ? j + 1 : 3] : ((q == 3) ? gface[1][x] : below);
-        const double fyr   = upwind_flux(uc, hy, P.vel[1], P.hs[1]);
-        const double fL[2] = { upwind_flux(lx, uc, P.vel[0], P.hs[0]), fy };
-        const double fR[2] = { upwind_flux(uc, hx, P.vel[0], P.hs[0]), fyr };
-        store_cell<NT>(out + y * 16 + x, update_from_fluxes<2>(uc, fL, fR, dtdx));
+        const double fyr   = upwind_flux(uc, hy, C.vel[1], C.hs[1]);
+        const double fL[2] = { upwind_flux(lx, uc, C.vel[0], C.hs[0]), fy };
+        const double fR[2] = { upwind_flux(uc, hx, C.vel[0], C.hs[0]), fyr };
+        store_cell<NT>(out + y * 16 + x, update_from_fluxes<2>(uc, fL, fR, C.dtdx));
         fy = fyr;
     }
 }
@@ -1109,18 +1163,16 @@ __global__ __launch_bounds__(64) void k_step_2d16(const double* __restrict__ u, 
 // layout of k_step_2d16 and the hand-over of k_step_3d8_run: the -x ghosts
 // of a leaf are the previous leaf's x = 15 column (left in LDS), its +x
 // ghosts the next leaf's x = 0 column (registers of the prefetched leaf).
-template <bool NT>
+template <bool NT, int FROM>
 __global__ __launch_bounds__(64) void k_step_2d16_run(const double* __restrict__ u, double* __restrict__ un,
                                                       const uint64_t* __restrict__ keys,
                                                       const face_link* __restrict__ links,
-                                                      const uint32_t* __restrict__ metas, step_params prm,
-                                                      const step_params* __restrict__ table,
-                                                      const uint16_t* __restrict__ inst,
-                                                      const leaf_run* __restrict__ runs, uint32_t nruns)
+                                                      const uint32_t* __restrict__ metas, uint32_t nruns, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst, const leaf_run* __restrict__ runs)
 {
     constexpr int NI = 256;
     __shared__ double gface[4][16]; // -y, +y (index x), -x, +x (index y)
-    const uint32_t r = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t r = sweep_item(blockIdx.x, walk);
     if (r >= nruns) return;
     const int      lane = threadIdx.x, x = lane & 15, q = lane >> 4;
     const leaf_run run  = runs[r];
@@ -1140,11 +1192,13 @@ __global__ __launch_bounds__(64) void k_step_2d16_run(const double* __restrict__
         const bool   more = i + 1 < run.len;
         const size_t e0   = static_cast<size_t>(leaf) * 4;
         // lanes of quarter q gather face q (y faces always, the run's end x faces)
-        uint32_t m[4];
-        int32_t  nb[4];
+        const uint32_t who = leaf_instance<FROM>(inst, leaf);
+        const int      lv  = key_level(keys[leaf]);
+        uint32_t       m[4];
+        int4           nb[4];
         load_faces<2>(links + e0, metas + e0, m, nb);
-        if (q < 2 || (q == 2 && i == 0) || (q == 3 && !more))
-            gface[q][x] = gather_ghost_2d16(u, m, nb, links + e0, q, x);
+        const step_consts<2> C = leaf_consts<FROM, 2>(prm, table, who, lv);
+        if (q < 2 || (q == 2 && i == 0) || (q == 3 && !more)) gface[q][x] = gather_ghost_2d16(u, m, nb, q, x);
         const uint32_t next = more ? static_cast<uint32_t>(links[e0 + 3].ids[0]) : leaf;
         if (more)
         {
@@ -1153,13 +1207,10 @@ __global__ __launch_bounds__(64) void k_step_2d16_run(const double* __restrict__
             for (int j = 0; j < 4; ++j) nxt[j] = np[(4 * q + j) * 16 + x];
         }
         __syncthreads();
-        const step_params& P       = params_for(prm, table, inst, leaf);
-        const int          lv      = key_level(keys[leaf]);
-        const double       dtdx[2] = { P.dtdx[lv][0], P.dtdx[lv][1] };
         const double       above   = __shfl_up(cur[3], 16, 64);  // row 4q - 1
         const double       below   = __shfl_down(cur[0], 16, 64); // row 4q + 4
         double*            out     = un + static_cast<size_t>(leaf) * NI;
-        double             fy      = upwind_flux((q == 0) ? gface[0][x] : above, cur[0], P.vel[1], P.hs[1]);
+        double             fy      = upwind_flux((q == 0) ? gface[0][x] : above, cur[0], C.vel[1], C.hs[1]);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
         {
@@ -1171,10 +1222,10 @@ __global__ __launch_bounds__(64) void k_step_2d16_run(const double* __restrict__
             const double lx = (x == 0) ? gface[2][y] : xl;
             const double hx = (x == 15) ? (more ? xn : gface[3][y]) : xr;
             const double hy = (j < 3) ? cur[j < 3 ? j + 1 : 3] : ((q == 3) ? gface[1][x] : below);
-            const double fyr   = upwind_flux(uc, hy, P.vel[1], P.hs[1]);
-            const double fL[2] = { upwind_flux(lx, uc, P.vel[0], P.hs[0]), fy };
-            const double fR[2] = { upwind_flux(uc, hx, P.vel[0], P.hs[0]), fyr };
-            store_cell<NT>(out + y * 16 + x, update_from_fluxes<2>(uc, fL, fR, dtdx));
+            const double fyr   = upwind_flux(uc, hy, C.vel[1], C.hs[1]);
+            const double fL[2] = { upwind_flux(lx, uc, C.vel[0], C.hs[0]), fy };
+            const double fR[2] = { upwind_flux(uc, hx, C.vel[0], C.hs[0]), fyr };
+            store_cell<NT>(out + y * 16 + x, update_from_fluxes<2>(uc, fL, fR, C.dtdx));
             fy = fyr;
         }
         __syncthreads();
@@ -1337,61 +1388,44 @@ __global__ __launch_bounds__(NT) void k_criterion_max(const double* __restrict__
 // decomposition per thread) and the divisions by multiplication.  us per step
 // against k_step_box on adapted trees: 2200 leaves of 12x10x6 12.9 for 26.6,
 // 990 of 16^3 28 for 93, 10000 of 6^3 21 for 54, 2200 of 32^2 12.4 for 20.4.
-template <int R, int NT, int CH>
-__global__ __launch_bounds__(NT) void k_step_box_tile(launch_box<R, true> B, box_walk W, const double* __restrict__ u,
+template <int R, int NT, int CH, int FROM>
+__global__ __launch_bounds__(NT) void k_step_box_tile(const double* __restrict__ u,
                                                       double* __restrict__ un, const uint64_t* __restrict__ keys,
                                                       const face_link* __restrict__ links,
-                                                      const uint32_t* __restrict__ metas, step_params prm,
-                                                      const step_params* __restrict__ table,
-                                                      const uint16_t* __restrict__ inst, uint32_t nleaves)
+                                                      const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, launch_box<R, true> B, box_walk W, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
     extern __shared__ double box_lds[];
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
-    const step_params&  P  = params_for(prm, table, inst, leaf);
-    const int           lv = key_level(keys[leaf]);
+    const uint32_t      who = leaf_instance<FROM>(inst, leaf);
+    const int           lv  = key_level(keys[leaf]);
     const box_tile<R>   T(B);
     const box_column<R> col(B, T, W);
     stage_box<R, NT, 1, CH>(B, T, col, W, box_lds, u, 0, leaf, links, metas);
-    double dtdx[R], vel[R], hs[R];
-#pragma unroll
-    for (int d = 0; d < R; ++d)
-    {
-        dtdx[d] = P.dtdx[lv][d];
-        vel[d]  = P.vel[d];
-        hs[d]   = P.hs[d];
-    }
+    const step_consts<R> C = leaf_consts<FROM, R>(prm, table, who, lv);
     __syncthreads();
     if (!col.on) return;
     double* out = un + static_cast<size_t>(leaf) * B.ni();
     for (int k = 0; col.z0 + k * col.dz < B.n(0); ++k)
-        out[col.i0 + k * col.di] = upwind_tile_cell<R>(box_lds, T, col.t0 + k * col.dt, dtdx, vel, hs);
+        out[col.i0 + k * col.di] = upwind_tile_cell<R>(box_lds, T, col.t0 + k * col.dt, C.dtdx, C.vel, C.hs);
 }
 
 // Patches whose tile does not fit: neighbours from memory.
-template <int R, int NT>
-__global__ __launch_bounds__(NT) void k_step_box(launch_box<R> B, const double* __restrict__ u, double* __restrict__ un,
+template <int R, int NT, int FROM>
+__global__ __launch_bounds__(NT) void k_step_box(const double* __restrict__ u, double* __restrict__ un,
                                                  const uint64_t* __restrict__ keys,
                                                  const face_link* __restrict__ links,
-                                                 const uint32_t* __restrict__ metas, step_params prm,
-                                                 const step_params* __restrict__ table,
-                                                 const uint16_t* __restrict__ inst, uint32_t nleaves)
+                                                 const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, launch_box<R> B, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
-    const uint32_t leaf = sweep_item(blockIdx.x, gridDim.x, prm.reverse);
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
-    const step_params& P  = params_for(prm, table, inst, leaf);
-    const int          lv = key_level(keys[leaf]);
-    double             dtdx[R], vel[R], hs[R];
-    for (int d = 0; d < R; ++d)
-    {
-        dtdx[d] = P.dtdx[lv][d];
-        vel[d]  = P.vel[d];
-        hs[d]   = P.hs[d];
-    }
+    const step_consts<R> C = leaf_consts<FROM, R>(prm, table, leaf_instance<FROM>(inst, leaf), key_level(keys[leaf]));
     const int ni  = B.ni();
     double*   out = un + static_cast<size_t>(leaf) * ni;
     for (int i = threadIdx.x; i < ni; i += NT)
-        out[i] = upwind_cell_direct<R>(B, u, leaf, links, metas, i, dtdx, vel, hs);
+        out[i] = upwind_cell_direct<R>(B, u, leaf, links, metas, i, C.dtdx, C.vel, C.hs);
 }
 
 template <int R, int NT>
