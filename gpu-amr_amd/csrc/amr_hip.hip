@@ -248,8 +248,15 @@ struct instance
                          hipStream_t s)
     {
         if (n == 0) return;
-        hipLaunchKernelGGL((k_adj_step<R, N, NT>), dim3(n), dim3(NT), 0, s, lam_next, u, keys, links, metas, prm, lam,
-                           vpart, n);
+        if constexpr (R == 3 && N == 8)
+            hipLaunchKernelGGL(k_adj_step_3d8, dim3(xcd_grid(n)), dim3(64), 0, s, lam_next, u, keys, links, metas, prm,
+                               lam, vpart, n, walk_of(n, 0));
+        else if constexpr (R == 2 && N == 16)
+            hipLaunchKernelGGL(k_adj_step_2d16, dim3(xcd_grid(n)), dim3(64), 0, s, lam_next, u, keys, links, metas,
+                               prm, lam, vpart, n, walk_of(n, 0));
+        else
+            hipLaunchKernelGGL((k_adj_step<R, N, NT>), dim3(n), dim3(NT), 0, s, lam_next, u, keys, links, metas, prm,
+                               lam, vpart, n);
         check_launch("k_adj_step");
     }
     static void adj_regrid(ops const&, const double* lam_new, const uint8_t* mark, const uint8_t* head, const uint32_t* counts,

@@ -416,6 +416,383 @@ __global__ __launch_bounds__(NT) void k_adj_step(const double* __restrict__ lam_
         }
 }
 
+// ---------------------------------------------------------------------------
+// One wave per leaf for the configurations' patches (3D 8^3, 2D 16^2): the
+// step kernels' lane layouts, lambda' and u in registers, lambda's halo terms
+// and u's ghosts through LDS.  A ghost of u and the transposed halo term of
+// the same face cell come from the same neighbour cell, so one address serves
+// both loads.  Operands and sums are k_adj_step's in its order, so the same
+// bits.
+//
+// Bound by the chain face records -> neighbour cells -> store; the LDS-tile
+// kernel walked it once per face through a switch on the relation, and spent
+// most of its instructions on indexes and on 6 R shuffles per wave of the
+// velocity sums.  us a launch, LDS tile -> one wave: 16^2, 214 adapted leaves
+// (launch and latency) 5.35 -> 3.94; 8^3, 4096 leaves (three passes over
+// 16.8 MB, 7.2 us at the copy rate) 28.8 -> 16.1.
+// ---------------------------------------------------------------------------
+
+// The level at whose dt/dx the neighbour across a face reads its ghost.
+__device__ inline int face_level(uint32_t meta, int lv)
+{
+    return lv + (rel_of(meta) == REL_FINER ? 1 : 0) - (rel_of(meta) == REL_COARSER ? 1 : 0);
+}
+
+// lambda' summed over the four fine cells across face cell c of direction DIR
+// (adj_face_term's finer rule).
+template <int DIR>
+__device__ inline double fine_sum_3d8(const double* __restrict__ lam, int4 nb, const int* c)
+{
+    constexpr box<3> B   = box<3>::cube(8);
+    constexpr int    dim = DIR >> 1;
+    int              k = 0, bit = 0, cc[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+        cc[d] = (d == dim) ? ((DIR & 1) ? 0 : 7) : B.fine(c[d], d);
+        if (d != dim)
+        {
+            k |= B.half_of(c[d], d) << bit;
+            ++bit;
+        }
+    }
+    const int32_t slot = (k & 2) ? ((k & 1) ? nb.w : nb.z) : ((k & 1) ? nb.y : nb.x);
+    const double* q    = lam + static_cast<size_t>(slot) * B.ni() + B.lin(cc);
+    constexpr int s1   = dim == 0 ? 8 : 64, s2 = dim == 2 ? 8 : 1; // strides of the two tangential dims
+    double        f[4];
+#pragma unroll
+    for (int o = 0; o < 4; ++o) f[o] = q[(o >> 1) * s1 + (o & 1) * s2];
+    double sum = 0.0;
+#pragma unroll
+    for (int o = 0; o < 4; ++o) sum += f[o];
+    return sum;
+}
+
+// a + b where the lane adds the value N lanes further within its row of 16
+// (rotated): with N = 8, 4, 2, 1 in turn every lane holds the row's sum in
+// the order of a shuffle-down tree.
+template <int N>
+__device__ inline double row_rotate_add(double v)
+{
+    const uint64_t b  = __builtin_bit_cast(uint64_t, v);
+    const int      lo = static_cast<int>(b), hi = static_cast<int>(b >> 32);
+    const int      l  = __builtin_amdgcn_update_dpp(0, lo, 0x120 + N, 0xF, 0xF, true); // row_ror:N
+    const int      h  = __builtin_amdgcn_update_dpp(0, hi, 0x120 + N, 0xF, 0xF, true);
+    return v + __builtin_bit_cast(double, (static_cast<uint64_t>(static_cast<uint32_t>(h)) << 32) |
+                                              static_cast<uint32_t>(l));
+}
+
+__device__ inline double row_sum(double v)
+{
+    return row_rotate_add<1>(row_rotate_add<2>(row_rotate_add<4>(row_rotate_add<8>(v))));
+}
+
+// One level of a tree sum of two values at once: of a over the lanes without
+// the WIDTH bit and of b over those with it, each with its partner WIDTH lanes
+// away (WIDTH = 32 or 16).
+template <int WIDTH>
+__device__ inline double fold_pair(double a, double b)
+{
+    const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+    uint32_t       p[2], q[2];
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+    {
+        const uint32_t xw = static_cast<uint32_t>(x >> (32 * w)), yw = static_cast<uint32_t>(y >> (32 * w));
+        if constexpr (WIDTH == 32)
+        {
+            const auto r = __builtin_amdgcn_permlane32_swap(xw, yw, false, false);
+            p[w] = r[0];
+            q[w] = r[1];
+        }
+        else
+        {
+            const auto r = __builtin_amdgcn_permlane16_swap(xw, yw, false, false);
+            p[w] = r[0];
+            q[w] = r[1];
+        }
+    }
+    return __builtin_bit_cast(double, (static_cast<uint64_t>(p[1]) << 32) | p[0]) +
+           __builtin_bit_cast(double, (static_cast<uint64_t>(q[1]) << 32) | q[0]);
+}
+
+// The sums of the four rows of 16 lanes (uniform in each row), in row order.
+__device__ inline double rows_in_order(double v)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    double         r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(b), 16 * k);
+        const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(b >> 32), 16 * k);
+        r[k]              = __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+    }
+    return ((r[0] + r[1]) + r[2]) + r[3];
+}
+
+// A leaf's adjoint constants: own-level coefficients of lambda's neighbours
+// (ap along +, am along -), of the cell itself (diag), dt/dx and sgn(v).
+template <int R>
+struct adj_consts
+{
+    double ap[R], am[R], dtdx[R], sgn[R], diag;
+
+    __device__ adj_consts(adjoint_params const& prm, int lv)
+    {
+        diag = 1.0;
+#pragma unroll
+        for (int d = 0; d < R; ++d)
+        {
+            dtdx[d] = prm.dtdx[lv][d];
+            sgn[d]  = prm.sgn[d];
+            ap[d]   = dtdx[d] * prm.vp[d];
+            am[d]   = dtdx[d] * prm.vm[d];
+            diag -= dtdx[d] * (prm.vp[d] - prm.vm[d]);
+        }
+    }
+};
+
+// 3D 8^3: lane l owns the z-column at (y, x) = (l / 8, l % 8).
+__global__ __launch_bounds__(64) void k_adj_step_3d8(const double* __restrict__ lam_next, const double* __restrict__ u,
+                                                     const uint64_t* __restrict__ keys,
+                                                     const face_link* __restrict__ links,
+                                                     const uint32_t* __restrict__ metas,
+                                                     const adjoint_params* __restrict__ prm_p,
+                                                     double* __restrict__ lam, double* __restrict__ vpart,
+                                                     uint32_t nleaves, uint32_t walk)
+{
+    constexpr int     NI = 512;
+    __shared__ double gface[4][64]; // ghosts of u: -y, +y (index z*8+x), -x, +x (index z*8+y)
+    __shared__ double hface[4][64]; // halo terms of lambda on the same faces
+    const uint32_t    leaf = sweep_item(blockIdx.x, walk);
+    if (leaf >= nleaves) return;
+    const int lane = threadIdx.x, hi3 = lane >> 3, lo3 = lane & 7;
+    const int lv   = key_level(keys[leaf]);
+    uint32_t  m[6];
+    int4      nb[6];
+    load_faces<3>(links + static_cast<size_t>(leaf) * 6, metas + static_cast<size_t>(leaf) * 6, m, nb);
+    const double* lp = lam_next + static_cast<size_t>(leaf) * NI;
+    const double* up = u + static_cast<size_t>(leaf) * NI;
+    double        l[8], r[8];
+#pragma unroll
+    for (int z = 0; z < 8; ++z) l[z] = lp[z * 64 + lane];
+#pragma unroll
+    for (int z = 0; z < 8; ++z) r[z] = up[z * 64 + lane];
+    const adjoint_params& prm = *prm_p;
+    const adj_consts<3>   C(prm, lv);
+    const int cf[6][3] = { { -1, hi3, lo3 }, { 8, hi3, lo3 }, { hi3, -1, lo3 },
+                           { hi3, 8, lo3 },  { hi3, lo3, -1 }, { hi3, lo3, 8 } };
+    double    g[6], h[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+    {
+        const size_t src = ghost_source<3, 8>(nb[k].x, m[k], k, cf[k]);
+        g[k]             = u[src];
+        h[k]             = lam_next[src];
+    }
+    if (!single_cell_ghosts<3>(m))
+    {
+        auto fine = [&](auto dir) {
+            constexpr int K = decltype(dir)::value;
+            if (rel_of(m[K]) != REL_FINER) return;
+            g[K] = fine_mean_3d8<K>(u, nb[K], cf[K]);
+            h[K] = fine_sum_3d8<K>(lam_next, nb[K], cf[K]);
+        };
+        fine(std::integral_constant<int, 0>{});
+        fine(std::integral_constant<int, 1>{});
+        fine(std::integral_constant<int, 2>{});
+        fine(std::integral_constant<int, 3>{});
+        fine(std::integral_constant<int, 4>{});
+        fine(std::integral_constant<int, 5>{});
+    }
+    bool coarse[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+    {
+        const int    d    = 2 - (k >> 1);
+        const double dtdx = prm.dtdx[face_level(m[k], lv)][d];
+        coarse[k]         = rel_of(m[k]) == REL_COARSER;
+        h[k]              = ((k & 1) ? dtdx * prm.vp[d] : -(dtdx * prm.vm[d])) * h[k] * (coarse[k] ? 0.125 : 1.0);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        gface[k][lane] = g[2 + k];
+        hface[k][lane] = h[2 + k];
+    }
+    __syncthreads();
+    const int y = hi3, x = lo3;
+    // the cells that a face's halo term reaches: the boundary layer and, next
+    // to a coarser neighbour, the one behind it
+    const bool ym = y == 0 || (y == 1 && coarse[2]), yp = y == 7 || (y == 6 && coarse[3]);
+    const bool xm = x == 0 || (x == 1 && coarse[4]), xp = x == 7 || (x == 6 && coarse[5]);
+    double     va[4][3] = {}; // k_adj_step's thread (z % 4, lane) sums its two cells
+    double*    out      = lam + static_cast<size_t>(leaf) * NI;
+#pragma unroll
+    for (int z = 0; z < 8; ++z)
+    {
+        const double lc = l[z], uc = r[z];
+        const double lxp = lane_plus1(lc), lxm = lane_minus1(lc);
+        const double lyp = __shfl_down(lc, 8, 64), lym = __shfl_up(lc, 8, 64);
+        double       acc = C.diag * lc, t;
+        t                = acc + C.ap[0] * lxp;
+        acc              = x < 7 ? t : acc;
+        t                = acc - C.am[0] * lxm;
+        acc              = x > 0 ? t : acc;
+        t                = acc + C.ap[1] * lyp;
+        acc              = y < 7 ? t : acc;
+        t                = acc - C.am[1] * lym;
+        acc              = y > 0 ? t : acc;
+        if (z < 7) acc += C.ap[2] * l[z < 7 ? z + 1 : 7];
+        if (z > 0) acc -= C.am[2] * l[z > 0 ? z - 1 : 0];
+        if (z == 0 || (z == 1 && coarse[0])) acc += h[0];
+        if (z == 7 || (z == 6 && coarse[1])) acc += h[1];
+        t   = acc + hface[0][z * 8 + x];
+        acc = ym ? t : acc;
+        t   = acc + hface[1][z * 8 + x];
+        acc = yp ? t : acc;
+        t   = acc + hface[2][z * 8 + y];
+        acc = xm ? t : acc;
+        t   = acc + hface[3][z * 8 + y];
+        acc = xp ? t : acc;
+        out[z * 64 + lane] = acc;
+        const double uxm = lane_minus1(uc), uxp = lane_plus1(uc);
+        const double uym = __shfl_up(uc, 8, 64), uyp = __shfl_down(uc, 8, 64);
+        const double lx = x == 0 ? gface[2][z * 8 + y] : uxm, hx = x == 7 ? gface[3][z * 8 + y] : uxp;
+        const double ly = y == 0 ? gface[0][z * 8 + x] : uym, hy = y == 7 ? gface[1][z * 8 + x] : uyp;
+        const double lz = z == 0 ? g[0] : r[z > 0 ? z - 1 : 0], hz = z == 7 ? g[1] : r[z < 7 ? z + 1 : 7];
+        va[z & 3][0] += adj_velocity_term(uc, lx, hx, lc, C.dtdx[0], C.sgn[0]);
+        va[z & 3][1] += adj_velocity_term(uc, ly, hy, lc, C.dtdx[1], C.sgn[1]);
+        va[z & 3][2] += adj_velocity_term(uc, lz, hz, lc, C.dtdx[2], C.sgn[2]);
+    }
+    // the tree of k_adj_step's four waves, all twelve sums at once: lanes 32
+    // apart (waves 0, 1 and 2, 3 together), lanes 16 apart (row w then holds
+    // wave w), each row, and the rows in order
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+        const double s02 = fold_pair<32>(va[0][d], va[2][d]), s13 = fold_pair<32>(va[1][d], va[3][d]);
+        const double sum = rows_in_order(row_sum(fold_pair<16>(s02, s13)));
+        if (lane == 0) vpart[static_cast<size_t>(leaf) * 3 + d] = sum;
+    }
+}
+
+// 2D 16^2: lane (q, x) owns x of rows 4q .. 4q + 3 and gathers cell x of
+// face q.
+__global__ __launch_bounds__(64) void k_adj_step_2d16(const double* __restrict__ lam_next,
+                                                      const double* __restrict__ u, const uint64_t* __restrict__ keys,
+                                                      const face_link* __restrict__ links,
+                                                      const uint32_t* __restrict__ metas,
+                                                      const adjoint_params* __restrict__ prm_p,
+                                                      double* __restrict__ lam, double* __restrict__ vpart,
+                                                      uint32_t nleaves, uint32_t walk)
+{
+    constexpr int     NI = 256;
+    __shared__ double gface[4][16]; // ghosts of u: -y, +y (index x), -x, +x (index y)
+    __shared__ double hface[4][16]; // halo terms of lambda
+    const uint32_t    leaf = sweep_item(blockIdx.x, walk);
+    if (leaf >= nleaves) return;
+    const int lane = threadIdx.x, x = lane & 15, q = lane >> 4;
+    const int lv   = key_level(keys[leaf]);
+    uint32_t  m[4];
+    int4      nb[4];
+    load_faces<2>(links + static_cast<size_t>(leaf) * 4, metas + static_cast<size_t>(leaf) * 4, m, nb);
+    const double* lp = lam_next + static_cast<size_t>(leaf) * NI;
+    const double* up = u + static_cast<size_t>(leaf) * NI;
+    double        l[4], r[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) l[j] = lp[(4 * q + j) * 16 + x];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = up[(4 * q + j) * 16 + x];
+    const adjoint_params& prm = *prm_p;
+    const adj_consts<2>   C(prm, lv);
+    ghost_cells_2d16      cells(m, nb, q, x);
+    double                ug, hg;
+    if (single_cell_ghosts<2>(m))
+    {
+        ug = u[cells.first];
+        hg = lam_next[cells.first];
+    }
+    else
+    {
+        // the two fine cells that touch the face: the layer of the 2 x 2
+        // block on our side, along the face
+        const bool   along_x = q < 2, far = (q & 1) == 0;
+        const size_t t0 = cells.first + (cells.finer && far ? (along_x ? 16 : 1) : 0);
+        const size_t t1 = t0 + (cells.finer ? (along_x ? 1 : 16) : 0);
+        const double h0 = lam_next[t0], h1 = lam_next[t1];
+        ug              = cells.value(u);
+        hg              = cells.finer ? (0.0 + h0) + h1 : h0;
+    }
+    bool   coarse[4];
+    double dtf = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        coarse[k]      = rel_of(m[k]) == REL_COARSER;
+        const double f = prm.dtdx[face_level(m[k], lv)][1 - (k >> 1)];
+        dtf            = q == k ? f : dtf;
+    }
+    const double vf = q == 0 ? -prm.vm[1] : q == 1 ? prm.vp[1] : q == 2 ? -prm.vm[0] : prm.vp[0];
+    const bool   cq = q == 0 ? coarse[0] : q == 1 ? coarse[1] : q == 2 ? coarse[2] : coarse[3];
+    gface[q][x]     = ug;
+    hface[q][x]     = (dtf * vf) * hg * (cq ? 0.25 : 1.0);
+    __syncthreads();
+    const double lup = __shfl_up(l[3], 16, 64), ldn = __shfl_down(l[0], 16, 64); // rows 4q - 1, 4q + 4
+    const double uup = __shfl_up(r[3], 16, 64), udn = __shfl_down(r[0], 16, 64);
+    const bool   xm = x == 0 || (x == 1 && coarse[2]), xp = x == 15 || (x == 14 && coarse[3]);
+    double       va[4][2];
+    double*      out = lam + static_cast<size_t>(leaf) * NI;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        const int    y  = 4 * q + j;
+        const double lc = l[j], uc = r[j];
+        const double lxp = lane_plus1(lc), lxm = lane_minus1(lc);
+        const double lyp = j < 3 ? l[j < 3 ? j + 1 : 3] : ldn, lym = j > 0 ? l[j > 0 ? j - 1 : 0] : lup;
+        double       acc = C.diag * lc, t;
+        t                = acc + C.ap[0] * lxp;
+        acc              = x < 15 ? t : acc;
+        t                = acc - C.am[0] * lxm;
+        acc              = x > 0 ? t : acc;
+        t                = acc + C.ap[1] * lyp;
+        acc              = y < 15 ? t : acc;
+        t                = acc - C.am[1] * lym;
+        acc              = y > 0 ? t : acc;
+        if (j < 2)
+        {
+            t   = acc + hface[0][x];
+            acc = q == 0 && (j == 0 || coarse[0]) ? t : acc;
+        }
+        if (j > 1)
+        {
+            t   = acc + hface[1][x];
+            acc = q == 3 && (j == 3 || coarse[1]) ? t : acc;
+        }
+        t   = acc + hface[2][y];
+        acc = xm ? t : acc;
+        t   = acc + hface[3][y];
+        acc = xp ? t : acc;
+        out[y * 16 + x] = acc;
+        const double uxm = lane_minus1(uc), uxp = lane_plus1(uc);
+        const double lx = x == 0 ? gface[2][y] : uxm, hx = x == 15 ? gface[3][y] : uxp;
+        const double ly = j > 0 ? r[j > 0 ? j - 1 : 0] : (q == 0 ? gface[0][x] : uup);
+        const double hy = j < 3 ? r[j < 3 ? j + 1 : 3] : (q == 3 ? gface[1][x] : udn);
+        va[j][0]        = 0.0 + adj_velocity_term(uc, lx, hx, lc, C.dtdx[0], C.sgn[0]);
+        va[j][1]        = 0.0 + adj_velocity_term(uc, ly, hy, lc, C.dtdx[1], C.sgn[1]);
+    }
+    // the tree of k_adj_step's four waves (wave q held rows 4q .. 4q + 3):
+    // lanes 32 and 16 apart were rows 2 and 1 apart
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+    {
+        const double sum = rows_in_order(row_sum((va[0][d] + va[2][d]) + (va[1][d] + va[3][d])));
+        if (lane == 0) vpart[static_cast<size_t>(leaf) * 3 + d] = sum;
+    }
+    if (lane == 0) vpart[static_cast<size_t>(leaf) * 3 + 2] = 0.0;
+}
+
 // Transposed regrid transfer of old leaf i (one workgroup; mark / head /
 // counts / pos recorded by the forward regrid).
 template <int R, int NT, class BX>

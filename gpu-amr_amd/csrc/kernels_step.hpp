@@ -366,62 +366,77 @@ __device__ inline void gather_ghosts_3d8(const double* __restrict__ u, const uin
     if (rel_of(m[5]) == REL_FINER && want_xp) g[5] = fine_mean_3d8<5>(u, nb[5], c[5]);
 }
 
-// The ghost value a lane of the 2D wave layout gathers: cell t of face q
-// (lane = 16 q + t).  Branch-free over the relation, so that the wave's
-// loads are all in flight at once: every lane loads the four cells a finer
-// neighbour's mean needs -- a same-level or coarser neighbour's single cell
-// four times -- and keeps the mean (summed from 0.0 in row-major order, as
-// ghost_value) or the first value.
+// The cells that give the ghost of cell t of face q, as a lane of the 2D wave
+// layout gathers it (lane = 16 q + t): the one of a same-level or coarser
+// neighbour or, next to finer neighbours, the 2 x 2 block of one of them, from
+// its first cell on.
+struct ghost_cells_2d16
+{
+    size_t first;
+    bool   finer;
+
+    __device__ ghost_cells_2d16(const uint32_t* ms, const int4* nbs, int q, int t)
+    {
+        using S = patch_shape<2, 16>;
+        int c[2];
+        c[0] = (q == 0) ? -1 : (q == 1) ? 16 : t;
+        c[1] = (q == 2) ? -1 : (q == 3) ? 16 : t;
+        // the lane's own face record, selected from the four uniform ones
+        uint32_t m   = ms[0];
+        int32_t  nb  = nbs[0].x;
+        int32_t  id1 = nbs[0].y; // second fine slot of a face with finer neighbours
+#pragma unroll
+        for (int k = 1; k < 4; ++k)
+        {
+            m   = q == k ? ms[k] : m;
+            nb  = q == k ? nbs[k].x : nb;
+            id1 = q == k ? nbs[k].y : id1;
+        }
+        finer = false;
+        if (single_cell_ghosts<2>(ms))
+        {
+            first = ghost_source<2, 16>(nb, m, q, c);
+            return;
+        }
+        finer = rel_of(m) == REL_FINER;
+        if (finer)
+        {
+            // ghost_value's finer rule: fine neighbour t / 8 of the face,
+            // cells (2 t) % 16 + {0, 1} along the face, the two layers next
+            // to it
+            const int dim = q >> 1, nrm = (q & 1) ? c[dim] - 16 : c[dim] + 16;
+            int       base[2];
+            for (int d = 0; d < 2; ++d) base[d] = (((d == dim) ? nrm : c[d]) * 2) % 16;
+            const int32_t fine = (t / S::HALF) ? id1 : nb;
+            first              = static_cast<size_t>(fine) * S::NI + S::lin(base);
+        }
+        else
+            first = ghost_source<2, 16>(nb, m, q, c);
+    }
+
+    // The ghost value where the leaf has finer neighbours.  Branch-free over
+    // the relation, so that the wave's loads are all in flight at once: every
+    // lane loads the four cells a finer neighbour's mean needs -- a
+    // same-level or coarser neighbour's single cell four times -- and keeps
+    // the mean (summed from 0.0 in row-major order, as ghost_value) or the
+    // first value.
+    __device__ double value(const double* __restrict__ u) const
+    {
+        double v[4];
+#pragma unroll
+        for (int o = 0; o < 4; ++o) v[o] = u[first + (finer ? (o >> 1) * 16 + (o & 1) : 0)];
+        double sum = 0.0;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) sum += v[o];
+        return finer ? sum / 4.0 : v[0];
+    }
+};
+
 __device__ inline double gather_ghost_2d16(const double* __restrict__ u, const uint32_t* ms, const int4* nbs, int q,
                                            int t)
 {
-    using S = patch_shape<2, 16>;
-    int c[2];
-    c[0] = (q == 0) ? -1 : (q == 1) ? 16 : t;
-    c[1] = (q == 2) ? -1 : (q == 3) ? 16 : t;
-    // the lane's own face record, selected from the four uniform ones
-    uint32_t m   = ms[0];
-    int32_t  nb  = nbs[0].x;
-    int32_t  id1 = nbs[0].y; // second fine slot of a face with finer neighbours
-#pragma unroll
-    for (int k = 1; k < 4; ++k)
-    {
-        m   = q == k ? ms[k] : m;
-        nb  = q == k ? nbs[k].x : nb;
-        id1 = q == k ? nbs[k].y : id1;
-    }
-    size_t src[4];
-    if (single_cell_ghosts<2>(ms))
-        return u[ghost_source<2, 16>(nb, m, q, c)];
-    const bool finer = rel_of(m) == REL_FINER;
-    if (finer)
-    {
-        // ghost_value's finer rule: fine neighbour t / 8 of the face, cells
-        // (2 t) % 16 + {0, 1} along the face, the two layers next to it
-        const int dim = q >> 1, nrm = (q & 1) ? c[dim] - 16 : c[dim] + 16;
-        int       base[2];
-        for (int d = 0; d < 2; ++d) base[d] = (((d == dim) ? nrm : c[d]) * 2) % 16;
-        const int32_t fine = (t / S::HALF) ? id1 : nb;
-#pragma unroll
-        for (int o = 0; o < 4; ++o)
-        {
-            const int cc[2] = { base[0] + ((o >> 1) & 1), base[1] + (o & 1) };
-            src[o]          = static_cast<size_t>(fine) * S::NI + S::lin(cc);
-        }
-    }
-    else
-    {
-        const size_t one = ghost_source<2, 16>(nb, m, q, c);
-#pragma unroll
-        for (int o = 0; o < 4; ++o) src[o] = one;
-    }
-    double v[4];
-#pragma unroll
-    for (int o = 0; o < 4; ++o) v[o] = u[src[o]];
-    double sum = 0.0;
-#pragma unroll
-    for (int o = 0; o < 4; ++o) sum += v[o];
-    return finer ? sum / static_cast<double>(S::F) : v[0];
+    const ghost_cells_2d16 cells(ms, nbs, q, t);
+    return single_cell_ghosts<2>(ms) ? u[cells.first] : cells.value(u);
 }
 
 // The value of lane l - 1 (row_shr) or l + 1 (row_shl) within the lane's

@@ -98,3 +98,34 @@ def test_any_shape_tiles(amr, rank, ext):
         exp = upwind_of_padded(g, vel, s.compute_dt())
         s.advance()
         assert_fields(g.get_interior(), exp, f"{ext} step {step}")
+
+
+@pytest.mark.parametrize("vel", [(1.0, -0.5, 0.25), (-0.3, 0.0, -1.0)])
+@pytest.mark.parametrize("rank,n", [(2, 16), (3, 8)])
+def test_adjoint_wave_kernels(amr, rank, n, vel):
+    """The one-wave-per-leaf adjoint steps (one ghost layer) against the
+    any-shape ones, which serve the same patches with two ghost layers: the
+    same sums in the same order, on a tree with same-level, finer and coarser
+    faces on every side, and on the root alone."""
+    import torch
+
+    say(f"case: adjoint of {n}^{rank} patches, velocity {vel}")
+    for adapted in (True, False):
+        got = []
+        for halo in (1, 2):
+            g = amr.NdTree(rank, 4, n, halo, 200)
+            s = amr.AmrSolver(g, vel[:rank], 0.4)
+            if adapted:
+                refine_mixed(g)
+            rng = np.random.default_rng(3)
+            u0 = rng.standard_normal(g.size() * g.ni)
+            g.set_interior(u0)
+            tape = amr.Tape(s, 3, None, 0, 2)
+            u = torch.from_numpy(u0).cuda()
+            lam = torch.from_numpy(rng.standard_normal(u0.size)).cuda()
+            uT, grad = torch.empty_like(u), torch.empty_like(u)
+            tape.forward(u.data_ptr(), vel[:rank], uT.data_ptr())
+            gv = tape.adjoint(lam.data_ptr(), grad.data_ptr())
+            got.append((uT.cpu().numpy(), grad.cpu().numpy(), gv))
+        for a, b, what in zip(*got, ("uT", "grad_u0", "grad_v")):
+            assert np.array_equal(a, b), (adapted, what, np.abs(a - b).max())
