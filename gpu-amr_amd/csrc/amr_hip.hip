@@ -68,6 +68,11 @@ constexpr int block_threads(int cells)
 // rows per wave of the 2D 64^2 Euler step (k_euler_step_2d64): 16 measured
 // best on the reference's 2D benchmarks (8 and 32 within 3 %, 4 12 % slower)
 constexpr int      kEuler2d64Rows   = 16;
+// 16^2 Euler patches: one wave per leaf walking its rows from this many leaves
+// on, below that four waves per leaf with a cell per thread, the shorter chain
+// (us per step, tile / walk: 121 leaves 9.0 / 12.3, 1945 23.7 / 25.4, 7780
+// 55.8 / 47.6).
+constexpr uint32_t kEulerWalk16     = 4096;
 constexpr int      kRunLists        = 2;
 constexpr uint32_t kRunK[kRunLists] = { 4, 8 };
 struct step_aux
@@ -140,6 +145,82 @@ void for_source(const step_params* table, const uint32_t* inst, Fn&& f)
         f(std::integral_constant<int, FROM_TABLE>{});
     else
         f(std::integral_constant<int, PER_LEAF>{});
+}
+
+constexpr size_t kBoxTileBytes = 64 * 1024; // largest LDS tile of the any-shape kernels
+
+// The split of a leaf for k_euler_step_layers and its workgroup size: the
+// smallest workgroup that holds a layer, with as many strips side by side as
+// fit in it, and the fewest, hence longest, strips with
+//  - at most 16 layers each,
+//  - a wave per SIMD (a chain of layers is latency: 32^2, 130 leaves, strips
+//    of 16 / 4 layers 19.4 / 14.7 us; 523 leaves 25.9 / 23.4; 1945 leaves
+//    42.5 / 44.5),
+//  - LDS for four (2D) or three (3D) waves per SIMD, what the registers allow
+//    (12^3, 1583 leaves, strips of 12 / 6 layers 126 / 92 us),
+// but not under four layers for these: a strip forms the states of one layer
+// below and one above its own.  0 where a layer has more than 512 cells or
+// its strip exceeds 64 KiB of LDS.
+template <int R>
+int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
+{
+    const launch_box<R> B    = launch_box<R>::of(o.ext);
+    const int           cols = B.face(0);
+    int                 nt   = 0;
+    for (int t : { 64, 128, 192, 256, 512 })
+        if (!nt && cols <= t) nt = t;
+    if (!nt) return 0;
+    for (int d = 1; d < R; ++d)
+        if (!B.m[d]) return 0; // too large for the divisions by multiplication
+    const int    side_by_side = std::min(nt / cols, static_cast<int>(o.ext[0]));
+    const size_t per_wave     = (160 * 1024 / 4) / (R == 2 ? 4 : 3);
+    size_t       lds          = 0;
+    for (int g = 1;; ++g)
+    {
+        const int layers = (o.ext[0] + side_by_side * g - 1) / (side_by_side * g);
+        if (g > 1 && (layers < 4 || layers == W.layers))
+        {
+            if (layers < 4) break;
+            continue;
+        }
+        const int strips = (o.ext[0] + layers - 1) / layers;
+        W.layers         = layers;
+        W.segs           = std::min(side_by_side, strips);
+        W.groups         = static_cast<uint32_t>((strips + W.segs - 1) / W.segs);
+        lds              = static_cast<size_t>(euler_layer_lds<R>(B, W)) * sizeof(double);
+        if (layers <= 16 && static_cast<uint64_t>(n) * W.groups * (nt / 64) >= 1024 && lds <= per_wave * (nt / 64)) break;
+    }
+    W.group_quot = W.groups > 1 ? static_cast<uint32_t>(((uint64_t{ 1 } << 32) + W.groups - 1) / W.groups) : 0u;
+    const bool divides = (static_cast<uint64_t>(n) * W.groups + kXcds) * W.groups < (uint64_t{ 1 } << 32);
+    return divides && lds <= kBoxTileBytes ? nt : 0;
+}
+
+// One Euler step by k_euler_step_layers; false where the shape does not fit.
+template <int R>
+bool launch_euler_layers(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys,
+                         const face_link* links, const uint32_t* metas, euler_params const& prm, euler_scalars* sc,
+                         uint32_t reverse, uint32_t n, hipStream_t s)
+{
+    euler_walk W{};
+    const int  nt = euler_walk_for<R>(o, n, W);
+    auto       go = [&](auto threads) {
+        constexpr int             NT    = decltype(threads)::value;
+        const launch_box<R, true> B     = launch_box<R, true>::of(o.ext);
+        const uint64_t            items = static_cast<uint64_t>(n) * W.groups;
+        const size_t              lds   = static_cast<size_t>(euler_layer_lds<R>(B, W)) * sizeof(double);
+        hipLaunchKernelGGL((k_euler_step_layers<R, NT>), dim3(xcd_grid(items)), dim3(NT), lds, s, u, un, fs, keys, links,
+                           metas, n, walk_of(items, reverse), B, W, prm, sc);
+    };
+    switch (nt)
+    {
+        case 64: go(std::integral_constant<int, 64>{}); break;
+        case 128: go(std::integral_constant<int, 128>{}); break;
+        case 192: go(std::integral_constant<int, 192>{}); break;
+        case 256: go(std::integral_constant<int, 256>{}); break;
+        case 512: go(std::integral_constant<int, 512>{}); break;
+        default: return false;
+    }
+    return true;
 }
 
 template <int R, int N, int H>
@@ -292,7 +373,7 @@ struct instance
         hipLaunchKernelGGL((k_euler_dt<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, fs, keys, prm, sc, n);
         check_launch("k_euler_dt");
     }
-    static void euler_step(ops const&, const double* u, double* un, size_t fs, const uint64_t* keys, const face_link* links,
+    static void euler_step(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys, const face_link* links,
                            const uint32_t* metas, euler_params const& prm, euler_scalars* sc, uint32_t reverse,
                            uint32_t n, hipStream_t s)
     {
@@ -311,6 +392,11 @@ struct instance
             hipLaunchKernelGGL((k_euler_step_2d64<kEuler2d64Rows>), dim3(xcd_grid(static_cast<uint64_t>(n) * (64 / kEuler2d64Rows))),
                                dim3(64), 0, s, u, un, fs, keys, links, metas,
                                n, walk_of(static_cast<uint64_t>(n) * (64 / kEuler2d64Rows), reverse), prm, sc);
+        else if (R == 2 && N == 16 && n >= kEulerWalk16 &&
+                 launch_euler_layers<R>(o, u, un, fs, keys, links, metas, prm, sc, reverse, n, s))
+        {
+            // a wave per leaf walking four layers
+        }
         else if constexpr (tile_bytes <= 48 * 1024)
             hipLaunchKernelGGL((k_euler_step_tile<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, un, fs, keys, links, metas,
                                n, walk, prm, sc);
@@ -368,8 +454,6 @@ ops const* find_ops(int rank, int n, int h)
 // 64 threads for patches of up to 64 cells and 256 otherwise.  They read
 // neighbour cells from memory instead of LDS tiles; the arithmetic is the
 // fixed-shape kernels', so results are the same bits.
-constexpr size_t kBoxTileBytes = 64 * 1024; // largest LDS tile of the any-shape kernels
-
 template <int R>
 struct box_instance
 {
@@ -497,8 +581,9 @@ struct box_instance
                            uint32_t reverse, uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
-        hipLaunchKernelGGL((k_euler_step_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, u, un, fs, keys, links, metas, n,
-                           walk_of(n, reverse), shape(o), prm, sc);
+        if (!launch_euler_layers<R>(o, u, un, fs, keys, links, metas, prm, sc, reverse, n, s))
+            hipLaunchKernelGGL((k_euler_step_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, u, un, fs, keys, links,
+                               metas, n, walk_of(n, reverse), shape(o), prm, sc);
         check_launch("k_euler_step_box");
     }
     static ops table(int h, const int32_t* ext)

@@ -495,6 +495,301 @@ __global__ __launch_bounds__(NT) void k_euler_step_box(const double* __restrict_
     euler_step_leaf<R, NT>(B, u, un, fstride, keys, links, metas, prm, sc, dt, leaf);
 }
 
+// face_values with the fine cells of one field at a time in flight: all
+// fields' 2^R cells together would take the registers of two waves.
+template <int R, int NV, int D, class BX>
+__device__ inline void ghost_fields(BX const& B, const double* __restrict__ u, size_t fstride, int4 L, uint32_t meta,
+                                    int side, const int* c, double* out)
+{
+    if (rel_of(meta) != REL_FINER)
+    {
+        const size_t at = face_source<R, D>(B, L.x, meta, side, c);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) out[v] = u[v * fstride + at];
+        return;
+    }
+    const size_t first = face_fine_source<R, D>(B, L, side, c);
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+    {
+        double sum = 0.0;
+#pragma unroll
+        for (int o = 0; o < (1 << R); ++o) sum += u[v * fstride + first + fine_offset<R>(B, o)];
+        out[v] = sum / static_cast<double>(1 << R);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// How the workgroups of k_euler_step_layers split a leaf: `segs` strips of
+// `layers` layers of layout dim 0 side by side in a workgroup, `groups`
+// workgroups per leaf, with the multiplier ceil(2^32 / groups) of the
+// division by it (0 for one group).
+struct euler_walk
+{
+    int32_t  segs, layers;
+    uint32_t groups, group_quot;
+};
+
+// Doubles per cell in LDS: its fields and its state, one after another (one
+// address register per cell), an odd number so that a wave's cells spread
+// over the banks.
+template <int R>
+constexpr int euler_slot = (R + 2 + 3) | 1;
+
+// LDS of k_euler_step_layers in doubles: one layer of each strip with its
+// states, the ghosts along the dims of a layer with theirs, and the layer
+// above the patch.
+template <int R, class BX>
+__host__ __device__ inline int euler_layer_cells(BX const& B, euler_walk const& W)
+{
+    return W.segs * B.face(0);
+}
+
+template <int R, class BX>
+__host__ __device__ inline int euler_side_cells(BX const& B, euler_walk const& W)
+{
+    int per_layer = 2 * B.n(R == 2 ? 0 : 2); // cells of the two sides of a layer
+    if (R == 2) per_layer = 2;
+    if (R == 3) per_layer += 2 * B.n(1);
+    return W.segs * W.layers * per_layer;
+}
+
+template <int R, class BX>
+__host__ __device__ inline int euler_layer_lds(BX const& B, euler_walk const& W)
+{
+    return euler_slot<R> * (euler_layer_cells<R>(B, W) + euler_side_cells<R>(B, W)) + ((R + 2) | 1) * euler_layer_cells<R>(B, W);
+}
+
+// Euler step of patches of any shape whose layers (cells of one coordinate of
+// layout dim 0) fit a workgroup.  A strip of layers is walked along dim 0,
+// each thread keeping its column: the state of a cell is formed once, the
+// fluxes along dim 0 once per face, the next layer is loaded while the current
+// one is updated.  Within a layer the cells and their states are exchanged
+// through LDS; the strips' ghosts are gathered first, one per thread, with
+// their states.  Operands and expressions are the other Euler kernels', so
+// the same bits.  Bound by FP64 issue and latency as they are (k_euler_step_box
+// formed 2 R + 1 states and 2 R fluxes per cell and read every neighbour from
+// memory).  us per step on adapted trees, from memory -> by layers: 1945
+// leaves of 32^2 64 -> 43 (32 MB read and written once: 9.2 at the copy
+// rate), 523 29 -> 22.5, 484 of 48^2 49 -> 36, 1583 of 6^3 35 -> 31, of
+// 12^3 158 -> 91, of 16^3 439 -> 204.  Cells one after another in LDS, the
+// leaf's fields by uniform pointers: with fields one after another in both,
+// the addresses alone took some 60 registers and 3D spilled (12^3: 192).  Five
+// (2D) or four (3D) waves per SIMD spill: 49 and 212.
+template <int R, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 : 3))) void k_euler_step_layers(
+    const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
+    const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
+    launch_box<R, true> B, euler_walk W, euler_params prm, euler_scalars* sc)
+{
+    constexpr int NV = R + 2;
+    using EF         = euler_flux<R>;
+    extern __shared__ double lds[];
+    const uint32_t item = sweep_item(blockIdx.x, walk);
+    const double   dt   = euler_step_dt(prm, sc);
+    const uint32_t leaf = W.group_quot ? static_cast<uint32_t>((static_cast<uint64_t>(item) * W.group_quot) >> 32) : item;
+    if (leaf >= nleaves) return;
+    const int tid = threadIdx.x;
+    const int zg  = static_cast<int>(item - leaf * W.groups) * W.segs * W.layers; // first layer of the workgroup
+    // the thread's column: coordinates in the layer, strip
+    int c[R], seg, col;
+    if constexpr (R == 2)
+    {
+        seg  = B.quot(tid, 1);
+        c[1] = col = tid - seg * B.n(1);
+    }
+    else
+    {
+        const int row = B.quot(tid, 2);
+        c[2]          = tid - row * B.n(2);
+        seg           = B.quot(row, 1);
+        c[1]          = row - seg * B.n(1);
+        col           = c[1] * B.n(2) + c[2];
+    }
+    const int cols = B.face(0);
+    int       z0   = zg + seg * W.layers;
+    const bool on  = seg < W.segs && z0 < B.n(0);
+    if (!on) // a copy of the first column, for the walk only
+    {
+        z0  = zg;
+        seg = col = 0;
+        for (int d = 1; d < R; ++d) c[d] = 0;
+    }
+    const int    z1   = z0 + W.layers < B.n(0) ? z0 + W.layers : B.n(0);
+    // the leaf's fields by uniform pointers: a lane's cell is a 32-bit offset
+    const double* up[NV];
+    double*       op[NV];
+    for (int v = 0; v < NV; ++v)
+    {
+        up[v] = u + v * fstride + static_cast<size_t>(leaf) * B.ni();
+        op[v] = un + v * fstride + static_cast<size_t>(leaf) * B.ni();
+    }
+    if (!(dt > 0.0))
+    {
+        for (int z = z0; on && z < z1; ++z)
+            for (int v = 0; v < NV; ++v) op[v][col + z * cols] = up[v][col + z * cols];
+        return;
+    }
+    const int lv = key_level(keys[leaf]);
+    uint32_t  m[2 * R];
+    int4      nb[2 * R];
+    load_faces<R>(links + static_cast<size_t>(leaf) * (2 * R), metas + static_cast<size_t>(leaf) * (2 * R), m, nb);
+    double dtdx[R], smax[R];
+    for (int d = 0; d < R; ++d)
+    {
+        dtdx[d] = dt / prm.cs[lv][d];
+        smax[d] = 0.0;
+    }
+    constexpr int ST = euler_slot<R>, TOP = NV | 1;
+    const int     LC = euler_layer_cells<R>(B, W), SC = euler_side_cells<R>(B, W);
+    double*       top = lds + ST * (LC + SC);
+    auto      load_cell = [&](int z, double* U) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) U[v] = up[v][col + z * cols];
+    };
+    // the layer just outside the patch
+    auto load_outside = [&](auto side, double* U) {
+        constexpr int SIDE = decltype(side)::value;
+        int           g[R];
+        for (int d = 1; d < R; ++d) g[d] = c[d];
+        g[0] = SIDE ? B.n(0) : -1;
+        ghost_fields<R, NV, 0>(B, u, fstride, nb[SIDE], m[SIDE], SIDE, g, U);
+    };
+    auto put = [&](int t, const double* U, typename EF::state const& s) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) lds[t * ST + v] = U[v];
+        lds[t * ST + NV]     = s.inv_rho;
+        lds[t * ST + NV + 1] = s.p;
+        lds[t * ST + NV + 2] = s.a;
+    };
+    // The ghosts along dim D of a layer, side major, then strip, layer and
+    // the cell along the other dim of a layer; slot(...) of a column's own.
+    auto tangential = [&](auto dim) { return R == 2 ? 1 : B.n(3 - decltype(dim)::value); };
+    auto gather_sides = [&](auto dim, int at) {
+        constexpr int D = decltype(dim)::value, T = R == 2 ? 1 : 3 - D;
+        const int     nt = tangential(dim), per_side = W.segs * W.layers * nt;
+        for (int q = tid; q < 2 * per_side; q += NT)
+        {
+            const int side = q >= per_side ? 1 : 0, f = side ? q - per_side : q;
+            const int line = R == 2 ? f : B.quot(f, T);
+            int       g[R];
+            if constexpr (R == 3) g[T] = f - line * nt;
+            g[0] = zg + line; // strips follow each other
+            if (g[0] >= B.n(0)) continue;
+            g[D] = side ? B.n(D) : -1;
+            uint32_t mk;
+            int4     nk;
+            mk   = side ? m[2 * D + 1] : m[2 * D];
+            nk.x = side ? nb[2 * D + 1].x : nb[2 * D].x; // element by element: a choice between array elements
+            nk.y = side ? nb[2 * D + 1].y : nb[2 * D].y; // would put the array into scratch memory
+            nk.z = side ? nb[2 * D + 1].z : nb[2 * D].z;
+            nk.w = side ? nb[2 * D + 1].w : nb[2 * D].w;
+            double U[NV];
+            ghost_fields<R, NV, D>(B, u, fstride, nk, mk, side, g, U);
+            put(at + q, U, EF::state_of(U, prm.gamma));
+        }
+    };
+    // where the column's neighbours along dim D of a layer are in LDS: own
+    // slot -+ the stride, or a ghost's, which moves on with the layer
+    const int own = seg * cols + col;
+    int       lo[R], hi[R], dlo[R], dhi[R];
+    auto      neighbours = [&](auto dim, int at) {
+        constexpr int D  = decltype(dim)::value;
+        const int     nt = tangential(dim), s = R == 3 && D == 1 ? B.n(2) : 1;
+        const int     gh = at + (seg * W.layers) * nt + (R == 3 ? c[3 - D] : 0);
+        const bool    low = c[D] == 0, high = c[D] == B.n(D) - 1;
+        lo[D]  = low ? gh : own - s;
+        dlo[D] = low ? nt : 0;
+        hi[D]  = high ? gh + W.segs * W.layers * nt : own + s;
+        dhi[D] = high ? nt : 0;
+    };
+    double Uc[NV], fz[NV];
+    {
+        double Ul[NV], Ut[NV];
+        load_cell(z0, Uc);
+        if (z0 > 0)
+            load_cell(z0 - 1, Ul);
+        else
+            load_outside(std::integral_constant<int, 0>{}, Ul);
+        if (on && z1 == B.n(0))
+        {
+            load_outside(std::integral_constant<int, 1>{}, Ut);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) top[own * TOP + v] = Ut[v];
+        }
+        EF::rusanov(Ul, EF::state_of(Ul, prm.gamma), Uc, EF::state_of(Uc, prm.gamma), fz, R - 1);
+    }
+    gather_sides(std::integral_constant<int, 1>{}, LC);
+    neighbours(std::integral_constant<int, 1>{}, LC);
+    if constexpr (R == 3)
+    {
+        const int at = LC + 2 * W.segs * W.layers * B.n(2);
+        gather_sides(std::integral_constant<int, 2>{}, at);
+        neighbours(std::integral_constant<int, 2>{}, at);
+    }
+    auto stc = EF::state_of(Uc, prm.gamma);
+    for (int k = 0; k < W.layers; ++k)
+    {
+        const int  z    = z0 + k < z1 ? z0 + k : z1 - 1;
+        const bool mine = on && z0 + k < z1;
+        if (on) put(own, Uc, stc);
+        double Un[NV];
+        if (z + 1 < B.n(0)) load_cell(z + 1, Un);
+        __syncthreads();
+        double total[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) total[v] = 0.0;
+#pragma unroll
+        for (int d = 0; d < R - 1; ++d)
+        {
+            const int j = R - 1 - d;
+            double    Us[NV], fL[NV], fR[NV];
+            auto      side = [&](int t) -> typename EF::state {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) Us[v] = lds[t * ST + v];
+                return { lds[t * ST + NV], lds[t * ST + NV + 1], lds[t * ST + NV + 2] };
+            };
+            const auto sl = side(lo[j]);
+            EF::rusanov(Us, sl, Uc, stc, fL, d);
+            const auto sr = side(hi[j]);
+            EF::rusanov(Uc, stc, Us, sr, fR, d);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) total[v] -= dtdx[d] * (fR[v] - fL[v]);
+            lo[j] += dlo[j];
+            hi[j] += dhi[j];
+        }
+        __syncthreads();
+        if (z + 1 >= B.n(0))
+        {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) Un[v] = top[own * TOP + v];
+        }
+        const auto stn = EF::state_of(Un, prm.gamma);
+        double     fR[NV], o[NV];
+        EF::rusanov(Uc, stc, Un, stn, fR, R - 1);
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+        {
+            total[v] -= dtdx[R - 1] * (fR[v] - fz[v]);
+            o[v] = Uc[v] + total[v];
+        }
+        if (mine)
+        {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) op[v][col + z * cols] = o[v];
+            if (prm.next_dt) cell_speeds<R>(o, prm.gamma, smax);
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+        {
+            Uc[v] = Un[v];
+            fz[v] = fR[v];
+        }
+        stc = stn;
+    }
+    if (prm.next_dt) fold_speed_max<R, NT>(smax, prm.cs[lv], sc + prm.next);
+}
+
 // k_euler_step with the leaf's fields staged in LDS: every field's (n+2)^R
 // tile (interior plus face ghosts, gathered once per ghost cell by the same
 // rules) is loaded cooperatively, then each cell reads its neighbours from

@@ -129,3 +129,110 @@ def test_adjoint_wave_kernels(amr, rank, n, vel):
             got.append((uT.cpu().numpy(), grad.cpu().numpy(), gv))
         for a, b, what in zip(*got, ("uT", "grad_u0", "grad_v")):
             assert np.array_equal(a, b), (adapted, what, np.abs(a - b).max())
+
+
+def euler_step_of_padded(tree, gamma, dt):
+    """One Euler step in numpy from the library's padded patches, in the
+    expression order of rusanovFlux and time_step_cpu."""
+    pad = tree.get_patches()  # [fields, leaves, ...]
+    level = (tree.keys() & np.uint64(63)).astype(np.int64)
+    cs = tree.cell_sizes(level)
+    h, rank = tree.halo, tree.rank
+    core = tuple(slice(h, -h) for _ in range(rank))
+
+    def shifted(d, by):
+        j = rank - 1 - d
+        at = list(core)
+        at[j] = slice(h + by, pad.shape[2 + j] - h + by)
+        return pad[(slice(None), slice(None), *at)]
+
+    def state(U):
+        inv = 1.0 / U[0]
+        kin = np.zeros_like(inv)
+        for d in range(rank):
+            kin = kin + U[1 + d] * U[1 + d]
+        kin = kin * (0.5 * inv)
+        p = (gamma - 1.0) * (U[rank + 1] - kin)
+        return inv, p, np.sqrt(gamma * p * inv)
+
+    def flux(UL, L, UR, Rt, d):
+        ul, ur = UL[1 + d] * L[0], UR[1 + d] * Rt[0]
+        sl, sr = np.abs(ul) + L[2], np.abs(ur) + Rt[2]
+        smax = np.where(sl < sr, sr, sl)
+        out = np.empty_like(UL)
+        out[0] = 0.5 * (UL[1 + d] + UR[1 + d] - smax * (UR[0] - UL[0]))
+        for k in range(rank):
+            fl, fr = UL[1 + k] * ul, UR[1 + k] * ur
+            if k == d:
+                fl, fr = fl + L[1], fr + Rt[1]
+            out[1 + k] = 0.5 * (fl + fr - smax * (UR[1 + k] - UL[1 + k]))
+        fl, fr = ul * (UL[rank + 1] + L[1]), ur * (UR[rank + 1] + Rt[1])
+        out[rank + 1] = 0.5 * (fl + fr - smax * (UR[rank + 1] - UL[rank + 1]))
+        return out
+
+    U = pad[(slice(None), slice(None), *core)]
+    sU, total = state(U), np.zeros_like(U)
+    for d in range(rank):
+        lo, hi = shifted(d, -1), shifted(d, 1)
+        left, right = flux(lo, state(lo), U, sU, d), flux(U, sU, hi, state(hi), d)
+        total -= (dt / cs[:, d]).reshape((1, -1) + (1,) * rank) * (right - left)
+    return U + total
+
+
+# (rank, extents): one strip and several, strips that end early, idle lanes, a
+# layer as wide as the workgroup, one too wide for it, and one whose strip is
+# too large for LDS (both from memory)
+EULER_BOXES = [(2, (2, 2)), (2, (2, 128)), (2, (130, 4)), (2, (32, 32)), (2, (22, 40)), (2, (6, 300)), (2, (4, 516)),
+               (3, (2, 2, 2)), (3, (12, 10, 6)), (3, (4, 6, 8)), (3, (6, 16, 16)), (3, (16, 16, 16)), (3, (2, 4, 30)),
+               (3, (10, 16, 32)), (3, (4, 24, 24))]
+
+
+@pytest.mark.parametrize("rank,ext", EULER_BOXES)
+def test_any_shape_euler(amr, rank, ext):
+    """Euler steps of any-shape patches, one call and a batch, on a tree with
+    same-level, finer and coarser faces."""
+    say(f"case: any-shape Euler {ext}")
+    rng = np.random.default_rng(sum(ext))
+    s, batch = (amr.EulerSolver(rank, 4, ext, 1, 200, (1.0,) * rank, 1.4, 0.3) for _ in range(2))
+    for t in (s.tree, batch.tree):
+        refine_mixed(t)
+    t = s.tree
+    u0 = np.empty((t.fields, t.size() * t.ni))
+    u0[0] = rng.uniform(0.5, 1.5, u0.shape[1])
+    u0[1:-1] = rng.uniform(-0.5, 0.5, u0[1:-1].shape)
+    u0[-1] = rng.uniform(2.0, 4.0, u0.shape[1])
+    for x in (s, batch):
+        x.tree.set_interior(u0)
+    time = 0.0
+    for step in range(3):
+        with np.errstate(all="ignore"):  # the corners of the padded patches are 0
+            exp = euler_step_of_padded(t, 1.4, s.compute_dt())
+        time += s.advance()
+        assert_fields(t.get_interior(), exp, f"{ext} step {step}")
+    batch.advance_batch_async(3)
+    assert batch.finish_advance_batch() == (time, 3)
+    assert_fields(batch.tree.get_interior(), t.get_interior(), f"{ext} batch")
+
+
+@pytest.mark.parametrize("n", [4093, 4096])
+def test_euler_walk_16(amr, n):
+    """16^2 patches on both sides of the leaf count from which a wave walks a
+    leaf."""
+    say(f"case: Euler 16^2, {n} leaves")
+    s = amr.EulerSolver(2, 7, 16, 1, 4200, (1.0, 1.0), 1.4, 0.3)
+    t = s.tree
+    for _ in range(6):
+        t.refine_all()
+    if n < 4096:  # one family coarsened
+        flags = np.zeros(t.size(), dtype=np.int8)
+        flags[:4] = amr.COARSEN
+        assert t.reconstruct_tree(flags)
+    assert t.size() == n
+    rng = np.random.default_rng(n)
+    u0 = np.empty((4, t.size() * t.ni))
+    u0[0], u0[1:3], u0[3] = rng.uniform(0.5, 1.5, u0.shape[1]), rng.uniform(-0.5, 0.5, u0[1:3].shape), 3.0
+    t.set_interior(u0)
+    with np.errstate(all="ignore"):
+        exp = euler_step_of_padded(t, 1.4, s.compute_dt())
+    s.advance()
+    assert_fields(t.get_interior(), exp, f"{t.size()} leaves")
