@@ -128,3 +128,38 @@ def test_batch_run_variant_with_graphs_and_switches(amr):
         bt.scatter()
         for k, t in enumerate(trees):
             assert np.array_equal(t.get_interior().view(np.uint64), exp[k].view(np.uint64)), f"plan step {i} instance {k}"
+
+
+@pytest.mark.parametrize("rank,n,level", [(2, 16, 7), (3, 8, 5), (2, 64, 5)])
+def test_batch_larger_than_the_cache_matches_sequential(amr, rank, n, level):
+    """A batch that is stepped in several groups of instances: uneven trees,
+    odd and even step counts, eager and graph launches, per-leaf and run
+    kernels."""
+    say(f"case: batch of {n}^{rank} patches in several groups")
+    cells = n**rank
+    solvers = []
+    leaves = 0
+    rng = np.random.default_rng(level)
+    while leaves * cells * 16 < 460e6:  # groups hold at most 224 MiB
+        k = level if len(solvers) % 3 else level - 1
+        tree = amr.NdTree(rank, level, n, 1, (1 << (rank * k)) + 1)
+        solvers.append(amr.AmrSolver(tree, tuple(rng.uniform(-1.0, 1.0, rank)), 0.4))
+        for _ in range(k):
+            tree.refine_all()
+        tree.set_interior(rng.standard_normal(tree.size() * tree.ni))
+        leaves += tree.size()
+    batch = amr.Batch([s.tree for s in solvers])
+    steps = 0
+    for variant, count, graph in ((0, 3, True), (4 if n < 64 else 0, 2, False), (0, 1, False), (0, 3, True)):
+        batch.set_step_variant(variant)
+        batch.advance(count, use_graph=graph)
+        steps += count
+    batch.synchronize()
+    expected = []
+    for s in solvers:
+        s.advance_batch_async(steps)
+        s.finish_advance_batch()
+        expected.append(s.tree.get_interior().copy())
+    batch.scatter()
+    for i, (s, u) in enumerate(zip(solvers, expected)):
+        assert np.array_equal(s.tree.get_interior().view(np.uint64), u.view(np.uint64)), f"instance {i}"
