@@ -656,7 +656,7 @@ __global__ __launch_bounds__(64) void k_adj_step_3d8(const double* __restrict__ 
         acc = xm ? t : acc;
         t   = acc + hface[3][z * 8 + y];
         acc = xp ? t : acc;
-        out[z * 64 + lane] = acc;
+        store_cell<false>(out + z * 64 + lane, acc);
         const double uxm = lane_minus1(uc), uxp = lane_plus1(uc);
         const double uym = __shfl_up(uc, 8, 64), uyp = __shfl_down(uc, 8, 64);
         const double lx = x == 0 ? gface[2][z * 8 + y] : uxm, hx = x == 7 ? gface[3][z * 8 + y] : uxp;
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(64) void k_adj_step_2d16(const double* __restrict__
         acc = xm ? t : acc;
         t   = acc + hface[3][y];
         acc = xp ? t : acc;
-        out[y * 16 + x] = acc;
+        store_cell<false>(out + y * 16 + x, acc);
         const double uxm = lane_minus1(uc), uxp = lane_plus1(uc);
         const double lx = x == 0 ? gface[2][y] : uxm, hx = x == 15 ? gface[3][y] : uxp;
         const double ly = j > 0 ? r[j > 0 ? j - 1 : 0] : (q == 0 ? gface[0][x] : uup);

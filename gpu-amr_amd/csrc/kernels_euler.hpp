@@ -776,7 +776,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 :
         if (mine)
         {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) op[v][col + z * cols] = o[v];
+            for (int v = 0; v < NV; ++v) store_cell<false>(op[v] + (col + z * cols), o[v]);
             if (prm.next_dt) cell_speeds<R>(o, prm.gamma, smax);
         }
 #pragma unroll
