@@ -696,7 +696,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 :
     auto      neighbours = [&](auto dim, int at) {
         constexpr int D  = decltype(dim)::value;
         const int     nt = tangential(dim), s = R == 3 && D == 1 ? B.n(2) : 1;
-        const int     gh = at + (seg * W.layers) * nt + (R == 3 ? c[3 - D] : 0);
+        int           gh = at + (seg * W.layers) * nt;
+        if constexpr (R == 3) gh += c[3 - D];
         const bool    low = c[D] == 0, high = c[D] == B.n(D) - 1;
         lo[D]  = low ? gh : own - s;
         dlo[D] = low ? nt : 0;
