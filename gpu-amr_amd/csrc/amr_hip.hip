@@ -114,10 +114,10 @@ struct ops
     // two fused steps of a single-level tree (null: not built for the shape)
     void (*step2)(const double*, double*, step2_params const&, uint32_t level, uint32_t reverse, uint32_t, hipStream_t);
     // Euler fields (field-major, stride fstride doubles between fields)
-    void (*euler_dt)(ops const&, const double*, size_t, const uint64_t*, euler_params const&, euler_scalars*, uint32_t,
+    void (*euler_dt)(ops const&, const double*, size_t, const uint64_t*, euler_params const&, euler_slot*, uint32_t,
                      hipStream_t);
     void (*euler_step)(ops const&, const double*, double*, size_t, const uint64_t*, const face_link*, const uint32_t*,
-                       euler_params const&, euler_scalars*, uint32_t reverse, uint32_t, hipStream_t);
+                       euler_params const&, euler_slot*, uint32_t reverse, uint32_t, hipStream_t);
 
     int ni() const { return (rank == 2) ? ext[0] * ext[1] : ext[0] * ext[1] * ext[2]; }
     int padded_cells() const
@@ -198,7 +198,7 @@ int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
 // One Euler step by k_euler_step_layers; false where the shape does not fit.
 template <int R>
 bool launch_euler_layers(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys,
-                         const face_link* links, const uint32_t* metas, euler_params const& prm, euler_scalars* sc,
+                         const face_link* links, const uint32_t* metas, euler_params const& prm, euler_slot* sc,
                          uint32_t reverse, uint32_t n, hipStream_t s)
 {
     euler_walk W{};
@@ -366,7 +366,7 @@ struct instance
         }
         check_launch("k_step2");
     }
-    static void euler_dt(ops const&, const double* u, size_t fs, const uint64_t* keys, euler_params const& prm, euler_scalars* sc,
+    static void euler_dt(ops const&, const double* u, size_t fs, const uint64_t* keys, euler_params const& prm, euler_slot* sc,
                          uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
@@ -374,7 +374,7 @@ struct instance
         check_launch("k_euler_dt");
     }
     static void euler_step(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys, const face_link* links,
-                           const uint32_t* metas, euler_params const& prm, euler_scalars* sc, uint32_t reverse,
+                           const uint32_t* metas, euler_params const& prm, euler_slot* sc, uint32_t reverse,
                            uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
@@ -569,7 +569,7 @@ struct box_instance
         check_launch("k_adj_regrid_box");
     }
     static void euler_dt(ops const& o, const double* u, size_t fs, const uint64_t* keys, euler_params const& prm,
-                         euler_scalars* sc, uint32_t n, hipStream_t s)
+                         euler_slot* sc, uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
         hipLaunchKernelGGL((k_euler_dt_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, shape(o), u, fs, keys, prm, sc,
@@ -577,7 +577,7 @@ struct box_instance
         check_launch("k_euler_dt_box");
     }
     static void euler_step(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys,
-                           const face_link* links, const uint32_t* metas, euler_params const& prm, euler_scalars* sc,
+                           const face_link* links, const uint32_t* metas, euler_params const& prm, euler_slot* sc,
                            uint32_t reverse, uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
@@ -848,16 +848,19 @@ struct host_mailbox
 {
     regrid_summary summary;
     euler_scalars  esc;
+    double         min; // the slot's minimum, when asked for
     uint32_t       seq;
     uint32_t       pad[3];
 };
 
-__global__ void k_publish(const regrid_summary* __restrict__ s, const euler_scalars* __restrict__ e,
-                          host_mailbox* box, uint32_t seq)
+__global__ void k_publish(const regrid_summary* __restrict__ s, const euler_slot* __restrict__ e,
+                          bool want_min, host_mailbox* box, uint32_t seq)
 {
+    const double min = want_min ? euler_min(*e) : 0.0;
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     if (s) box->summary = *s;
-    if (e) box->esc = *e;
+    if (e) box->esc = e->sums;
+    if (want_min) box->min = min;
     __threadfence_system();
     __hip_atomic_store(&box->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -914,7 +917,7 @@ struct amr_ctx
     // field-major (field v of slot s at u + v * fstride() + s * ni)
     int             nvar  = 1;
     double          gamma = 1.4;
-    euler_scalars*  esc   = nullptr; // the kEulerSlots device scalars of the dt logic
+    euler_slot*     esc   = nullptr; // the kEulerSlots device scalars of the dt logic
     uint32_t        euler_last = 1;  // slot with the last batch's sums
     bool            euler_cut  = false; // a launch of the last batch failed: slot 0 may not be empty
     size_t          fstride() const { return static_cast<size_t>(cap) * static_cast<size_t>(ni); }
@@ -960,10 +963,10 @@ struct amr_ctx
     // null): spins on the mailbox's sequence number for up to
     // kMailboxSpinUs, then synchronizes the stream (which also reports a
     // failure of the queued work).
-    void publish_wait(const regrid_summary* s, const euler_scalars* e)
+    void publish_wait(const regrid_summary* s, const euler_slot* e, bool want_min = false)
     {
         const uint32_t want = ++box_seq;
-        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, stream, s, e, box, want);
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, stream, s, e, want_min, box, want);
         check_launch("k_publish");
         const auto t0 = std::chrono::steady_clock::now();
         for (uint32_t i = 1;; ++i)
@@ -1144,7 +1147,7 @@ struct amr_ctx
 
     void euler_clear(uint32_t slot)
     {
-        hipLaunchKernelGGL(k_euler_clear, dim3(1), dim3(1), 0, stream, esc + slot);
+        hipLaunchKernelGGL(k_euler_clear, dim3(1), dim3(64), 0, stream, esc + slot);
         check_launch("k_euler_clear");
     }
 
@@ -1164,10 +1167,8 @@ struct amr_ctx
         prm.next = kEulerNowSlot;
         prm.clear = 3; // free outside a batch's steps
         op->euler_dt(*op, u[cur], fstride(), keys[kc], prm, esc, static_cast<uint32_t>(n), stream);
-        const euler_scalars e = euler_read(kEulerNowSlot);
-        double raw;
-        std::memcpy(&raw, &e.dtmin_bits, sizeof(raw));
-        return cfl * raw;
+        publish_wait(nullptr, esc + kEulerNowSlot, true);
+        return cfl * box->min;
     }
 
     void scan(uint32_t count) { exclusive_scan(counts, pos, count, block_sums, summary, stream); }
@@ -1952,7 +1953,7 @@ int amr_euler_create(const amr_tree_config* cfg, double gamma, double cfl, amr_c
             auto c   = create_ctx(cfg, cfg->rank + 2);
             c->gamma = gamma;
             c->cfl   = cfl;
-            c->esc   = dev_alloc<euler_scalars>(kEulerSlots);
+            c->esc   = dev_alloc<euler_slot>(kEulerSlots);
             for (uint32_t k = 0; k < kEulerSlots; ++k) c->euler_clear(k);
             *out = c.release();
         }

@@ -19,10 +19,10 @@ namespace amrhip
 {
 
 // Device scalars of the dt logic (the CPU loop of amr_solver.hpp:221-241):
-// the running minimum of dx / speed (as the bits of a non-negative double, so
-// that an integer atomicMin orders it), the summed dt, the remaining time,
-// the executed step count and a stop flag (the loop's break).  A context
-// holds kEulerSlots of them: the first step of a batch takes its dt from
+// the summed dt, the remaining time, the executed step count and a stop flag
+// (the loop's break) and the running minimum of dx / speed (as the bits of a
+// non-negative double, so that an integer atomicMin orders it) in
+// kEulerParts parts.  A context holds kEulerSlots of them: the first step of a batch takes its dt from
 // slot 0, which k_euler_dt filled, the later ones from slots 1, 2, 3 in turn.
 // A step launch reads its own slot, folds the next step's minimum and writes
 // the sums into the next one and empties the minimum of the one after that,
@@ -33,12 +33,31 @@ namespace amrhip
 // regrids included).
 struct euler_scalars
 {
-    uint64_t dtmin_bits;
     double   acc;
     double   remaining;
     uint64_t executed;
     uint32_t stopped;
     uint32_t pad;
+};
+
+// The parts of the minimum, a cache line and an XCD each (workgroups go to
+// the XCDs in turn): a workgroup folds into its part without looking at it
+// first, so it ends without a round trip.  With one minimum for all, read
+// before the atomic to keep most workgroups from it, the waves that end
+// together all found it unset and queued on one address, 4.5 ns each.  us per
+// step, one minimum -> parts: 1945 leaves of 16^2 22.8 -> 17.7, 130 / 523 of
+// 32^2 14.7 / 21.3 -> 13.1 / 19.3, 121 / 775 of 64^2 21.0 / 51.2 -> 17.9 /
+// 48.3, 512 / 7659 of 8^3 21.1 / 111.9 -> 17.8 / 107; 1024 of 64^2 and 32768
+// of 8^3 unchanged; 16 or 32 parts no better (every wave reads them all).
+constexpr uint32_t kEulerParts = kXcds;
+
+struct alignas(128) euler_slot
+{
+    euler_scalars sums;
+    struct alignas(128) part
+    {
+        uint64_t bits;
+    } min[kEulerParts];
 };
 
 constexpr uint32_t kEulerNowSlot = 4; // amr_solver_compute_dt's minimum
@@ -62,6 +81,37 @@ struct euler_params
 
 // An empty minimum: the largest double (compute_time_step_cpu's start value).
 constexpr uint64_t kEulerNoMinimum = 0x7FEFFFFFFFFFFFFFull;
+
+// A value every lane holds alike, read from the first active lane into
+// scalar registers (the VALU result of a uniform division otherwise holds
+// vector registers).
+__device__ inline double wave_uniform(double v)
+{
+    const uint64_t b  = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b >> 32));
+    return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
+}
+
+// Empties a slot's minimum; for the first wave of a workgroup.
+__device__ inline void euler_empty_min(euler_slot& slot)
+{
+    if (threadIdx.x < kEulerParts) slot.min[threadIdx.x].bits = kEulerNoMinimum;
+}
+
+// A slot's minimum in every lane; all 64 lanes must be active.
+__device__ inline double euler_min(euler_slot const& slot)
+{
+    static_assert((kEulerParts & (kEulerParts - 1)) == 0 && kEulerParts <= 32, "a power of two");
+    double v = __longlong_as_double(static_cast<long long>(slot.min[threadIdx.x % kEulerParts].bits));
+#pragma unroll
+    for (int o = kEulerParts / 2; o > 0; o >>= 1)
+    {
+        const double w = __shfl_xor(v, o, 64);
+        v              = (w < v) ? w : v;
+    }
+    return v;
+}
 
 template <int R>
 struct euler_flux
@@ -275,7 +325,7 @@ __device__ inline void cell_speeds(const double* U, double gamma, double* smax)
 // Folded into the launch-wide minimum; every lane of the workgroup must call
 // it.
 template <int R, int NT>
-__device__ inline void fold_speed_max(double* smax, const double* cs, euler_scalars* __restrict__ sc)
+__device__ inline void fold_speed_max(double* smax, const double* cs, euler_slot* __restrict__ sc)
 {
     for (int d = 0; d < R; ++d)
         for (int off = 32; off > 0; off >>= 1)
@@ -309,13 +359,9 @@ __device__ inline void fold_speed_max(double* smax, const double* cs, euler_scal
                 dt             = (q < dt) ? q : dt;
             }
         }
-        // non-negative doubles order like their bit patterns; most
-        // workgroups do not lower the minimum and skip the atomic (a stale
-        // read only costs an extra one), which keeps thousands of
-        // workgroups from queueing on one address
-        const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(dt));
-        if (bits < *reinterpret_cast<volatile unsigned long long*>(&sc->dtmin_bits))
-            atomicMin(reinterpret_cast<unsigned long long*>(&sc->dtmin_bits), bits);
+        // non-negative doubles order like their bit patterns
+        atomicMin(reinterpret_cast<unsigned long long*>(&sc->min[blockIdx.x % kEulerParts].bits),
+                  static_cast<unsigned long long>(__double_as_longlong(dt)));
     }
 }
 
@@ -326,7 +372,7 @@ __device__ inline void fold_speed_max(double* smax, const double* cs, euler_scal
 template <int R, int NT, class BX>
 __device__ inline void euler_dt_leaf(BX const& B, const double* __restrict__ u, size_t fstride,
                                      const uint64_t* __restrict__ keys, euler_params const& prm,
-                                     euler_scalars* sc, uint32_t leaf)
+                                     euler_slot* sc, uint32_t leaf)
 {
     constexpr int NV = R + 2;
     const int     ni = B.ni();
@@ -345,11 +391,11 @@ __device__ inline void euler_dt_leaf(BX const& B, const double* __restrict__ u, 
 template <int R, int N, int NT>
 __global__ __launch_bounds__(NT) void k_euler_dt(const double* __restrict__ u, size_t fstride,
                                                  const uint64_t* __restrict__ keys, euler_params prm,
-                                                 euler_scalars* sc, uint32_t nleaves)
+                                                 euler_slot* sc, uint32_t nleaves)
 {
     constexpr box<R> B    = box<R>::cube(N);
     const uint32_t   leaf = xcd_item(blockIdx.x, gridDim.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc[prm.clear].dtmin_bits = kEulerNoMinimum;
+    if (blockIdx.x == 0) euler_empty_min(sc[prm.clear]);
     if (leaf >= nleaves) return;
     euler_dt_leaf<R, NT>(B, u, fstride, keys, prm, sc + prm.next, leaf);
 }
@@ -358,10 +404,10 @@ __global__ __launch_bounds__(NT) void k_euler_dt(const double* __restrict__ u, s
 template <int R, int NT>
 __global__ __launch_bounds__(NT) void k_euler_dt_box(launch_box<R> B, const double* __restrict__ u, size_t fstride,
                                                      const uint64_t* __restrict__ keys, euler_params prm,
-                                                     euler_scalars* sc, uint32_t nleaves)
+                                                     euler_slot* sc, uint32_t nleaves)
 {
     const uint32_t leaf = xcd_item(blockIdx.x, gridDim.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) sc[prm.clear].dtmin_bits = kEulerNoMinimum;
+    if (blockIdx.x == 0) euler_empty_min(sc[prm.clear]);
     if (leaf >= nleaves) return;
     euler_dt_leaf<R, NT>(B, u, fstride, keys, prm, sc + prm.next, leaf);
 }
@@ -370,10 +416,10 @@ __global__ __launch_bounds__(NT) void k_euler_dt_box(launch_box<R> B, const doub
 // the same operations (amr_solver.hpp:225-241): 0 and stop when the remaining
 // time is used up, else min(cfl * dtmin, remaining).  The first workgroup
 // writes the sums the next step (or the host) reads.
-__device__ inline double euler_step_dt(euler_params const& prm, euler_scalars* ring)
+__device__ inline double euler_step_dt(euler_params const& prm, euler_slot* ring)
 {
-    const euler_scalars& now       = ring[prm.now];
-    const double         raw       = __longlong_as_double(static_cast<long long>(now.dtmin_bits));
+    const euler_scalars& now       = ring[prm.now].sums;
+    const double         raw       = wave_uniform(euler_min(ring[prm.now]));
     const double         remaining = prm.first ? prm.remaining : now.remaining;
     const uint32_t       stopped   = prm.first ? 0u : now.stopped;
     double               step_dt   = 0.0;
@@ -385,26 +431,28 @@ __device__ inline double euler_step_dt(euler_params const& prm, euler_scalars* r
     const bool stop = step_dt <= 0.0;
     if (blockIdx.x == 0 && threadIdx.x == 0)
     {
-        euler_scalars& next     = ring[prm.next];
+        euler_scalars& next     = ring[prm.next].sums;
         const double   acc      = prm.first ? 0.0 : now.acc;
         const uint64_t executed = prm.first ? 0u : now.executed;
         next.acc                = stop ? acc : acc + step_dt;
         next.remaining          = stop ? remaining : remaining - step_dt;
         next.executed           = stop ? executed : executed + 1;
         next.stopped            = stop ? 1u : 0u;
-        ring[prm.clear].dtmin_bits = kEulerNoMinimum;
-        if (prm.clear_dt) ring[0].dtmin_bits = kEulerNoMinimum;
+    }
+    if (blockIdx.x == 0)
+    {
+        euler_empty_min(ring[prm.clear]);
+        if (prm.clear_dt) euler_empty_min(ring[0]);
     }
     return stop ? 0.0 : step_dt;
 }
 
 // Empties one slot (a kernel, not a memset, so that a captured graph replays
 // it).
-__global__ void k_euler_clear(euler_scalars* __restrict__ slot)
+__global__ __launch_bounds__(64) void k_euler_clear(euler_slot* __restrict__ slot)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    *slot            = euler_scalars{};
-    slot->dtmin_bits = kEulerNoMinimum;
+    if (threadIdx.x == 0) slot->sums = euler_scalars{};
+    euler_empty_min(*slot);
 }
 
 // time_step_cpu (amr_solver.hpp:265-353) for the Euler fields: per cell and
@@ -416,7 +464,7 @@ template <int R, int NT, class BX>
 __device__ inline void euler_step_leaf(BX const& B, const double* __restrict__ u, double* __restrict__ un,
                                        size_t fstride, const uint64_t* __restrict__ keys,
                                        const face_link* __restrict__ links, const uint32_t* __restrict__ metas,
-                                       euler_params const& prm, euler_scalars* sc, double dt, uint32_t leaf)
+                                       euler_params const& prm, euler_slot* sc, double dt, uint32_t leaf)
 {
     constexpr int NV   = R + 2;
     const int     ni   = B.ni();
@@ -472,7 +520,7 @@ __global__ __launch_bounds__(NT) void k_euler_step(const double* __restrict__ u,
                                                    size_t fstride, const uint64_t* __restrict__ keys,
                                                    const face_link* __restrict__ links,
                                                    const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    euler_params prm, euler_scalars* sc)
+    euler_params prm, euler_slot* sc)
 {
     constexpr box<R> B    = box<R>::cube(N);
     const uint32_t   leaf = sweep_item(blockIdx.x, walk);
@@ -487,7 +535,7 @@ __global__ __launch_bounds__(NT) void k_euler_step_box(const double* __restrict_
                                                        size_t fstride, const uint64_t* __restrict__ keys,
                                                        const face_link* __restrict__ links,
                                                        const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    launch_box<R> B, euler_params prm, euler_scalars* sc)
+    launch_box<R> B, euler_params prm, euler_slot* sc)
 {
     const uint32_t leaf = sweep_item(blockIdx.x, walk);
     const double   dt   = euler_step_dt(prm, sc);
@@ -534,7 +582,7 @@ struct euler_walk
 // address register per cell), an odd number so that a wave's cells spread
 // over the banks.
 template <int R>
-constexpr int euler_slot = (R + 2 + 3) | 1;
+constexpr int euler_cell_slot = (R + 2 + 3) | 1;
 
 // LDS of k_euler_step_layers in doubles: one layer of each strip with its
 // states, the ghosts along the dims of a layer with theirs, and the layer
@@ -557,7 +605,7 @@ __host__ __device__ inline int euler_side_cells(BX const& B, euler_walk const& W
 template <int R, class BX>
 __host__ __device__ inline int euler_layer_lds(BX const& B, euler_walk const& W)
 {
-    return euler_slot<R> * (euler_layer_cells<R>(B, W) + euler_side_cells<R>(B, W)) + ((R + 2) | 1) * euler_layer_cells<R>(B, W);
+    return euler_cell_slot<R> * (euler_layer_cells<R>(B, W) + euler_side_cells<R>(B, W)) + ((R + 2) | 1) * euler_layer_cells<R>(B, W);
 }
 
 // Euler step of patches of any shape whose layers (cells of one coordinate of
@@ -580,7 +628,7 @@ template <int R, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 : 3))) void k_euler_step_layers(
     const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
     const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    launch_box<R, true> B, euler_walk W, euler_params prm, euler_scalars* sc)
+    launch_box<R, true> B, euler_walk W, euler_params prm, euler_slot* sc)
 {
     constexpr int NV = R + 2;
     using EF         = euler_flux<R>;
@@ -640,7 +688,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 :
         dtdx[d] = dt / prm.cs[lv][d];
         smax[d] = 0.0;
     }
-    constexpr int ST = euler_slot<R>, TOP = NV | 1;
+    constexpr int ST = euler_cell_slot<R>, TOP = NV | 1;
     const int     LC = euler_layer_cells<R>(B, W), SC = euler_side_cells<R>(B, W);
     double*       top = lds + ST * (LC + SC);
     auto      load_cell = [&](int z, double* U) {
@@ -800,7 +848,7 @@ __global__ __launch_bounds__(NT) void k_euler_step_tile(const double* __restrict
                                                         size_t fstride, const uint64_t* __restrict__ keys,
                                                         const face_link* __restrict__ links,
                                                         const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    euler_params prm, euler_scalars* sc)
+    euler_params prm, euler_slot* sc)
 {
     using S          = patch_shape<R, N>;
     using T          = tile_shape<R, N>;
@@ -859,17 +907,6 @@ __global__ __launch_bounds__(NT) void k_euler_step_tile(const double* __restrict
     if (prm.next_dt) fold_speed_max<R, NT>(smax, prm.cs[key_level(keys[leaf])], sc + prm.next);
 }
 
-// A value every lane holds alike, read from the first active lane into
-// scalar registers (the VALU result of a uniform division otherwise holds
-// vector registers).
-__device__ inline double wave_uniform(double v)
-{
-    const uint64_t b  = __double_as_longlong(v);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b));
-    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(b >> 32));
-    return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
-}
-
 // The five conservative values and the state of one cell moved across
 // lanes as 64-bit DPP rows (lane_plus1) or LDS permutes (__shfl_down by 8),
 // every lane active.
@@ -925,7 +962,7 @@ template <bool NTS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_euler_step_3d8(
     const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
     const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    euler_params prm, euler_scalars* sc)
+    euler_params prm, euler_slot* sc)
 {
     using F            = euler_flux<3>;
     constexpr int NV   = 5;
@@ -1177,7 +1214,7 @@ template <int B>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_euler_step_2d64(
     const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
     const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    euler_params prm, euler_scalars* sc)
+    euler_params prm, euler_slot* sc)
 {
     static_assert(B >= 2 && 64 % B == 0 && 2 * B <= 64, "strips of at least two rows");
     using F           = euler_flux<2>;
@@ -1475,7 +1512,7 @@ __global__ __launch_bounds__(NT) void k_euler_step_strip(const double* __restric
                                                          size_t fstride, const uint64_t* __restrict__ keys,
                                                          const face_link* __restrict__ links,
                                                          const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk,
-    euler_params prm, euler_scalars* sc)
+    euler_params prm, euler_slot* sc)
 {
     using S          = patch_shape<R, N>;
     using T          = strip_shape<R, N, B>;
