@@ -981,19 +981,37 @@ struct amr_ctx
             throw amr_error(AMR_ERR_HIP, "the read-back of a finished stream did not arrive");
     }
 
+    // Queues the build of the table of the leaves k (at most `most` of them,
+    // see k_build_table); `leaves`: the current count, which says whether the
+    // searches are likely to run on keys in LDS.
+    void launch_table(const uint64_t* k, uint64_t leaves, uint32_t most, uint32_t guard_cap)
+    {
+        const unsigned grid = grid1d(most * static_cast<uint64_t>(ndir), 256);
+        auto           go   = [&](auto r, auto small) {
+            constexpr int  R     = decltype(r)::value;
+            constexpr bool SMALL = decltype(small)::value;
+            hipLaunchKernelGGL((k_build_table<R, SMALL>), dim3(grid), dim3(256), 0, stream, k, most, depth, links, metas,
+                               summary, guard_cap);
+        };
+        auto by_size = [&](auto r) {
+            if (leaves <= kLdsKeys)
+                go(r, std::true_type{});
+            else
+                go(r, std::false_type{});
+        };
+        if (rank == 2)
+            by_size(std::integral_constant<int, 2>{});
+        else
+            by_size(std::integral_constant<int, 3>{});
+        check_launch("k_build_table");
+    }
+
     // Neighbour records of the current leaves (a regrid builds its new table
     // itself, see regrid).
     void build_table()
     {
         AMR_HIP_CHECK(hipMemsetAsync(summary, 0, sizeof(regrid_summary), stream));
-        const uint64_t items = n * static_cast<uint64_t>(ndir);
-        if (rank == 2)
-            hipLaunchKernelGGL(k_build_table<2>, dim3(grid1d(items, 256)), dim3(256), 0, stream, keys[kc],
-                               static_cast<uint32_t>(n), depth, links, metas, summary, 0u);
-        else
-            hipLaunchKernelGGL(k_build_table<3>, dim3(grid1d(items, 256)), dim3(256), 0, stream, keys[kc],
-                               static_cast<uint32_t>(n), depth, links, metas, summary, 0u);
-        check_launch("k_build_table");
+        launch_table(keys[kc], n, static_cast<uint32_t>(n), 0u);
         publish_wait(summary, nullptr);
         if (box->summary.err & 1u)
         {
@@ -1243,14 +1261,7 @@ struct amr_ctx
                  fstride(), cap32, stream);
         // the new table: at most 2^R leaves per old leaf, and no more than the capacity
         const uint64_t most  = std::min<uint64_t>(static_cast<uint64_t>(nn) << rank, cap);
-        const uint64_t items = most * static_cast<uint64_t>(ndir);
-        if (rank == 2)
-            hipLaunchKernelGGL(k_build_table<2>, dim3(grid1d(items, 256)), dim3(256), 0, stream, keys[1 - kc],
-                               static_cast<uint32_t>(most), depth, links, metas, summary, cap32);
-        else
-            hipLaunchKernelGGL(k_build_table<3>, dim3(grid1d(items, 256)), dim3(256), 0, stream, keys[1 - kc],
-                               static_cast<uint32_t>(most), depth, links, metas, summary, cap32);
-        check_launch("k_build_table");
+        launch_table(keys[1 - kc], nn, static_cast<uint32_t>(most), cap32);
         publish_wait(summary, nullptr);
         const regrid_summary s = box->summary;
         if (s.err & 2u) throw amr_error(AMR_ERR_UNSUPPORTED, "coarsening to the root level is not supported");

@@ -40,15 +40,6 @@ __host__ __device__ inline uint32_t quad_of(uint32_t meta, int d) { return (meta
 // Morton keys: key = (interleave(x, y[, z]) << 6) | level, x in bit 0.
 // ---------------------------------------------------------------------------
 template <int R>
-__host__ __device__ inline uint64_t interleave(const uint32_t* c)
-{
-    uint64_t m = 0;
-    for (int b = 0; b < kMaxDepth; ++b)
-        for (int i = 0; i < R; ++i) m |= static_cast<uint64_t>((c[i] >> b) & 1u) << (R * b + i);
-    return m;
-}
-
-template <int R>
 __host__ __device__ inline void deinterleave(uint64_t m, uint32_t* c)
 {
     for (int i = 0; i < R; ++i) c[i] = 0;
@@ -66,12 +57,6 @@ struct leaf_run
 {
     uint32_t head, len;
 };
-
-template <int R>
-__host__ __device__ inline uint64_t make_key(const uint32_t* c, int level)
-{
-    return (interleave<R>(c) << 6) | static_cast<uint64_t>(level & 0x3F);
-}
 
 // ---------------------------------------------------------------------------
 // Compact patch layout: n^R interior doubles, row-major, last index fastest.

@@ -46,12 +46,40 @@ __device__ inline bool regrid_applies(const regrid_summary* summary, uint32_t ca
     return !(s.err & 2u) && s.total <= cap && (s.n_refine | s.n_coarsen) != 0;
 }
 
-// Index of the leaf containing integer point p (resolution 2^depth) among the
-// sorted keys, or -1 when no leaf contains it.
+// ---------------------------------------------------------------------------
+// Morton arithmetic: a leaf's neighbours, parent and children straight from
+// its interleaved coordinates.  (Taking them apart and together again bit by
+// bit, some hundred instructions each way, was most of what the planning
+// workgroup did.)
+// ---------------------------------------------------------------------------
+
+// The bits of axis a among R * depth.
 template <int R>
-__host__ __device__ inline int32_t locate(const uint64_t* __restrict__ keys, uint32_t n, const uint32_t* p, int depth)
+__host__ __device__ inline uint64_t axis_bits(int a, int depth)
 {
-    const uint64_t mp     = interleave<R>(p);
+    const uint64_t all = R == 2 ? 0x5555555555555555ull : 0x1249249249249249ull; // axis 0
+    return (all << a) & ((uint64_t{ 1 } << (R * depth)) - 1u);
+}
+
+// m with the coordinate of axis a advanced / taken back by 2^k, periodic.
+template <int R>
+__host__ __device__ inline uint64_t axis_add(uint64_t m, int a, int k, int depth)
+{
+    const uint64_t bits = axis_bits<R>(a, depth);
+    return (((m | ~bits) + (uint64_t{ 1 } << (R * k + a))) & bits) | (m & ~bits);
+}
+template <int R>
+__host__ __device__ inline uint64_t axis_sub(uint64_t m, int a, int k, int depth)
+{
+    const uint64_t bits = axis_bits<R>(a, depth);
+    return (((m & bits) - (uint64_t{ 1 } << (R * k + a))) & bits) | (m & ~bits);
+}
+
+// Index of the leaf containing the point with interleaved coordinates mp
+// (resolution 2^depth) among the sorted keys, or -1 when no leaf contains it.
+template <int R>
+__host__ __device__ inline int32_t locate(const uint64_t* __restrict__ keys, uint32_t n, uint64_t mp, int depth)
+{
     const uint64_t target = (mp << 6) | 63u;
     uint32_t       lo = 0, hi = n; // first index with key > target
     while (lo < hi)
@@ -76,22 +104,15 @@ template <int R>
 __host__ __device__ inline bool table_entry(const uint64_t* __restrict__ keys, uint32_t n, int depth, uint32_t leaf,
                                             int dir, face_link* out_link, uint32_t* out_meta)
 {
-    const uint64_t key = keys[leaf];
-    const int      lv  = key_level(key);
-    uint32_t       c[R];
-    deinterleave<R>(key >> 6, c);
-    const uint32_t mask = (1u << depth) - 1u;
-    const uint32_t s    = 1u << (depth - lv);
-    const int      dim  = dir >> 1;
-    const bool     pos  = (dir & 1) != 0;
-    const int      a    = R - 1 - dim; // physical axis of the normal
-    uint32_t       p[R];
-    for (int i = 0; i < R; ++i) p[i] = c[i];
-    p[a]           = pos ? ((c[a] + s) & mask) : ((c[a] - 1u) & mask);
-    face_link L    = { { -1, -1, -1, -1 } };
-    uint32_t  meta = REL_NONE;
-    bool      ok   = true;
-    const int32_t j = locate<R>(keys, n, p, depth);
+    const uint64_t key = keys[leaf], m = key >> 6;
+    const int      lv  = key_level(key), up = depth - lv; // 2^up: the leaf's extent
+    const int      dim = dir >> 1;
+    const bool     pos = (dir & 1) != 0;
+    const int      a   = R - 1 - dim; // physical axis of the normal
+    face_link      L    = { { -1, -1, -1, -1 } };
+    uint32_t       meta = REL_NONE;
+    bool           ok   = true;
+    const int32_t  j    = locate<R>(keys, n, pos ? axis_add<R>(m, a, up, depth) : axis_sub<R>(m, a, 0, depth), depth);
     if (j < 0)
         ok = false;
     else
@@ -108,26 +129,26 @@ __host__ __device__ inline bool table_entry(const uint64_t* __restrict__ keys, u
             meta     = REL_COARSER;
             for (int jd = 0; jd < R; ++jd)
             {
-                const uint32_t q = (jd == dim) ? (pos ? 0u : 1u) : ((c[R - 1 - jd] >> (depth - lv)) & 1u);
+                const uint32_t q =
+                    (jd == dim) ? (pos ? 0u : 1u) : static_cast<uint32_t>((m >> (R * up + R - 1 - jd)) & 1u);
                 meta |= q << (2 + jd);
             }
         }
         else if (lq == lv + 1)
         {
-            meta = REL_FINER;
+            meta               = REL_FINER;
+            const uint64_t far = pos ? axis_add<R>(m, a, up, depth) : axis_sub<R>(m, a, up - 1, depth);
             for (int q = 0; q < (1 << (R - 1)); ++q)
             {
-                uint32_t p2[R];
-                for (int i = 0; i < R; ++i) p2[i] = c[i];
-                p2[a]   = pos ? ((c[a] + s) & mask) : ((c[a] - s / 2) & mask);
-                int bit = 0;
+                uint64_t p   = far;
+                int      bit = 0;
                 for (int jd = 0; jd < R; ++jd)
                 {
                     if (jd == dim) continue;
-                    p2[R - 1 - jd] += ((q >> bit) & 1) * (s / 2);
+                    p |= static_cast<uint64_t>((q >> bit) & 1) << (R * (up - 1) + R - 1 - jd);
                     ++bit;
                 }
-                const int32_t jj = locate<R>(keys, n, p2, depth);
+                const int32_t jj = locate<R>(keys, n, p, depth);
                 if (jj < 0 || key_level(keys[jj]) != lv + 1) ok = false;
                 L.ids[q] = jj;
             }
@@ -154,11 +175,17 @@ __host__ __device__ inline void close_item(const uint64_t* __restrict__ keys, in
                                            uint8_t* mark, uint32_t i)
 {
     if (!mark[i] || key_level(keys[i]) != level) return;
+    // every record first: one round trip, not one per face
+    uint32_t m[2 * R];
+    int32_t  id[2 * R];
     for (int k = 0; k < 2 * R; ++k)
     {
         const size_t e = static_cast<size_t>(i) * 2 * R + k;
-        if (rel_of(metas[e]) == REL_COARSER) mark[links[e].ids[0]] = 1;
+        m[k]           = metas[e];
+        id[k]          = links[e].ids[0];
     }
+    for (int k = 0; k < 2 * R; ++k)
+        if (rel_of(m[k]) == REL_COARSER) mark[id[k]] = 1;
 }
 
 // Morton offset of a key within its parent (morton_id.hpp:55-62).
@@ -166,12 +193,7 @@ template <int R>
 __host__ __device__ inline int offset_in_parent(uint64_t key, int depth)
 {
     const int lv = key_level(key);
-    if (lv == 0) return 0;
-    uint32_t c[R];
-    deinterleave<R>(key >> 6, c);
-    int o = 0;
-    for (int a = 0; a < R; ++a) o |= static_cast<int>((c[a] >> (depth - lv)) & 1u) << a;
-    return o;
+    return lv == 0 ? 0 : static_cast<int>((key >> 6) >> (R * (depth - lv))) & ((1 << R) - 1);
 }
 
 // Coarsening family test for leaf i (ndtree.hpp:904-940 eligibility,
@@ -190,14 +212,10 @@ __host__ __device__ inline bool coarsen_family_head(const int8_t* __restrict__ f
     const int      lv  = key_level(key);
     *root_family       = false;
     if (lv == 0 || offset_in_parent<R>(key, depth) != 0 || i + F > n) return false;
-    uint32_t c[R];
-    deinterleave<R>(key >> 6, c);
-    const uint32_t s = 1u << (depth - lv);
     for (int o = 0; o < F; ++o)
     {
-        uint32_t cc[R];
-        for (int a = 0; a < R; ++a) cc[a] = c[a] + ((o >> a) & 1) * s;
-        if (keys[i + o] != make_key<R>(cc, lv)) return false; // a child is not a leaf
+        // the first child's key, o extents further
+        if (keys[i + o] != key + (static_cast<uint64_t>(o) << (R * (depth - lv) + 6))) return false; // a child is not a leaf
         if (flags[i + o] != 2) return false;
     }
     if (lv == 1)
@@ -205,21 +223,31 @@ __host__ __device__ inline bool coarsen_family_head(const int8_t* __restrict__ f
         *root_family = true; // the reference aborts when the root's children recombine
         return false;
     }
-    for (int o = 0; o < F; ++o)
+    // the outer faces of the family's leaves: every record first, as above
+    constexpr int K = 1 << (R - 1); // leaves on a face of the family
+    uint32_t      m[2 * R][K];
+    int32_t       id[2 * R][K];
+    bool          kept = true;
+    for (int o = 0; o < F; ++o) kept = kept && !mark[i + o];
+    if (!kept) return false;
+    for (int k = 0; k < 2 * R; ++k)
     {
-        if (mark[i + o]) return false;
-        for (int k = 0; k < 2 * R; ++k)
+        const int dim = k >> 1, at = R - 1 - dim; // o's bit of layout dim
+        for (int q = 0; q < K; ++q)
         {
-            const int  dim = k >> 1;
-            const bool pos = (k & 1) != 0;
-            const int  bit = (o >> (R - 1 - dim)) & 1; // child position on layout dim
-            if (bit != (pos ? 1 : 0)) continue;       // not on that face of the parent
-            const size_t   e   = static_cast<size_t>(i + o) * 2 * R + k;
-            const uint32_t rel = rel_of(metas[e]);
-            if (rel == REL_FINER) return false;
-            if (rel == REL_SAME && mark[links[e].ids[0]]) return false;
+            // the q-th child on side k & 1
+            const int    o = ((q >> at) << (at + 1)) | ((k & 1) << at) | (q & ((1 << at) - 1));
+            const size_t e = static_cast<size_t>(i + o) * 2 * R + k;
+            m[k][q]        = metas[e];
+            id[k][q]       = links[e].ids[0];
         }
     }
+    for (int k = 0; k < 2 * R; ++k)
+        for (int q = 0; q < K; ++q)
+        {
+            const uint32_t rel = rel_of(m[k][q]);
+            if (rel == REL_FINER || (rel == REL_SAME && mark[id[k][q]])) return false;
+        }
     return true;
 }
 
@@ -241,20 +269,8 @@ template <int R>
 __host__ __device__ inline uint64_t emit_key(uint64_t key, int depth, bool refine, bool family_head, int j)
 {
     const int lv = key_level(key);
-    uint32_t  c[R];
-    deinterleave<R>(key >> 6, c);
-    if (refine)
-    {
-        const uint32_t s = 1u << (depth - lv - 1);
-        for (int a = 0; a < R; ++a) c[a] += ((j >> a) & 1) * s;
-        return make_key<R>(c, lv + 1);
-    }
-    if (family_head)
-    {
-        const uint32_t s = 1u << (depth - lv);
-        for (int a = 0; a < R; ++a) c[a] &= ~s;
-        return make_key<R>(c, lv - 1);
-    }
+    if (refine) return key + (static_cast<uint64_t>(j) << (R * (depth - lv - 1) + 6)) + 1u; // one level deeper
+    if (family_head) return (key & ~(static_cast<uint64_t>((1 << R) - 1) << (R * (depth - lv) + 6))) - 1u;
     return key;
 }
 
@@ -311,8 +327,18 @@ __host__ __device__ inline double restrict_value(const double* __restrict__ u, u
 // Kernels
 // ---------------------------------------------------------------------------
 
-template <int R>
-__global__ void k_build_table(const uint64_t* __restrict__ keys, uint32_t n, int depth, face_link* __restrict__ links,
+// Trees of up to this many leaves: the table's binary searches and the
+// regrid's planning passes run on copies of the keys in LDS (32 KB).  Both are
+// chains of dependent reads, about ten per search, that cost an L2 round trip
+// each.  us a launch within adaptive solves on about 300 leaves of 16^2 / 700
+// of 64^2, before -> after (Morton arithmetic, records read together, the
+// deepest level formed by the plan instead of an atomic per emitted leaf):
+// table 4.9 -> 3.5 / 3.2 -> 2.8, planning 7.0 -> 6.6 / 7.1 -> 7.7 (bound by
+// one workgroup's barriers and integer work, LDS or not), emit 4.4 -> 3.3.
+constexpr uint32_t kLdsKeys = 4096;
+
+template <int R, bool SMALL>
+__global__ __launch_bounds__(256) void k_build_table(const uint64_t* __restrict__ keys, uint32_t n, int depth, face_link* __restrict__ links,
                               uint32_t* __restrict__ metas, regrid_summary* __restrict__ summary, uint32_t guard_cap)
 {
     // after a regrid planned on the device (guard_cap = the capacity): the
@@ -323,12 +349,31 @@ __global__ void k_build_table(const uint64_t* __restrict__ keys, uint32_t n, int
         if (!regrid_applies(summary, guard_cap)) return;
         n = summary->total;
     }
-    const uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n * 2 * R) return;
-    face_link L;
-    uint32_t  meta;
-    if (!table_entry<R>(keys, n, depth, idx / (2 * R), static_cast<int>(idx % (2 * R)), &L, &meta))
-        atomicOr(&summary->err, 1u);
+    const uint32_t idx  = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t leaf = idx / (2 * R);
+    const int      dir  = static_cast<int>(idx % (2 * R));
+    face_link      L;
+    uint32_t       meta;
+    bool           ok;
+    if constexpr (SMALL)
+    {
+        __shared__ uint64_t sk[kLdsKeys];
+        if (blockIdx.x * blockDim.x >= n * 2 * R) return; // the whole workgroup
+        if (n <= kLdsKeys)
+        {
+            for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) sk[k] = keys[k];
+            __syncthreads();
+        }
+        if (idx >= n * 2 * R) return;
+        ok = n <= kLdsKeys ? table_entry<R>(sk, n, depth, leaf, dir, &L, &meta)
+                           : table_entry<R>(keys, n, depth, leaf, dir, &L, &meta);
+    }
+    else
+    {
+        if (idx >= n * 2 * R) return;
+        ok = table_entry<R>(keys, n, depth, leaf, dir, &L, &meta);
+    }
+    if (!ok) atomicOr(&summary->err, 1u);
     links[idx] = L;
     metas[idx] = meta;
 }
@@ -465,7 +510,7 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* total)
 // barriers take the place of the launches between the passes, so a small
 // tree's regrid costs one launch instead of about a dozen.
 constexpr int kPlanThreads   = 1024;
-constexpr int kPlanMaxLeaves = 4 * kPlanThreads;
+constexpr int kPlanMaxLeaves = kLdsKeys;
 
 template <int R>
 __global__ __launch_bounds__(kPlanThreads) void k_regrid_plan(
@@ -473,22 +518,33 @@ __global__ __launch_bounds__(kPlanThreads) void k_regrid_plan(
     const face_link* __restrict__ links, const uint32_t* __restrict__ metas, uint8_t* mark, uint8_t* head,
     uint32_t* __restrict__ counts, uint32_t* __restrict__ pos, regrid_summary* __restrict__ summary)
 {
+    __shared__ uint64_t sk[kPlanMaxLeaves];                         // keys
+    __shared__ uint8_t  sm[kPlanMaxLeaves], sh[kPlanMaxLeaves]; // marks, family heads
+    __shared__ int8_t   sf[kPlanMaxLeaves];                     // flags
+    __shared__ uint32_t sums[4];                                // refined, coarsened, errors, deepest level
     const uint32_t t = threadIdx.x;
-    if (t == 0) *summary = regrid_summary{}; // the counts below and the emit's deepest level start from 0
-    for (uint32_t i = t; i < n; i += kPlanThreads) mark[i] = refine_mark(flags[i], keys[i], depth);
+    if (t < 4) sums[t] = 0;
+    for (uint32_t i = t; i < n; i += kPlanThreads)
+    {
+        sk[i] = keys[i];
+        sf[i] = flags[i];
+        sm[i] = refine_mark(sf[i], sk[i], depth);
+    }
     __syncthreads();
     for (int l = top_level; l >= 1; --l)
     {
-        for (uint32_t i = t; i < n; i += kPlanThreads) close_item<R>(keys, l, links, metas, mark, i);
+        for (uint32_t i = t; i < n; i += kPlanThreads) close_item<R>(sk, l, links, metas, sm, i);
         __syncthreads();
     }
-    uint32_t n_coarsen = 0, n_refine = 0;
+    uint32_t n_coarsen = 0, n_refine = 0, deepest = 0;
     bool     root_any  = false;
     for (uint32_t i = t; i < n; i += kPlanThreads)
     {
         bool       root = false;
-        const bool h    = coarsen_family_head<R>(flags, keys, n, depth, links, metas, mark, i, &root);
-        head[i]         = h ? 1 : 0;
+        const bool h    = coarsen_family_head<R>(sf, sk, n, depth, links, metas, sm, i, &root);
+        sh[i]           = h ? 1 : 0;
+        head[i]         = sh[i];
+        mark[i]         = sm[i];
         n_coarsen += h ? 1u : 0u;
         root_any = root_any || root;
     }
@@ -500,22 +556,27 @@ __global__ __launch_bounds__(kPlanThreads) void k_regrid_plan(
     uint32_t       sum = 0;
     for (uint32_t i = lo; i < hi; ++i)
     {
-        const uint32_t c = emit_count<R>(keys, depth, mark, head, i);
+        const uint32_t c = emit_count<R>(sk, depth, sm, sh, i);
         counts[i]        = c;
         sum += c;
-        n_refine += mark[i] ? 1u : 0u;
+        n_refine += sm[i] ? 1u : 0u;
+        // the level of its output, if any
+        const uint32_t lv = static_cast<uint32_t>(key_level(sk[i])) + (sm[i] ? 1u : 0u) - (sh[i] ? 1u : 0u);
+        deepest           = c != 0 && lv > deepest ? lv : deepest;
     }
     uint32_t total;
     uint32_t off = block_exclusive_scan<kPlanThreads>(sum, &total);
     for (uint32_t i = lo; i < hi; ++i)
     {
         pos[i] = off;
-        off += counts[i];
+        off += emit_count<R>(sk, depth, sm, sh, i);
     }
-    if (n_coarsen) atomicAdd(&summary->n_coarsen, n_coarsen);
-    if (n_refine) atomicAdd(&summary->n_refine, n_refine);
-    if (root_any) atomicOr(&summary->err, 2u);
-    if (t == 0) summary->total = total;
+    if (n_refine) atomicAdd(&sums[0], n_refine);
+    if (n_coarsen) atomicAdd(&sums[1], n_coarsen);
+    if (root_any) atomicOr(&sums[2], 2u);
+    if (deepest) atomicMax(&sums[3], deepest);
+    __syncthreads();
+    if (t == 0) *summary = regrid_summary{ total, sums[0], sums[1], sums[2], sums[3], {} };
 }
 
 __global__ void k_scan_blocks(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t n,

@@ -236,3 +236,25 @@ def test_euler_walk_16(amr, n):
         exp = euler_step_of_padded(t, 1.4, s.compute_dt())
     s.advance()
     assert_fields(t.get_interior(), exp, f"{t.size()} leaves")
+
+
+@pytest.mark.parametrize("rank,level", [(2, 5), (2, 6), (3, 3), (3, 4)])
+def test_regrid_on_both_sides_of_the_lds_limit(amr, rank, level):
+    """Regrids that start and end below, at and above 4096 leaves (keys in LDS
+    or in memory), against the oracle: keys and neighbour tables."""
+    from oracle import OracleTree
+
+    say(f"case: regrids of a {rank}D tree at level {level}")
+    n = 4
+    g = amr.NdTree(rank, level + 2, n, 1, 80000)
+    o = OracleTree(rank, n, 1, level + 2, 80000)
+    for _ in range(level):
+        g.refine_all()
+        o.refine_all()
+    assert g.size() == 1 << (rank * level)
+    rng = np.random.default_rng(rank * 10 + level)
+    for share in (0.3, 0.05, 0.0):
+        flags = np.where(rng.random(g.size()) < share, amr.REFINE, amr.COARSEN).astype(np.int8)
+        assert bool(g.reconstruct_tree(flags)) == bool(o.reconstruct(flags))
+        assert np.array_equal(g.keys(), o.keys()), share
+        assert g.neighbor_metadata().tobytes() == o.metadata().tobytes(), share
