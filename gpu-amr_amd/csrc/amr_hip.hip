@@ -109,6 +109,9 @@ struct ops
                  hipStream_t);
     void (*adj_step)(ops const&, const double*, const double*, const uint64_t*, const face_link*, const uint32_t*,
                      const adjoint_params*, double*, double*, uint32_t, hipStream_t);
+    // an adjoint and a forward step in one launch (null: not built for the shape)
+    void (*adj_pair)(const double*, const double*, const uint64_t*, const face_link*, const uint32_t*,
+                     const adjoint_params*, double*, double*, uint32_t, forward_args const&, hipStream_t);
     void (*adj_regrid)(ops const&, const double*, const uint8_t*, const uint8_t*, const uint32_t*, const uint32_t*,
                        double*, uint32_t, hipStream_t);
     // two fused steps of a single-level tree (null: not built for the shape)
@@ -331,14 +334,23 @@ struct instance
         if (n == 0) return;
         if constexpr (R == 3 && N == 8)
             hipLaunchKernelGGL(k_adj_step_3d8, dim3(xcd_grid(n)), dim3(64), 0, s, lam_next, u, keys, links, metas, prm,
-                               lam, vpart, n, walk_of(n, 0));
+                               lam, n, walk_of(n, 0), vpart);
         else if constexpr (R == 2 && N == 16)
-            hipLaunchKernelGGL(k_adj_step_2d16, dim3(xcd_grid(n)), dim3(64), 0, s, lam_next, u, keys, links, metas,
-                               prm, lam, vpart, n, walk_of(n, 0));
+            adj_pair(lam_next, u, keys, links, metas, prm, lam, vpart, n, forward_args{}, s);
         else
             hipLaunchKernelGGL((k_adj_step<R, N, NT>), dim3(n), dim3(NT), 0, s, lam_next, u, keys, links, metas, prm,
                                lam, vpart, n);
         check_launch("k_adj_step");
+    }
+    // 2D 16^2: one adjoint step and, where F has leaves, a forward step in one launch.
+    static void adj_pair(const double* lam_next, const double* u, const uint64_t* keys, const face_link* links,
+                         const uint32_t* metas, const adjoint_params* prm, double* lam, double* vpart, uint32_t n,
+                         forward_args const& F, hipStream_t s)
+    {
+        const uint32_t blocks = xcd_grid(n);
+        hipLaunchKernelGGL(k_adj_step_2d16, dim3(blocks + xcd_grid(F.nleaves)), dim3(64), 0, s, lam_next, u, keys,
+                           links, metas, prm, lam, n, walk_of(n, 0), blocks, vpart, F);
+        check_launch("k_adj_step_2d16");
     }
     static void adj_regrid(ops const&, const double* lam_new, const uint8_t* mark, const uint8_t* head, const uint32_t* counts,
                            const uint32_t* pos, double* lam_old, uint32_t n_old, hipStream_t s)
@@ -424,6 +436,7 @@ struct instance
                     &criterion,
                     &emit,
                     &adj_step,
+                    R == 2 && N == 16 ? &adj_pair : nullptr,
                     &adj_regrid,
                     fused ? &step2 : nullptr,
                     &euler_dt,
@@ -590,7 +603,7 @@ struct box_instance
     {
         return ops{ R,       0,          h,     { ext[0], ext[1], R == 3 ? ext[2] : 1 },
                     &step,   &variant_count, &variant_name, &variant_needs,
-                    &padded, &criterion, &emit, &adj_step,
+                    &padded, &criterion, &emit, &adj_step, nullptr,
                     &adj_regrid, nullptr, &euler_dt, &euler_step };
     }
 };
@@ -1535,7 +1548,9 @@ struct amr_tape
     std::vector<uint32_t>      h_leaves;
     uint64_t*                  scratch_keys    = nullptr;
     regrid_summary*            scratch_summary = nullptr;
-    std::vector<double*>       seg; // recomputed states of one segment
+    // Recomputed states of one segment and, where adjoint and forward steps
+    // share launches (adj_pair) and there is memory, of the one before it.
+    std::vector<double*>       seg[2];
     // The launch sequence of a recorded tape is fixed (steps, regrids,
     // buffers), so the forward replay and the adjoint pass are each captured
     // once into a hipGraph and replayed; the kernels read the velocity-
@@ -1558,7 +1573,7 @@ struct amr_tape
         for (auto& t : topos) ptrs.insert(ptrs.end(), { t.keys, t.links, t.metas });
         for (auto& r : regrids) ptrs.insert(ptrs.end(), { r.mark, r.head, r.counts, r.pos });
         for (double* c : ckpts) ptrs.push_back(c);
-        for (double* s : seg) ptrs.push_back(s);
+        for (auto& set : seg) ptrs.insert(ptrs.end(), set.begin(), set.end());
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
@@ -1686,7 +1701,20 @@ struct amr_tape
         for (uint64_t k = 0; k < steps; ++k) h_leaves[k] = static_cast<uint32_t>(topo(k).n);
         AMR_HIP_CHECK(hipMemcpyAsync(step_leaves, h_leaves.data(), steps * sizeof(uint32_t), hipMemcpyHostToDevice,
                                      stream));
-        for (uint64_t j = 1; j < ckpt_every; ++j) seg.push_back(dev_alloc<double>(max_n * ni));
+        for (uint64_t j = 1; j < ckpt_every; ++j) seg[0].push_back(dev_alloc<double>(max_n * ni));
+        if (op->adj_pair && variant == 0 && ckpt_every > 1 && steps > ckpt_every)
+        {
+            try
+            {
+                for (uint64_t j = 1; j < ckpt_every; ++j) seg[1].push_back(dev_alloc<double>(max_n * ni));
+            }
+            catch (amr_error const&) // no memory for a second segment: one after the other
+            {
+                for (double* b : seg[1]) (void)hipFree(b);
+                seg[1].clear();
+                (void)hipGetLastError();
+            }
+        }
         upload_constants();
     }
 
@@ -1779,35 +1807,93 @@ struct amr_tape
         for (int d = 0; d < 3; ++d) grad_v[d] = d < rank ? h[d] : 0.0;
     }
 
+    // The recomputation of the states entering the steps of segment s from
+    // its checkpoint, one launch at a time: the steps (but the segment's
+    // last) and the regrid transfers between them.
+    struct recomputation
+    {
+        std::vector<double*> const* set = nullptr; // where the states go
+        std::vector<const double*>  states;        // entering each step of the segment
+        uint64_t                    first = 0, next = 0, last = 0;
+        bool                        transfer = false; // step next - 1's result is in `work`, to be transferred
+
+        bool done() const { return next == last && !transfer; }
+    };
+
+    recomputation begin_segment(uint64_t s, std::vector<double*> const& set) const
+    {
+        const uint64_t c = s * ckpt_every, e = std::min(steps, c + ckpt_every);
+        recomputation  r;
+        r.set    = &set;
+        r.states = { ckpts[s] };
+        r.first = r.next = c;
+        r.last           = e - 1;
+        return r;
+    }
+
+    // Queues the pending transfer, if any.
+    void finish_transfer(recomputation& r)
+    {
+        if (!r.transfer) return;
+        replay_transfer(*regrid_before(r.next), work, const_cast<double*>(r.states.back()));
+        r.transfer = false;
+    }
+
+    // The next step: where from and to; the caller launches it.
+    forward_args next_step(recomputation& r)
+    {
+        const uint64_t  k = r.next++;
+        topology const& t = topo(k);
+        double*         to = (*r.set)[k - r.first];
+        const double*   from = r.states.back();
+        r.states.push_back(to);
+        r.transfer = regrid_before(k + 1) != nullptr;
+        return { from,    r.transfer ? work : to,         t.keys,
+                 t.links, t.metas,                        step_tab + k,
+                 static_cast<uint32_t>(t.n), walk_of(t.n, static_cast<uint32_t>(k & 1)) };
+    }
+
+    void finish_segment(recomputation& r)
+    {
+        while (!r.done())
+        {
+            finish_transfer(r);
+            if (r.next == r.last) break;
+            const uint64_t     k = r.next;
+            const forward_args f = next_step(r);
+            forward_step(k, f.u, f.un);
+        }
+    }
+
     // The backward sweep from lambda_T in lam[0]: grad_u0 in the returned
-    // buffer, grad_v in acc.
+    // buffer, grad_v in acc.  A segment's recomputation needs only its
+    // checkpoint: with two sets of buffers its steps ride along with the
+    // adjoint steps of the segment after it, one launch for both.
     double* adjoint_sweep()
     {
-        double*                    l  = lam[0];
-        double*                    lo = lam[1];
-        std::vector<const double*> states(ckpt_every);
-        const uint64_t             nseg = (steps + ckpt_every - 1) / ckpt_every;
+        double*        l  = lam[0];
+        double*        lo = lam[1];
+        const bool     pair = !seg[1].empty();
+        const uint64_t nseg = (steps + ckpt_every - 1) / ckpt_every;
+        recomputation  now, ahead;
         for (uint64_t s = nseg; s-- > 0;)
         {
             const uint64_t c = s * ckpt_every, e = std::min(steps, c + ckpt_every);
-            states[0]        = ckpts[s];
-            for (uint64_t k = c; k + 1 < e; ++k)
-            {
-                double* next = seg[k - c];
-                if (auto const* r = regrid_before(k + 1))
-                {
-                    forward_step(k, states[k - c], work);
-                    replay_transfer(*r, work, next);
-                }
-                else
-                    forward_step(k, states[k - c], next);
-                states[k + 1 - c] = next;
-            }
+            now              = pair && s + 1 < nseg ? std::move(ahead) : begin_segment(s, seg[pair ? s & 1 : 0]);
+            finish_segment(now);
+            const bool along = pair && s > 0;
+            if (along) ahead = begin_segment(s - 1, seg[(s - 1) & 1]);
             for (uint64_t k = e; k-- > c;)
             {
                 topology const& t = topo(k);
-                op->adj_step(*op, l, states[k - c], t.keys, t.links, t.metas, adj_tab + k, lo,
-                             vpart + (k - c) * max_n * 3, static_cast<uint32_t>(t.n), stream);
+                const double*   u = now.states[k - c];
+                double*         v = vpart + (k - c) * max_n * 3;
+                const uint32_t  n = static_cast<uint32_t>(t.n);
+                if (along) finish_transfer(ahead);
+                if (along && !ahead.done())
+                    op->adj_pair(l, u, t.keys, t.links, t.metas, adj_tab + k, lo, v, n, next_step(ahead), stream);
+                else
+                    op->adj_step(*op, l, u, t.keys, t.links, t.metas, adj_tab + k, lo, v, n, stream);
                 std::swap(l, lo);
                 if (auto const* r = regrid_before(k))
                 {

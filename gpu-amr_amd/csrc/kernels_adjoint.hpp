@@ -554,19 +554,14 @@ struct adj_consts
 };
 
 // 3D 8^3: lane l owns the z-column at (y, x) = (l / 8, l % 8).
-__global__ __launch_bounds__(64) void k_adj_step_3d8(const double* __restrict__ lam_next, const double* __restrict__ u,
-                                                     const uint64_t* __restrict__ keys,
-                                                     const face_link* __restrict__ links,
-                                                     const uint32_t* __restrict__ metas,
-                                                     const adjoint_params* __restrict__ prm_p,
-                                                     double* __restrict__ lam, double* __restrict__ vpart,
-                                                     uint32_t nleaves, uint32_t walk)
+__device__ inline void adj_leaf_3d8(const double* __restrict__ lam_next, const double* __restrict__ u,
+                                    const uint64_t* __restrict__ keys, const face_link* __restrict__ links,
+                                    const uint32_t* __restrict__ metas, const adjoint_params* __restrict__ prm_p,
+                                    double* __restrict__ lam, double* __restrict__ vpart, uint32_t leaf)
 {
     constexpr int     NI = 512;
     __shared__ double gface[4][64]; // ghosts of u: -y, +y (index z*8+x), -x, +x (index z*8+y)
     __shared__ double hface[4][64]; // halo terms of lambda on the same faces
-    const uint32_t    leaf = sweep_item(blockIdx.x, walk);
-    if (leaf >= nleaves) return;
     const int lane = threadIdx.x, hi3 = lane >> 3, lo3 = lane & 7;
     const int lv   = key_level(keys[leaf]);
     uint32_t  m[6];
@@ -680,19 +675,14 @@ __global__ __launch_bounds__(64) void k_adj_step_3d8(const double* __restrict__ 
 
 // 2D 16^2: lane (q, x) owns x of rows 4q .. 4q + 3 and gathers cell x of
 // face q.
-__global__ __launch_bounds__(64) void k_adj_step_2d16(const double* __restrict__ lam_next,
-                                                      const double* __restrict__ u, const uint64_t* __restrict__ keys,
-                                                      const face_link* __restrict__ links,
-                                                      const uint32_t* __restrict__ metas,
-                                                      const adjoint_params* __restrict__ prm_p,
-                                                      double* __restrict__ lam, double* __restrict__ vpart,
-                                                      uint32_t nleaves, uint32_t walk)
+__device__ inline void adj_leaf_2d16(const double* __restrict__ lam_next, const double* __restrict__ u,
+                                    const uint64_t* __restrict__ keys, const face_link* __restrict__ links,
+                                    const uint32_t* __restrict__ metas, const adjoint_params* __restrict__ prm_p,
+                                    double* __restrict__ lam, double* __restrict__ vpart, uint32_t leaf)
 {
     constexpr int     NI = 256;
     __shared__ double gface[4][16]; // ghosts of u: -y, +y (index x), -x, +x (index y)
     __shared__ double hface[4][16]; // halo terms of lambda
-    const uint32_t    leaf = sweep_item(blockIdx.x, walk);
-    if (leaf >= nleaves) return;
     const int lane = threadIdx.x, x = lane & 15, q = lane >> 4;
     const int lv   = key_level(keys[leaf]);
     uint32_t  m[4];
@@ -791,6 +781,58 @@ __global__ __launch_bounds__(64) void k_adj_step_2d16(const double* __restrict__
         if (lane == 0) vpart[static_cast<size_t>(leaf) * 3 + d] = sum;
     }
     if (lane == 0) vpart[static_cast<size_t>(leaf) * 3 + 2] = 0.0;
+}
+
+__global__ __launch_bounds__(64) void k_adj_step_3d8(const double* __restrict__ lam_next, const double* __restrict__ u,
+                                                     const uint64_t* __restrict__ keys,
+                                                     const face_link* __restrict__ links,
+                                                     const uint32_t* __restrict__ metas,
+                                                     const adjoint_params* __restrict__ prm_p,
+                                                     double* __restrict__ lam, uint32_t nleaves, uint32_t walk,
+                                                     double* __restrict__ vpart)
+{
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
+    if (leaf < nleaves) adj_leaf_3d8(lam_next, u, keys, links, metas, prm_p, lam, vpart, leaf);
+}
+
+// A forward step that shares an adjoint step's launch.
+struct forward_args
+{
+    const double*      u;
+    double*            un;
+    const uint64_t*    keys;
+    const face_link*   links;
+    const uint32_t*    metas;
+    const step_params* table;
+    uint32_t           nleaves, walk;
+};
+
+// One adjoint step by the first adj_blocks workgroups and, by the others, one
+// forward step of another topology: the recomputation of the segment before,
+// independent of it.  Alone either leaves most of the GPU idle on the trees of
+// a few hundred leaves that a 2D gradient steps on; together they take one
+// launch (300 steps with 285 recomputed, levels 3 to 6: 3150 -> 2570 us a
+// forward and backward pass; on two branches of the captured graph instead:
+// 3110).  For 8^3 patches the pair takes 162 registers and the GPU is busier:
+// 4096 leaves 526 -> 597 us, 512 leaves unchanged, so 3D keeps to itself.
+__global__ __launch_bounds__(64) void k_adj_step_2d16(const double* __restrict__ lam_next,
+                                                      const double* __restrict__ u, const uint64_t* __restrict__ keys,
+                                                      const face_link* __restrict__ links,
+                                                      const uint32_t* __restrict__ metas,
+                                                      const adjoint_params* __restrict__ prm_p,
+                                                      double* __restrict__ lam, uint32_t nleaves, uint32_t walk,
+                                                      uint32_t adj_blocks, double* __restrict__ vpart, forward_args F)
+{
+    // both grids are multiples of kXcds, so a workgroup keeps its XCD
+    if (blockIdx.x < adj_blocks)
+    {
+        const uint32_t leaf = sweep_item(blockIdx.x, walk);
+        if (leaf < nleaves) adj_leaf_2d16(lam_next, u, keys, links, metas, prm_p, lam, vpart, leaf);
+        return;
+    }
+    const uint32_t leaf = sweep_item(blockIdx.x - adj_blocks, F.walk);
+    if (leaf >= F.nleaves) return;
+    step_leaf_2d16<false, FROM_TABLE>(F.u, F.un, F.keys, F.links, F.metas, leaf, step_params{}, F.table, nullptr);
 }
 
 // Transposed regrid transfer of old leaf i (one workgroup; mark / head /

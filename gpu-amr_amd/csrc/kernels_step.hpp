@@ -980,16 +980,13 @@ __global__ __launch_bounds__(NT) void k_step(const double* __restrict__ u, doubl
 // lane that needs them, the -+y / -+x faces go through 2 KiB of LDS.  With
 // no interior tile in LDS, 32 leaves are in flight per CU.
 template <bool NT, int FROM>
-__global__ __launch_bounds__(64) void k_step_3d8(const double* __restrict__ u, double* __restrict__ un,
-                                                 const uint64_t* __restrict__ keys,
-                                                 const face_link* __restrict__ links,
-                                                 const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
-    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
+__device__ inline void step_leaf_3d8(const double* __restrict__ u, double* __restrict__ un,
+                                     const uint64_t* __restrict__ keys, const face_link* __restrict__ links,
+                                     const uint32_t* __restrict__ metas, uint32_t leaf, step_params const& prm,
+                                     const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
     constexpr int NI = 512;
     __shared__ double gface[4][64]; // -y, +y (index z*8+x), -x, +x (index z*8+y)
-    const uint32_t leaf = sweep_item(blockIdx.x, walk);
-    if (leaf >= nleaves) return;
     const int      lane = threadIdx.x, hi3 = lane >> 3, lo3 = lane & 7;
     const uint32_t who  = leaf_instance<FROM>(inst, leaf);
     const int      lv   = key_level(keys[leaf]);
@@ -1030,6 +1027,18 @@ __global__ __launch_bounds__(64) void k_step_3d8(const double* __restrict__ u, d
         store_cell<NT>(out + z * 64 + lane, update_from_fluxes<3>(uc, fL, fR, C.dtdx));
         fz = fzr;
     }
+}
+
+template <bool NT, int FROM>
+__global__ __launch_bounds__(64) void k_step_3d8(const double* __restrict__ u, double* __restrict__ un,
+                                                 const uint64_t* __restrict__ keys,
+                                                 const face_link* __restrict__ links,
+                                                 const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
+{
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
+    if (leaf >= nleaves) return;
+    step_leaf_3d8<NT, FROM>(u, un, keys, links, metas, leaf, prm, table, inst);
 }
 
 // 3D 8^3 patches, one wave per run of same-level leaves along +x (leaf_run).
@@ -1133,16 +1142,13 @@ __global__ __launch_bounds__(64) void k_step_3d8_run(const double* __restrict__ 
 // above / below a lane's four from lanes l -+ 16; the four ghost faces are
 // gathered one face cell per lane into 512 B of LDS.
 template <bool NT, int FROM>
-__global__ __launch_bounds__(64) void k_step_2d16(const double* __restrict__ u, double* __restrict__ un,
-                                                  const uint64_t* __restrict__ keys,
-                                                  const face_link* __restrict__ links,
-                                                  const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
-    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
+__device__ inline void step_leaf_2d16(const double* __restrict__ u, double* __restrict__ un,
+                                      const uint64_t* __restrict__ keys, const face_link* __restrict__ links,
+                                      const uint32_t* __restrict__ metas, uint32_t leaf, step_params const& prm,
+                                      const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
     constexpr int NI = 256;
     __shared__ double gface[4][16]; // -y, +y (index x), -x, +x (index y)
-    const uint32_t leaf = sweep_item(blockIdx.x, walk);
-    if (leaf >= nleaves) return;
     const int      lane = threadIdx.x, x = lane & 15, q = lane >> 4;
     const uint32_t who  = leaf_instance<FROM>(inst, leaf);
     const int      lv   = key_level(keys[leaf]);
@@ -1178,6 +1184,18 @@ __global__ __launch_bounds__(64) void k_step_2d16(const double* __restrict__ u, 
         store_cell<NT>(out + y * 16 + x, update_from_fluxes<2>(uc, fL, fR, C.dtdx));
         fy = fyr;
     }
+}
+
+template <bool NT, int FROM>
+__global__ __launch_bounds__(64) void k_step_2d16(const double* __restrict__ u, double* __restrict__ un,
+                                                  const uint64_t* __restrict__ keys,
+                                                  const face_link* __restrict__ links,
+                                                  const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, step_params prm,
+    const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
+{
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
+    if (leaf >= nleaves) return;
+    step_leaf_2d16<NT, FROM>(u, un, keys, links, metas, leaf, prm, table, inst);
 }
 
 // 2D 16^2 patches, one wave per run of same-level leaves along +x, the lane

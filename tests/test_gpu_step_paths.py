@@ -258,3 +258,37 @@ def test_regrid_on_both_sides_of_the_lds_limit(amr, rank, level):
         assert bool(g.reconstruct_tree(flags)) == bool(o.reconstruct(flags))
         assert np.array_equal(g.keys(), o.keys()), share
         assert g.neighbor_metadata().tobytes() == o.metadata().tobytes(), share
+
+
+def test_adjoint_segments_ride_along(amr):
+    """2D 16^2 gradients whose recomputed segments share the adjoint steps'
+    launches: the same bits for every checkpoint interval (1: nothing to
+    recompute; 7: a short last segment; 23: one segment, nothing to share),
+    with regrids inside and between segments, first pass and replay."""
+    import torch
+
+    say("case: 2D adjoint, checkpoint intervals")
+    want = None
+    for keep in (23, 1, 2, 5, 7, 22):
+        g = amr.NdTree(2, 6, 16, 1, 4100)
+        s = amr.AmrSolver(g, (1.0, 0.5), 0.4)
+        for _ in range(3):
+            g.refine_all()
+        s.initialize(lambda c: np.exp(-((c[..., 0] - 0.4) ** 2 + (c[..., 1] - 0.5) ** 2) / (2 * 0.06**2)))
+        x = g.get_interior().reshape(-1).copy()
+        crit = amr.make_criterion(amr.CRITERION_GRADIENT, 0.01, 0.002, 3, 6)
+        tape = amr.Tape(s, 23, crit, 3, keep)
+        info = tape.info()
+        u0 = torch.from_numpy(x).cuda()
+        uT = torch.empty(info["final_leaves"] * info["cells_per_leaf"], dtype=torch.float64, device="cuda")
+        lam = torch.from_numpy(np.random.default_rng(6).standard_normal(uT.numel())).cuda()
+        grad = torch.empty_like(u0)
+        for _ in range(2):
+            tape.forward(u0.data_ptr(), (0.9, -0.4), uT.data_ptr())
+            gv = tape.adjoint(lam.data_ptr(), grad.data_ptr())
+            got = (uT.cpu().numpy(), grad.cpu().numpy(), gv)
+            if want is None:
+                want = got
+                assert info["topologies"] > 2, info
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b), keep
