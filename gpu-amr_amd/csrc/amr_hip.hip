@@ -569,8 +569,13 @@ struct box_instance
                          double* vpart, uint32_t n, hipStream_t s)
     {
         if (n == 0) return;
-        hipLaunchKernelGGL((k_adj_step_box<R, 256>), dim3(n), dim3(256), 0, s, shape(o), lam_next, u, keys, links,
-                           metas, prm, lam, vpart, n);
+        const size_t lds = tile_bytes(o, 2);
+        if (lds <= kBoxTileBytes)
+            hipLaunchKernelGGL((k_adj_step_box_tile<R, 256>), dim3(xcd_grid(n)), dim3(256), lds, s, lam_next, u, keys,
+                               links, metas, prm, lam, n, walk_of(n, 0), small_shape(o), vpart);
+        else
+            hipLaunchKernelGGL((k_adj_step_box<R, 256>), dim3(n), dim3(256), 0, s, shape(o), lam_next, u, keys, links,
+                               metas, prm, lam, vpart, n);
         check_launch("k_adj_step_box");
     }
     static void adj_regrid(ops const& o, const double* lam_new, const uint8_t* mark, const uint8_t* head,

@@ -949,6 +949,119 @@ __global__ __launch_bounds__(NT) void k_adj_step_box(launch_box<R> B, const doub
         }
 }
 
+// k_adj_step_box for patches whose two tiles fit in LDS: u with its ghosts,
+// and lambda' with the transposed halo term of each ghost cell in that cell's
+// place.  A cell then reads its neighbours from LDS instead of walking the
+// face records of up to 4 R of them.  Cells per thread, sums and their order
+// as in k_adj_step_box.  Bound by latency on the trees that a gradient steps
+// on.  us of a 60-step forward and backward pass, from memory -> tiles: 67
+// leaves of 32^2 1847 -> 1207, 331 of 12x8 1105 -> 877, 435 of 6^3 1664 ->
+// 1203.
+template <int R, int NT>
+__global__ __launch_bounds__(NT) void k_adj_step_box_tile(const double* __restrict__ lam_next,
+                                                          const double* __restrict__ u,
+                                                          const uint64_t* __restrict__ keys,
+                                                          const face_link* __restrict__ links,
+                                                          const uint32_t* __restrict__ metas,
+                                                          const adjoint_params* __restrict__ prm_p,
+                                                          double* __restrict__ lam, uint32_t nleaves, uint32_t walk,
+                                                          launch_box<R, true> B, double* __restrict__ vpart)
+{
+    constexpr int NW = NT / 64;
+    __shared__ double red[R][NW];
+    extern __shared__ double lds[];
+    const uint32_t leaf = sweep_item(blockIdx.x, walk);
+    if (leaf >= nleaves) return;
+    const adjoint_params& prm = *prm_p;
+    const face_link*  L  = links + static_cast<size_t>(leaf) * box<R>::NDIR;
+    const uint32_t*   M  = metas + static_cast<size_t>(leaf) * box<R>::NDIR;
+    const int         lv = key_level(keys[leaf]), ni = B.ni(), tid = threadIdx.x;
+    const box_tile<R> T(B);
+    double *          ut = lds, *lt = lds + box_tile<R>::cells(B);
+    const double*     up = u + static_cast<size_t>(leaf) * ni;
+    const double*     lp = lam_next + static_cast<size_t>(leaf) * ni;
+    for (int i = tid; i < ni; i += NT)
+    {
+        int c[R];
+        B.coords(i, c);
+        const int t = T.idx(c);
+        ut[t]       = up[i];
+        lt[t]       = lp[i];
+    }
+    // the ghosts of each pair of faces, the pairs starting on different waves
+    auto ghosts = [&](auto dim) {
+        constexpr int D     = decltype(dim)::value;
+        constexpr int shift = (D * NT / R) / 64 * 64;
+        for (int q = (tid + NT - shift) % NT; q < 2 * B.face(D); q += NT)
+        {
+            int       c[R];
+            const int side = face_pair_item<R, D>(B, q, c), dir = 2 * D + side;
+            const int t    = T.idx(c);
+            double    g;
+            face_values<R, 1, D>(B, u, 0, link_ids(L + dir), M[dir], side, c, &g);
+            ut[t] = g;
+            c[D]  = 0;
+            lt[t] = adj_face_term<R>(B, lam_next, L[dir], M[dir], dir, c, lv, prm);
+        }
+    };
+    ghosts(std::integral_constant<int, 0>{});
+    ghosts(std::integral_constant<int, 1>{});
+    if constexpr (R == 3) ghosts(std::integral_constant<int, 2>{});
+    const adj_consts<R> C(prm, lv);
+    bool                coarse[2 * R];
+    for (int k = 0; k < 2 * R; ++k) coarse[k] = rel_of(M[k]) == REL_COARSER;
+    double acc_v[R];
+    for (int d = 0; d < R; ++d) acc_v[d] = 0.0;
+    __syncthreads();
+    double* out = lam + static_cast<size_t>(leaf) * ni;
+    for (int i = tid; i < ni; i += NT)
+    {
+        int c[R];
+        B.coords(i, c);
+        const int    t  = T.idx(c);
+        const double lc = lt[t], uc = ut[t];
+        double       acc = C.diag * lc;
+#pragma unroll
+        for (int d = 0; d < R; ++d)
+        {
+            const int    j = R - 1 - d, s = T.st[j]; // layout dim of physical axis d
+            const double hi = lt[t + s], lo = lt[t - s];
+            if (c[j] + 1 < B.n(j)) acc += C.ap[d] * hi;
+            if (c[j] - 1 >= 0) acc -= C.am[d] * lo;
+        }
+#pragma unroll
+        for (int dir = 0; dir < 2 * R; ++dir)
+        {
+            const int j = dir >> 1, depth = (dir & 1) ? B.n(j) - 1 - c[j] : c[j];
+            if (depth == 0 || (depth == 1 && coarse[dir]))
+                acc += lt[t + ((dir & 1) ? T.st[j] : -T.st[j]) * (depth + 1)];
+        }
+        store_cell<false>(out + i, acc);
+#pragma unroll
+        for (int d = 0; d < R; ++d)
+        {
+            const int s = T.st[R - 1 - d];
+            acc_v[d] += adj_velocity_term(uc, ut[t - s], ut[t + s], lc, C.dtdx[d], C.sgn[d]);
+        }
+    }
+    for (int d = 0; d < R; ++d)
+        for (int o = 32; o > 0; o >>= 1) acc_v[d] += __shfl_down(acc_v[d], o, 64);
+    if ((tid & 63) == 0)
+        for (int d = 0; d < R; ++d) red[d][tid >> 6] = acc_v[d];
+    __syncthreads();
+    if (tid == 0)
+        for (int d = 0; d < 3; ++d)
+        {
+            double sum = 0.0;
+            if (d < R)
+            {
+                sum = red[d][0];
+                for (int w = 1; w < NW; ++w) sum += red[d][w];
+            }
+            vpart[static_cast<size_t>(leaf) * 3 + d] = sum;
+        }
+}
+
 // The velocity partials of a run of adjoint steps, one workgroup per step:
 // step first + b wrote its leaves' triples at vpart + b * stride * 3 (leaves[]
 // per step); they are summed in one fixed order (leaves t, t + 256, ... per

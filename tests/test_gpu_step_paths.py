@@ -292,3 +292,47 @@ def test_adjoint_segments_ride_along(amr):
                 assert info["topologies"] > 2, info
             for a, b in zip(got, want):
                 assert np.array_equal(a, b), keep
+
+
+# (rank, extents): smallest, uneven, tiles that just fit in LDS and just do not
+ADJOINT_BOXES = [(2, (2, 2)), (2, (12, 8)), (2, (62, 62)), (2, (62, 64)), (2, (6, 300)), (3, (2, 2, 2)),
+                 (3, (12, 10, 6)), (3, (14, 14, 14)), (3, (14, 14, 16))]
+
+
+@pytest.mark.parametrize("rank,ext", ADJOINT_BOXES)
+def test_any_shape_adjoint(amr, rank, ext):
+    """One step of any-shape patches is linear in u and, with dt and the signs
+    of v fixed, in v: the adjoint satisfies the dot-product identity and
+    grad_v is the central difference of any width, both up to rounding (a few
+    ulp of each of the products summed, over the width)."""
+    import math
+
+    import torch
+
+    say(f"case: any-shape adjoint {ext}")
+    vel = (0.8, -0.5, 0.25)[:rank]
+    g = amr.NdTree(rank, 4, ext, 1, 200)
+    s = amr.AmrSolver(g, vel, 0.4)
+    refine_mixed(g)
+    rng = np.random.default_rng(sum(ext))
+    u0, lam = rng.standard_normal((2, g.size() * g.ni))
+    g.set_interior(u0)
+    tape = amr.Tape(s, 1, None, 0, 1)
+    u, l = torch.from_numpy(u0).cuda(), torch.from_numpy(lam).cuda()
+    out, grad = torch.empty_like(u), torch.empty_like(u)
+
+    def image(v):
+        tape.forward(u.data_ptr(), v, out.data_ptr())
+        return math.fsum(lam * out.cpu().numpy())
+
+    lhs = image(vel)
+    gv = tape.adjoint(l.data_ptr(), grad.data_ptr())
+    scale = np.linalg.norm(u0) * np.linalg.norm(lam)
+    assert abs(lhs - math.fsum(u0 * grad.cpu().numpy())) <= 1e-13 * scale
+    h = 0.125
+    for d in range(rank):
+        lo, hi = list(vel), list(vel)
+        lo[d] -= h
+        hi[d] += h
+        fd = (image(hi) - image(lo)) / (2 * h)
+        assert abs(fd - gv[d]) <= 1e-13 * scale / h, (d, fd, gv[d])
