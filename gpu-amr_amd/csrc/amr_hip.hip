@@ -161,8 +161,9 @@ constexpr size_t kBoxTileBytes = 64 * 1024; // largest LDS tile of the any-shape
 //    42.5 / 44.5),
 //  - LDS for four (2D) or three (3D) waves per SIMD, what the registers allow
 //    (12^3, 1583 leaves, strips of 12 / 6 layers 126 / 92 us),
-// but not under four layers for these: a strip forms the states of one layer
-// below and one above its own.  0 where a layer has more than 512 cells or
+// but not under four layers (three of patches with fewer than eight: 64 leaves
+// of 6^3, six / three layers 20.7 / 15.3 us) for these: a strip forms the states of one
+// layer below and one above its own.  0 where a layer has more than 512 cells or
 // its strip exceeds 64 KiB of LDS.
 template <int R>
 int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
@@ -181,11 +182,8 @@ int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
     for (int g = 1;; ++g)
     {
         const int layers = (o.ext[0] + side_by_side * g - 1) / (side_by_side * g);
-        if (g > 1 && (layers < 4 || layers == W.layers))
-        {
-            if (layers < 4) break;
-            continue;
-        }
+        if (g > 1 && layers < (o.ext[0] < 8 ? 3 : 4)) break;
+        if (g > 1 && layers == W.layers) continue;
         const int strips = (o.ext[0] + layers - 1) / layers;
         W.layers         = layers;
         W.segs           = std::min(side_by_side, strips);

@@ -969,8 +969,19 @@ __global__ __launch_bounds__(NT) void k_step(const double* __restrict__ u, doubl
     const step_consts<R> C = leaf_consts<FROM, R>(prm, table, who, lv);
     __syncthreads();
     double* out = un + static_cast<size_t>(leaf) * S::NI;
+    // Through L2 (store_cell) only where a step writes enough for it: us per
+    // step, plain / through, 64^2: 64 leaves 8.5 / 10.2, 256 11.6 / 12.6, 484
+    // 14.8 / 13.6, 1024 19.7 / 17.2; of the small patches 484 leaves of 8^2 6.7 / 7.1, 2339 of
+    // 4^3 (three steps) 33.6 / 35.8 us, 12692 of 4^3 12.3 / 12.8.
+    const bool through = S::NI >= 4096 && nleaves >= 400;
     for (int i = threadIdx.x; i < S::NI; i += NT)
-        store_cell<false>(out + i, upwind_cell<R, N>(tile, i, C.dtdx, C.vel, C.hs));
+    {
+        const double v = upwind_cell<R, N>(tile, i, C.dtdx, C.vel, C.hs);
+        if (through)
+            store_cell<false>(out + i, v);
+        else
+            out[i] = v;
+    }
 }
 
 // 3D 8^3 patches, one wave (64 lanes) per leaf.  Lane l owns the z-column at
