@@ -460,11 +460,11 @@ ops const* find_ops(int rank, int n, int h)
     return nullptr;
 }
 
-// Kernels for every other patch shape (any even extents, square or not):
-// the box kernels, the extents passed at launch, one workgroup per leaf of
-// 64 threads for patches of up to 64 cells and 256 otherwise.  They read
-// neighbour cells from memory instead of LDS tiles; the arithmetic is the
-// fixed-shape kernels', so results are the same bits.
+// Kernels for every other patch shape (any even extents, square or not): the
+// extents are launch arguments.  Steps, Euler steps and adjoint steps go
+// through LDS where their tile or strip fits; the others, and larger patches,
+// read neighbour cells from memory.  The arithmetic is the fixed-shape
+// kernels', so results are the same bits.
 template <int R>
 struct box_instance
 {
