@@ -308,10 +308,10 @@ struct instance
     {
         if (n == 0) return;
         if (kind == AMR_CRITERION_GRADIENT)
-            hipLaunchKernelGGL((k_criterion_gradient<R, N, NT>), dim3(n), dim3(NT), 0, s, u, keys, links, metas, r, c,
+            hipLaunchKernelGGL((k_criterion_gradient<R, N, NT>), dim3(xcd_grid(n)), dim3(NT), 0, s, u, keys, links, metas, r, c,
                                mn, mx, flags, n);
         else
-            hipLaunchKernelGGL((k_criterion_max<R, N, H, NTP>), dim3(n), dim3(NTP), 0, s, u, keys, links, metas, r, c,
+            hipLaunchKernelGGL((k_criterion_max<R, N, H, NTP>), dim3(xcd_grid(n)), dim3(NTP), 0, s, u, keys, links, metas, r, c,
                                mn, mx, flags, n);
         check_launch("k_criterion");
     }
@@ -545,10 +545,10 @@ struct box_instance
     {
         if (n == 0) return;
         if (kind == AMR_CRITERION_GRADIENT)
-            hipLaunchKernelGGL((k_criterion_gradient_box<R, 256>), dim3(n), dim3(256), 0, s, shape(o), u, keys, links,
+            hipLaunchKernelGGL((k_criterion_gradient_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, shape(o), u, keys, links,
                                metas, r, c, mn, mx, flags, n);
         else
-            hipLaunchKernelGGL((k_criterion_max_box<R, 256>), dim3(n), dim3(256), 0, s, shape(o), o.h, u, keys, links,
+            hipLaunchKernelGGL((k_criterion_max_box<R, 256>), dim3(xcd_grid(n)), dim3(256), 0, s, shape(o), o.h, u, keys, links,
                                metas, r, c, mn, mx, flags, n);
         check_launch("k_criterion_box");
     }

@@ -1312,14 +1312,13 @@ __global__ __launch_bounds__(NT) void k_padded_view(const double* __restrict__ u
 template <int NT>
 __device__ inline double block_max(double v, double* red)
 {
-    red[threadIdx.x] = v;
+    // each wave by shuffles, then the waves' values: one barrier
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_down(v, o, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int s = NT / 2; s > 0; s >>= 1)
-    {
-        if (static_cast<int>(threadIdx.x) < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
-    }
-    return red[0];
+    v = red[0];
+    for (int w = 1; w < NT / 64; ++w) v = fmax(v, red[w]);
+    return v;
 }
 
 // Undivided-gradient criterion: one workgroup per leaf.
@@ -1333,15 +1332,16 @@ __global__ __launch_bounds__(NT) void k_criterion_gradient(const double* __restr
 {
     using S = patch_shape<R, N>;
     __shared__ double tile[tile_shape<R, N>::TS];
-    __shared__ double red[NT];
-    const uint32_t leaf = blockIdx.x;
+    __shared__ double red[NT / 64];
+    const uint32_t leaf = xcd_item(blockIdx.x, gridDim.x);
     if (leaf >= nleaves) return;
+    const int lv = key_level(keys[leaf]);
     stage_tile<R, N, NT>(tile, u, leaf, links, metas);
     __syncthreads();
     double g = 0.0;
     for (int i = threadIdx.x; i < S::NI; i += NT) g = fmax(g, gradient_cell<R, N>(tile, i));
     g = block_max<NT>(g, red);
-    if (threadIdx.x == 0) flags[leaf] = decide(g, key_level(keys[leaf]), rthr, cthr, min_level, max_level);
+    if (threadIdx.x == 0) flags[leaf] = decide(g, lv, rthr, cthr, min_level, max_level);
 }
 
 // Face-halo cells of a patch with h ghost layers: h * face(dim) items per
@@ -1393,10 +1393,20 @@ __device__ inline double leaf_max_value(BX const& B, int h, const double* __rest
                                         const face_link* __restrict__ links, const uint32_t* __restrict__ metas,
                                         double* red)
 {
-    double        m  = 0.0;
+    // the first cells of a thread are in flight while it follows its ghost's
+    // record (with that, leaves kept to their XCD and a maximum of one barrier
+    // instead of nine: 900 leaves of 64^2 on average 10.8 -> 7.4 us, of 32^2
+    // 6.5 -> 5.1; the gradient criterion on 200 leaves of 16^2 4.4 -> 3.7)
+    constexpr int CH = 16;
+    double        m  = 0.0, r[CH];
     const int     ni = B.ni();
     const double* up = u + static_cast<size_t>(leaf) * ni;
-    for (int i = threadIdx.x; i < ni; i += NT) m = fmax(m, up[i]);
+#pragma unroll
+    for (int k = 0; k < CH; ++k)
+    {
+        const int i = threadIdx.x + k * NT;
+        r[k]        = i < ni ? up[i] : 0.0;
+    }
     const int items = halo_items<R>(B, h);
     for (int g = threadIdx.x; g < items; g += NT)
     {
@@ -1405,6 +1415,9 @@ __device__ inline double leaf_max_value(BX const& B, int h, const double* __rest
         const size_t   e   = static_cast<size_t>(leaf) * box<R>::NDIR + dir;
         m                  = fmax(m, ghost_value<R>(B, u, links[e], metas[e], dir, c));
     }
+#pragma unroll
+    for (int k = 0; k < CH; ++k) m = fmax(m, r[k]);
+    for (int i = threadIdx.x + CH * NT; i < ni; i += NT) m = fmax(m, up[i]);
     return block_max<NT>(m, red);
 }
 
@@ -1419,11 +1432,12 @@ __global__ __launch_bounds__(NT) void k_criterion_max(const double* __restrict__
                                                       uint32_t nleaves)
 {
     constexpr box<R>  B = box<R>::cube(N);
-    __shared__ double red[NT];
-    const uint32_t    leaf = blockIdx.x;
+    __shared__ double red[NT / 64];
+    const uint32_t    leaf = xcd_item(blockIdx.x, gridDim.x);
     if (leaf >= nleaves) return;
+    const int lv = key_level(keys[leaf]);
     const double m = leaf_max_value<R, NT>(B, H, u, leaf, links, metas, red);
-    if (threadIdx.x == 0) flags[leaf] = decide(m, key_level(keys[leaf]), rthr, cthr, min_level, max_level);
+    if (threadIdx.x == 0) flags[leaf] = decide(m, lv, rthr, cthr, min_level, max_level);
 }
 
 // ---------------------------------------------------------------------------
@@ -1502,14 +1516,15 @@ __global__ __launch_bounds__(NT) void k_criterion_gradient_box(launch_box<R> B, 
                                                                double cthr, int min_level, int max_level,
                                                                int8_t* __restrict__ flags, uint32_t nleaves)
 {
-    __shared__ double red[NT];
-    const uint32_t    leaf = blockIdx.x;
+    __shared__ double red[NT / 64];
+    const uint32_t    leaf = xcd_item(blockIdx.x, gridDim.x);
     if (leaf >= nleaves) return;
+    const int lv = key_level(keys[leaf]);
     double    g  = 0.0;
     const int ni = B.ni();
     for (int i = threadIdx.x; i < ni; i += NT) g = fmax(g, gradient_cell_direct<R>(B, u, leaf, links, metas, i));
     g = block_max<NT>(g, red);
-    if (threadIdx.x == 0) flags[leaf] = decide(g, key_level(keys[leaf]), rthr, cthr, min_level, max_level);
+    if (threadIdx.x == 0) flags[leaf] = decide(g, lv, rthr, cthr, min_level, max_level);
 }
 
 template <int R, int NT>
@@ -1520,11 +1535,12 @@ __global__ __launch_bounds__(NT) void k_criterion_max_box(launch_box<R> B, int h
                                                           int min_level, int max_level, int8_t* __restrict__ flags,
                                                           uint32_t nleaves)
 {
-    __shared__ double red[NT];
-    const uint32_t    leaf = blockIdx.x;
+    __shared__ double red[NT / 64];
+    const uint32_t    leaf = xcd_item(blockIdx.x, gridDim.x);
     if (leaf >= nleaves) return;
+    const int lv = key_level(keys[leaf]);
     const double m = leaf_max_value<R, NT>(B, h, u, leaf, links, metas, red);
-    if (threadIdx.x == 0) flags[leaf] = decide(m, key_level(keys[leaf]), rthr, cthr, min_level, max_level);
+    if (threadIdx.x == 0) flags[leaf] = decide(m, lv, rthr, cthr, min_level, max_level);
 }
 
 } // namespace amrhip
