@@ -934,7 +934,6 @@ struct amr_ctx
     int             nvar  = 1;
     double          gamma = 1.4;
     euler_slot*     esc   = nullptr; // the kEulerSlots device scalars of the dt logic
-    uint32_t        euler_last = 1;  // slot with the last batch's sums
     bool            euler_cut  = false; // a launch of the last batch failed: slot 0 may not be empty
     size_t          fstride() const { return static_cast<size_t>(cap) * static_cast<size_t>(ni); }
     bool            euler() const { return nvar > 1; }
@@ -1142,15 +1141,14 @@ struct amr_ctx
     // slot 0, then one launch per step, which forms its dt itself
     // (euler_step_dt) and folds the next step's dt minimum over the cells it
     // writes (the values the reduction would read back, so the same
-    // minimum); dt never visits the host.  Every batch leaves slot 0 empty,
-    // so that a captured batch can be replayed.
+    // minimum); dt never visits the host.  Every batch leaves slot 0 empty
+    // and its sums in kEulerSumSlot, so that a captured batch can be replayed.
     void euler_advance(uint64_t steps, double remaining)
     {
         ensure_usable();
         if (steps == 0)
         {
-            euler_clear(1);
-            euler_last = 1;
+            euler_clear(kEulerSumSlot);
             return;
         }
         euler_params   prm = make_euler_params();
@@ -1166,7 +1164,7 @@ struct amr_ctx
         {
             prm.next_dt  = s + 1 < steps ? 1u : 0u;
             prm.now      = s == 0 ? 0u : 1u + static_cast<uint32_t>((s - 1) % 3);
-            prm.next     = 1u + static_cast<uint32_t>(s % 3);
+            prm.next     = s + 1 < steps ? 1u + static_cast<uint32_t>(s % 3) : kEulerSumSlot;
             prm.clear    = 1u + static_cast<uint32_t>((s + 1) % 3);
             prm.first    = s == 0 ? 1u : 0u;
             prm.clear_dt = s == 1 ? 1u : 0u;
@@ -1174,7 +1172,6 @@ struct amr_ctx
                            static_cast<uint32_t>(sweeps++ & 1), nn, stream);
             cur = 1 - cur;
         }
-        euler_last = prm.next;
         if (steps == 1) euler_clear(0);
         euler_cut = false;
     }
@@ -2524,7 +2521,7 @@ int amr_solver_finish_advance_batch(amr_ctx* ctx, double* dt_sum, uint64_t* exec
             if (!ctx) throw amr_error(AMR_ERR_ARGUMENT, "null argument");
             if (ctx->euler())
             {
-                const euler_scalars e = ctx->euler_read(ctx->euler_last);
+                const euler_scalars e = ctx->euler_read(kEulerSumSlot);
                 ctx->pending_dt       = e.acc;
                 ctx->pending_steps    = e.executed;
             }

@@ -23,7 +23,10 @@ namespace amrhip
 // (the loop's break) and the running minimum of dx / speed (as the bits of a
 // non-negative double, so that an integer atomicMin orders it) in
 // kEulerParts parts.  A context holds kEulerSlots of them: the first step of a batch takes its dt from
-// slot 0, which k_euler_dt filled, the later ones from slots 1, 2, 3 in turn.
+// slot 0, which k_euler_dt filled, the later ones from slots 1, 2, 3 in turn;
+// the last one leaves the batch's sums in a slot of their own, the same for
+// every batch, so that they are found there also after a batch that a captured
+// graph ran without the host's knowing.
 // A step launch reads its own slot, folds the next step's minimum and writes
 // the sums into the next one and empties the minimum of the one after that,
 // so every workgroup forms the step's dt itself and no launch is needed
@@ -61,7 +64,8 @@ struct alignas(128) euler_slot
 };
 
 constexpr uint32_t kEulerNowSlot = 4; // amr_solver_compute_dt's minimum
-constexpr uint32_t kEulerSlots   = 5;
+constexpr uint32_t kEulerSumSlot = 5; // the last batch's sums
+constexpr uint32_t kEulerSlots   = 6;
 
 // Per-launch constants of the Euler kernels: gamma, the cell sizes of every
 // level (physics_system::cell_sizes, formed on the host) and the step's place

@@ -54,6 +54,37 @@ def test_euler_batch_lengths(amr):
     assert_fields(s.tree.get_interior(), o.get_interior(), "after the batches")
 
 
+def test_euler_batch_captured(amr):
+    """An Euler batch recorded into a graph on the context's stream and
+    replayed, with plain batches in between: finish_advance_batch returns the
+    sums of whichever ran last."""
+    import torch
+
+    say("case: captured Euler batch")
+    made = []
+    for _ in range(2):
+        s = amr.EulerSolver(2, 6, 16, 1, 72, (1.0, 1.0), 1.4, 0.3)
+        for _ in range(2):
+            s.tree.refine_all()
+        rng = np.random.default_rng(11)
+        u0 = np.empty((4, s.tree.size() * s.tree.ni))
+        u0[0], u0[1:3], u0[3] = rng.uniform(0.5, 1.5, u0.shape[1]), rng.uniform(-0.5, 0.5, u0[1:3].shape), 3.0
+        s.tree.set_interior(u0)
+        made.append(s)
+    s, plain = made
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(torch.cuda.ExternalStream(s.tree.stream())):
+        graph.capture_begin()
+        s.advance_batch_async(2)  # recorded, not run
+        graph.capture_end()
+        for steps in (4, None, None, 6, None, 2, None):
+            (s.advance_batch_async(steps) if steps else graph.replay())
+            plain.advance_batch_async(steps or 2)
+            assert s.finish_advance_batch() == plain.finish_advance_batch(), steps
+            assert s.compute_dt() == plain.compute_dt(), steps
+            assert_fields(s.tree.get_interior(), plain.tree.get_interior(), f"after {steps}")
+
+
 def upwind_of_padded(g, vel, dt):
     """One step in numpy from the library's padded patches (the halos that
     brute-force geometry checks elsewhere), in time_step_cpu's expression
