@@ -6,6 +6,7 @@
 // constants; all per-cell and per-leaf work runs in the kernels of
 // kernels_step.hpp / kernels_tree.hpp.
 #include "amr_hip.h"
+#include "batch_groups.hpp"
 #include "device_common.hpp"
 #include "kernels_adjoint.hpp"
 #include "kernels_euler.hpp"
@@ -1324,7 +1325,8 @@ struct amr_batch
     // of the group fit: us per step (GB/s) of 16^2 patches in one launch, 225
     // MB 33.4 (6716), 246 MB 36.9 (6651), 268 MB 50.7 (5290), 358 MB 82.5
     // (4337); of 8^3 226 MB 40.4 (5593), 254 MB 46.3 (5499), 283 MB 63.0
-    // (4495).  A tree larger than that is a group of its own.
+    // (4495).  A group holds consecutive trees of kGroupBytes at most, with
+    // their tables; a tree larger than that is a group of its own.
     static constexpr uint64_t kGroupBytes = 224ull << 20;
     struct group
     {
@@ -1333,25 +1335,24 @@ struct amr_batch
     };
     std::vector<std::unique_ptr<group>> groups;
 
-    // Splits the instances (`off`, `total`) into groups of about equal size.
+    // Leaves of instance i.
+    uint64_t leaves_of(size_t i) const { return (i + 1 < off.size() ? off[i + 1] : total) - off[i]; }
+
+    // Splits the instances (`off`, `total`) into the fewest groups that keep
+    // to kGroupBytes, of about equal size.
     void make_groups()
     {
         const uint64_t leaf_bytes = 2 * static_cast<uint64_t>(ni) * sizeof(double) + sizeof(uint64_t) + sizeof(uint32_t) +
                                     static_cast<uint64_t>(ndir) * (sizeof(face_link) + sizeof(uint32_t));
-        const uint64_t want = std::max<uint64_t>((total * leaf_bytes + kGroupBytes - 1) / kGroupBytes, 1);
-        uint64_t       last = 0;
-        for (size_t i = 0; i < off.size(); ++i)
+        std::vector<uint64_t> leaves(off.size());
+        for (size_t i = 0; i < off.size(); ++i) leaves[i] = leaves_of(i);
+        for (size_t i : even_runs(leaves, kGroupBytes / leaf_bytes))
         {
-            const uint64_t end = i + 1 < off.size() ? off[i + 1] : total;
-            const uint64_t at  = total ? std::min((off[i] + end) / 2 * want / total, want - 1) : 0;
-            if (groups.empty() || at != last)
-            {
-                groups.push_back(std::make_unique<group>());
-                groups.back()->first = off[i];
-            }
-            groups.back()->leaves = end - groups.back()->first;
-            last                  = at;
+            groups.push_back(std::make_unique<group>());
+            groups.back()->first = off[i];
         }
+        for (size_t g = 0; g < groups.size(); ++g)
+            groups[g]->leaves = (g + 1 < groups.size() ? groups[g + 1]->first : total) - groups[g]->first;
     }
     group& group_of(size_t instance)
     {

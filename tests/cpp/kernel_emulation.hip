@@ -1,12 +1,14 @@
 // kernel_emulation.hip -- runs the HIP kernels' per-item bodies on the CPU
 // (host-only build), one "workgroup" after another, so that the device logic
 // can be compared with the oracle without a GPU.  Test infrastructure only.
+#include "batch_groups.hpp"
 #include "device_common.hpp"
 #include "kernels_step.hpp"
 #include "kernels_tree.hpp"
 #include "kernels_adjoint.hpp"
 #include "kernels_fused.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -584,6 +586,15 @@ int emu_adj_regrid_box(int rank, const int* ext, const double* lam_new, const ui
     else
         adj_regrid_box<3>(ext, lam_new, maps, n_old, lam_old);
     return 0;
+}
+
+// The batch's split of trees of `size` leaves into groups of at most `most`:
+// their first trees in `first`, their number returned.
+uint32_t emu_batch_groups(const uint64_t* size, uint64_t count, uint64_t most, uint64_t* first)
+{
+    const auto runs = even_runs(std::vector<uint64_t>(size, size + count), most);
+    std::copy(runs.begin(), runs.end(), first);
+    return static_cast<uint32_t>(runs.size());
 }
 
 } // extern "C"

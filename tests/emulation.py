@@ -230,3 +230,13 @@ def adj_regrid_box(rank, ext, lam_new, maps, n_old):
     lam_old = np.zeros(n_old * int(np.prod(ext)))
     load().emu_adj_regrid_box(rank, _ext(ext), _p(lam_new), _p(maps), ctypes.c_uint32(n_old), _p(lam_old))
     return lam_old
+
+
+def batch_groups(sizes, most):
+    """First tree of every group of a batch of trees of `sizes` leaves."""
+    sizes = np.ascontiguousarray(sizes, dtype=np.uint64)
+    first = np.zeros(sizes.size, dtype=np.uint64)
+    fn = load().emu_batch_groups
+    fn.restype = ctypes.c_uint32
+    count = fn(_p(sizes), ctypes.c_uint64(sizes.size), ctypes.c_uint64(int(most)), _p(first))
+    return first[:count].astype(int).tolist()
