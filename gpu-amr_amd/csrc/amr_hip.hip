@@ -820,14 +820,17 @@ int autotune_steps(ops const* op, const double* u_cur, double* u_other, uint64_t
     return best;
 }
 
-// Batch packing: shift an instance's neighbour slots by its leaf offset, and
-// tag its leaves with the instance index.
-__global__ void k_offset_links(face_link* __restrict__ links, uint64_t count, int32_t offset)
+// Batch packing: an instance's neighbour records with their slots shifted by
+// its leaf offset, and the tag of its leaves with the instance index.
+__global__ void k_offset_links(const face_link* __restrict__ from, face_link* __restrict__ to, uint64_t count,
+                               int32_t offset)
 {
     const uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
     if (i >= count) return;
+    face_link l = from[i];
     for (int j = 0; j < 4; ++j)
-        if (links[i].ids[j] >= 0) links[i].ids[j] += offset;
+        if (l.ids[j] >= 0) l.ids[j] += offset;
+    to[i] = l;
 }
 
 // The states of up to kScatterTrees instances from the batch's buffer back to
@@ -1312,9 +1315,9 @@ struct amr_batch
     double*                  u[2]{};
     int                      cur     = 0;
     int                      variant = 0;
-    uint64_t                 sweeps  = 0;
     uint64_t*                keys    = nullptr;
-    face_link*               links   = nullptr;
+    face_link*               links   = nullptr; // neighbour slots count from the group's first leaf
+    face_link*               whole_links = nullptr; // from the batch's; with several groups only
     uint32_t*                metas   = nullptr;
     uint32_t*                inst    = nullptr;
     step_params*             table   = nullptr;
@@ -1330,10 +1333,21 @@ struct amr_batch
     static constexpr uint64_t kGroupBytes = 224ull << 20;
     struct group
     {
-        uint64_t  first = 0, leaves = 0; // its leaves; neighbour slots count from `first`
-        run_lists runs;
+        uint64_t         first = 0, leaves = 0;
+        const face_link* links = nullptr; // of its leaves, slots counting from `first`
+        run_lists        runs;
     };
     std::vector<std::unique_ptr<group>> groups;
+    group                               whole; // all leaves; with several groups only
+
+    // Calls of up to this many steps step the whole batch at once: a group
+    // stepped once or twice finds little of itself in the cache, and one
+    // launch over all leaves, whose direction alternates from step to step,
+    // starts on the part of the last step's result that is still there.  us a
+    // call of 1 / 2 / 3 steps, by groups -> at once: 448 MB of 16^2 122 / 233 /
+    // 304 -> 103 / 208 / 297, 699 MB 180 / 347 / 452 -> 168 / 334 / 484, 437 MB
+    // of 8^3 130 / 243 / 313 -> 117 / 232 / 331.
+    static constexpr uint64_t kWholeSteps = 2;
 
     // Leaves of instance i.
     uint64_t leaves_of(size_t i) const { return (i + 1 < off.size() ? off[i + 1] : total) - off[i]; }
@@ -1353,6 +1367,7 @@ struct amr_batch
         }
         for (size_t g = 0; g < groups.size(); ++g)
             groups[g]->leaves = (g + 1 < groups.size() ? groups[g + 1]->first : total) - groups[g]->first;
+        whole.leaves = total;
     }
     group& group_of(size_t instance)
     {
@@ -1373,7 +1388,8 @@ struct amr_batch
     {
         if (stream) (void)hipStreamSynchronize(stream);
         for (auto& g : graphs) (void)hipGraphExecDestroy(g.exec);
-        for (void* p : { (void*)u[0], (void*)u[1], (void*)keys, (void*)links, (void*)metas, (void*)inst, (void*)table })
+        for (void* p : { (void*)u[0], (void*)u[1], (void*)keys, (void*)links, (void*)whole_links, (void*)metas, (void*)inst,
+                         (void*)table })
             if (p) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -1384,19 +1400,28 @@ struct amr_batch
     {
         step_params prm = host_table[0];
         prm.reverse     = reverse;
-        op->step(*op, v, in, out, keys + g.first, links + g.first * ndir,
-                 metas + g.first * ndir, prm, table, inst + g.first, static_cast<uint32_t>(g.leaves), g.runs.view(), stream);
+        op->step(*op, v, in, out, keys + g.first, g.links, metas + g.first * ndir, prm, table, inst + g.first,
+                 static_cast<uint32_t>(g.leaves), g.runs.view(), stream);
+    }
+
+    // The steps of an advance on one group.  A step walks its leaves forwards
+    // from buffer 0 and backwards from buffer 1, so consecutive steps
+    // alternate, also across calls and graph replays.
+    void launch_group(group& g, uint64_t steps)
+    {
+        for (uint64_t k = 0; k < steps; ++k)
+        {
+            const int from = cur ^ static_cast<int>(k & 1);
+            step_group(g, variant, u[from] + g.first * ni, u[1 - from] + g.first * ni, static_cast<uint32_t>(from));
+        }
     }
 
     void launch_steps(uint64_t steps)
     {
-        for (auto& g : groups)
-            for (uint64_t k = 0; k < steps; ++k)
-            {
-                const int from = cur ^ static_cast<int>(k & 1);
-                step_group(*g, variant, u[from] + g->first * ni, u[1 - from] + g->first * ni,
-                           static_cast<uint32_t>((sweeps + k) & 1));
-            }
+        if (groups.size() > 1 && steps <= kWholeSteps)
+            launch_group(whole, steps);
+        else
+            for (auto& g : groups) launch_group(*g, steps);
     }
 
     // Every instance advances `steps` steps with its own dt.  With use_graph
@@ -1407,7 +1432,6 @@ struct amr_batch
         if (!use_graph)
         {
             launch_steps(steps);
-            sweeps += steps;
             cur ^= static_cast<int>(steps & 1);
             return;
         }
@@ -2711,6 +2735,8 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
             b->keys  = dev_alloc<uint64_t>(b->total);
             b->links = dev_alloc<face_link>(b->total * b->ndir);
             b->metas = dev_alloc<uint32_t>(b->total * b->ndir);
+            if (b->groups.size() > 1) b->whole.links = b->whole_links = dev_alloc<face_link>(b->total * b->ndir);
+            for (auto& g : b->groups) g->links = b->links + g->first * b->ndir;
             b->inst  = dev_alloc<uint32_t>(b->total);
             b->table = dev_alloc<step_params>(count);
             for (uint32_t i = 0; i < count; ++i)
@@ -2721,13 +2747,14 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
                                              hipMemcpyDeviceToDevice, b->stream));
                 AMR_HIP_CHECK(hipMemcpyAsync(b->keys + o, t->keys[t->kc], t->n * sizeof(uint64_t),
                                              hipMemcpyDeviceToDevice, b->stream));
-                AMR_HIP_CHECK(hipMemcpyAsync(b->links + o * b->ndir, t->links, t->n * b->ndir * sizeof(face_link),
-                                             hipMemcpyDeviceToDevice, b->stream));
                 AMR_HIP_CHECK(hipMemcpyAsync(b->metas + o * b->ndir, t->metas, t->n * b->ndir * sizeof(uint32_t),
                                              hipMemcpyDeviceToDevice, b->stream));
                 const uint64_t nl = t->n * b->ndir;
-                hipLaunchKernelGGL(k_offset_links, dim3(grid1d(nl, 256)), dim3(256), 0, b->stream, b->links + o * b->ndir,
-                                   nl, static_cast<int32_t>(o - b->group_of(i).first));
+                hipLaunchKernelGGL(k_offset_links, dim3(grid1d(nl, 256)), dim3(256), 0, b->stream, t->links,
+                                   b->links + o * b->ndir, nl, static_cast<int32_t>(o - b->group_of(i).first));
+                if (b->whole_links)
+                    hipLaunchKernelGGL(k_offset_links, dim3(grid1d(nl, 256)), dim3(256), 0, b->stream, t->links,
+                                       b->whole_links + o * b->ndir, nl, static_cast<int32_t>(o));
                 hipLaunchKernelGGL(k_fill_instance, dim3(grid1d(t->n, 256)), dim3(256), 0, b->stream, b->inst + o, t->n,
                                    i);
                 check_launch("batch packing");
@@ -2736,12 +2763,15 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
             AMR_HIP_CHECK(hipMemcpyAsync(b->table, b->host_table.data(), count * sizeof(step_params),
                                          hipMemcpyHostToDevice, b->stream));
             if (run_lists::wanted(b->op))
-                for (auto& g : b->groups)
-                {
-                    g->runs.allocate(g->leaves);
-                    g->runs.build(b->op->rank, b->keys + g->first, static_cast<uint32_t>(g->leaves), trees[0]->depth,
-                                  b->links + g->first * b->ndir, b->metas + g->first * b->ndir, b->stream);
-                }
+            {
+                auto build_runs = [&](amr_batch::group& g) {
+                    g.runs.allocate(g.leaves);
+                    g.runs.build(b->op->rank, b->keys + g.first, static_cast<uint32_t>(g.leaves), trees[0]->depth,
+                                 g.links, b->metas + g.first * b->ndir, b->stream);
+                };
+                for (auto& g : b->groups) build_runs(*g);
+                if (b->whole_links) build_runs(b->whole);
+            }
             AMR_HIP_CHECK(hipStreamSynchronize(b->stream));
             *out = b.release();
         }

@@ -163,3 +163,37 @@ def test_batch_larger_than_the_cache_matches_sequential(amr, rank, n, level):
     batch.scatter()
     for i, (s, u) in enumerate(zip(solvers, expected)):
         assert np.array_equal(s.tree.get_interior().view(np.uint64), u.view(np.uint64)), f"instance {i}"
+
+
+def test_batch_of_groups_short_and_long_calls(amr):
+    """Calls of one to four steps on a batch of several groups (the short ones
+    run on all leaves at once), per-leaf and run kernels, eager and by graph,
+    against the sequential solves after every call."""
+    say("case: short and long calls on a batch of several groups")
+    rng = np.random.default_rng(12)
+    solvers = []
+    for _ in range(8):  # 8 x 64 MiB of state
+        tree = amr.NdTree(2, 7, 16, 1, 1 << 14)
+        solvers.append(amr.AmrSolver(tree, tuple(rng.uniform(-1.0, 1.0, 2)), 0.4))
+        for _ in range(7):
+            tree.refine_all()
+        tree.set_interior(rng.standard_normal(tree.size() * tree.ni))
+    other = []
+    for s in solvers:
+        tree = amr.NdTree(2, 7, 16, 1, 1 << 14)
+        other.append(amr.AmrSolver(tree, s.velocity, 0.4))
+        for _ in range(7):
+            tree.refine_all()
+        tree.set_interior(s.tree.get_interior())
+    batch = amr.Batch([s.tree for s in solvers])
+    run8 = solvers[0].step_variants().index("run8")
+    for variant, steps, graph in ((0, 1, False), (run8, 3, False), (run8, 1, True), (run8, 1, True), (0, 2, True),
+                                  (0, 4, False), (run8, 2, False), (0, 1, True), (0, 1, True), (0, 2, True)):
+        batch.set_step_variant(variant)
+        batch.advance(steps, use_graph=graph)
+        batch.scatter()
+        for i, (s, o) in enumerate(zip(solvers, other)):
+            o.advance_batch_async(steps)
+            o.finish_advance_batch()
+            a, b = s.tree.get_interior(), o.tree.get_interior()
+            assert np.array_equal(a.view(np.uint64), b.view(np.uint64)), (variant, steps, graph, i)
