@@ -280,7 +280,9 @@ int amr_batch_size(amr_batch* batch, uint64_t* total_leaves);
  * replays it as a single graph launch.  Returns without waiting. */
 int amr_batch_advance(amr_batch* batch, uint64_t steps, int use_graph);
 int amr_batch_synchronize(amr_batch* batch);
-/* Writes each instance's current interiors back into its source tree. */
+/* Writes each instance's current interiors back into its source tree.  A tree
+ * whose leaf count has changed since the batch was made is refused
+ * (AMR_ERR_ARGUMENT) before any tree is written. */
 int amr_batch_scatter(amr_batch* batch);
 int amr_batch_stream(amr_batch* batch, void** hip_stream);
 int amr_batch_set_step_variant(amr_batch* batch, int32_t variant);

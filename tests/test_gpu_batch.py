@@ -197,3 +197,53 @@ def test_batch_of_groups_short_and_long_calls(amr):
             o.finish_advance_batch()
             a, b = s.tree.get_interior(), o.tree.get_interior()
             assert np.array_equal(a.view(np.uint64), b.view(np.uint64)), (variant, steps, graph, i)
+
+
+def test_scatter_refuses_a_regridded_tree(amr):
+    """A tree refined or coarsened since the batch was made, first, in the
+    middle or last: scatter raises and no tree is written."""
+    say("case: scatter into regridded trees")
+    for which, flag in ((1, "REFINE"), (1, "COARSEN"), (0, "REFINE"), (2, "REFINE"), (2, "COARSEN")):
+        trees = []
+        for k in range(3):
+            t = amr.NdTree(2, 6, 16, 1, 200)
+            s = amr.AmrSolver(t, (1.0, 0.5), 0.4)
+            for _ in range(3):
+                t.refine_all()
+            t.set_interior(np.random.default_rng(k).standard_normal(t.size() * t.ni))
+            trees.append((t, s))
+        batch = amr.Batch([t for t, _ in trees])
+        batch.advance(2, use_graph=False)
+        flags = np.zeros(64, dtype=np.int8)
+        flags[:4] = getattr(amr, flag)
+        assert trees[which][0].reconstruct_tree(flags)
+        before = [t.get_interior() for t, _ in trees]
+        with pytest.raises(amr.AmrError):
+            batch.scatter()
+        batch.synchronize()
+        for (t, _), u in zip(trees, before):
+            assert np.array_equal(t.get_interior().view(np.uint64), u.view(np.uint64)), (which, flag)
+
+
+def test_batch_of_more_trees_than_a_scatter_launch(amr):
+    """300 trees of different sizes: the scatter takes several launches."""
+    say("case: batch of 300 trees")
+    rng = np.random.default_rng(5)
+    solvers, other = [], []
+    for k in range(300):
+        u = None
+        v = tuple(rng.uniform(-1.0, 1.0, 2))
+        for made in (solvers, other):
+            t = amr.NdTree(2, 4, 8, 1, 16)
+            made.append(amr.AmrSolver(t, v, 0.4))
+            for _ in range(k % 3):
+                t.refine_all()
+            u = rng.standard_normal(t.size() * t.ni) if u is None else u
+            t.set_interior(u)
+    batch = amr.Batch([s.tree for s in solvers])
+    batch.advance(3)
+    batch.scatter()
+    for k, (s, o) in enumerate(zip(solvers, other)):
+        o.advance_batch_async(3)
+        o.finish_advance_batch()
+        assert np.array_equal(s.tree.get_interior().view(np.uint64), o.tree.get_interior().view(np.uint64)), k
