@@ -659,9 +659,9 @@ T* dev_alloc(size_t count)
 inline unsigned grid1d(uint64_t items, unsigned threads) { return static_cast<unsigned>((items + threads - 1) / threads); }
 
 // Times `trials` launches of every variant, three interleaved rounds, and
-// returns the variant with the lowest per-launch time (min over rounds).
+// returns each variant's time per launch in us (min over rounds).
 template <typename Launch>
-int pick_fastest(int nvar, Launch&& launch, hipStream_t stream, uint32_t trials, float* best_us)
+std::vector<float> time_variants(int nvar, Launch&& launch, hipStream_t stream, uint32_t trials)
 {
     hipEvent_t e0, e1;
     AMR_HIP_CHECK(hipEventCreate(&e0));
@@ -684,9 +684,15 @@ int pick_fastest(int nvar, Launch&& launch, hipStream_t stream, uint32_t trials,
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    const auto it = std::min_element(best.begin(), best.end());
+    return best;
+}
+
+// The variant with the lowest time, which goes to best_us if given.
+int fastest(std::vector<float> const& us, float* best_us)
+{
+    const auto it = std::min_element(us.begin(), us.end());
     if (best_us) *best_us = *it;
-    return static_cast<int>(it - best.begin());
+    return static_cast<int>(it - us.begin());
 }
 
 // Exclusive scan of n uint32 values into out; the total lands in
@@ -787,27 +793,27 @@ struct run_lists
 // Times every step-kernel variant on trial steps that evolve a copy of the
 // state u_cur, ping-ponging between u_other and a temporary buffer, so that
 // every launch reads what the previous one wrote (as in a solve); u_cur is
-// not modified.  launch(v, src, dst, aux) queues one step.  Returns the
-// fastest variant.
+// not modified.  launch(v, src, dst) queues one step.  Returns every
+// variant's time per step in us.
 template <typename Launch>
-int autotune_steps(ops const* op, const double* u_cur, double* u_other, uint64_t leaves, int ni, Launch&& launch,
-                   hipStream_t stream, uint32_t trials, float* best_us)
+std::vector<float> autotune_steps(ops const* op, const double* u_cur, double* u_other, uint64_t leaves, int ni,
+                                  Launch&& launch, hipStream_t stream, uint32_t trials)
 {
-    double* tmp  = dev_alloc<double>(leaves * ni);
-    int     best = 0;
+    double*            tmp = dev_alloc<double>(leaves * ni);
+    std::vector<float> us;
     try
     {
         double* bufs[2] = { tmp, u_other };
         int     p       = 0;
         AMR_HIP_CHECK(hipMemcpyAsync(tmp, u_cur, leaves * ni * sizeof(double), hipMemcpyDeviceToDevice, stream));
-        best = pick_fastest(
+        us = time_variants(
             op->variant_count(),
             [&](int v)
             {
                 launch(v, bufs[p], bufs[1 - p]);
                 p = 1 - p;
             },
-            stream, trials, best_us);
+            stream, trials);
     }
     catch (...)
     {
@@ -817,7 +823,7 @@ int autotune_steps(ops const* op, const double* u_cur, double* u_other, uint64_t
     }
     AMR_HIP_CHECK(hipStreamSynchronize(stream));
     AMR_HIP_CHECK(hipFree(tmp));
-    return best;
+    return us;
 }
 
 // Batch packing: an instance's neighbour records with their slots shifted by
@@ -1120,7 +1126,7 @@ struct amr_ctx
         ensure_usable();
         ensure_runs(-1);
         step_params prm = make_params(compute_dt());
-        variant         = autotune_steps(
+        const auto  us  = autotune_steps(
             op, u[cur], u[1 - cur], n, ni,
             [&](int v, const double* src, double* dst)
             {
@@ -1128,8 +1134,8 @@ struct amr_ctx
                 op->step(*op, v, src, dst, keys[kc], links, metas, prm, nullptr, nullptr, static_cast<uint32_t>(n),
                          runs.view(), stream);
             },
-            stream, trials, best_us);
-        return variant;
+            stream, trials);
+        return variant = fastest(us, best_us);
     }
 
     // ---- Euler (EulerPhysics<R>, amr_solver.hpp:155-413) -----------------
@@ -2880,22 +2886,23 @@ int amr_batch_autotune(amr_batch* b, uint32_t trial_steps, int32_t* chosen, floa
         [&]
         {
             if (!b) throw amr_error(AMR_ERR_ARGUMENT, "null argument");
-            // on the largest group: its trial steps meet the caches that an
-            // advance's steps meet
-            auto&    g       = **std::max_element(b->groups.begin(), b->groups.end(),
-                                                  [](auto const& x, auto const& y) { return x->leaves < y->leaves; });
-            uint32_t reverse = 0;
-            float    us      = 0.0f;
-            b->variant       = autotune_steps(
-                b->op, b->u[b->cur] + g.first * b->ni, b->u[1 - b->cur] + g.first * b->ni, g.leaves, b->ni,
-                [&](int v, const double* src, double* dst)
-                {
-                    reverse ^= 1u;
-                    b->step_group(g, v, src, dst, reverse);
-                },
-                b->stream, trial_steps, &us);
-            // per step of the whole batch
-            if (best_us && g.leaves) *best_us = us * static_cast<float>(b->total) / static_cast<float>(g.leaves);
+            // group after group, as an advance steps them: a variant's time is
+            // the sum over the groups
+            std::vector<float> us(static_cast<size_t>(b->op->variant_count()), 0.0f);
+            for (auto& g : b->groups)
+            {
+                uint32_t   reverse = 0;
+                const auto of_group = autotune_steps(
+                    b->op, b->u[b->cur] + g->first * b->ni, b->u[1 - b->cur] + g->first * b->ni, g->leaves, b->ni,
+                    [&](int v, const double* src, double* dst)
+                    {
+                        reverse ^= 1u;
+                        b->step_group(*g, v, src, dst, reverse);
+                    },
+                    b->stream, trial_steps);
+                for (size_t v = 0; v < us.size(); ++v) us[v] += of_group[v];
+            }
+            b->variant = fastest(us, best_us);
             if (chosen) *chosen = b->variant;
         }
     );

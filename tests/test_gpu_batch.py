@@ -247,3 +247,34 @@ def test_batch_of_more_trees_than_a_scatter_launch(amr):
         o.advance_batch_async(3)
         o.finish_advance_batch()
         assert np.array_equal(s.tree.get_interior().view(np.uint64), o.tree.get_interior().view(np.uint64)), k
+
+
+def test_autotune_of_a_batch_of_groups(amr):
+    """Autotuning a batch of two groups, one of them small, leaves every
+    tree's state as it was, and its time covers both."""
+    say("case: autotune of a batch of two groups")
+    solvers, states = [], []
+    rng = np.random.default_rng(9)
+    for level in (7, 7, 7, 6):  # 3 x 64 MiB, then 16 MiB that do not fit with them
+        t = amr.NdTree(2, 7, 16, 1, 1 << (2 * level))
+        solvers.append(amr.AmrSolver(t, (0.5, -1.0), 0.4))
+        for _ in range(level):
+            t.refine_all()
+        states.append(rng.standard_normal(t.size() * t.ni))
+        t.set_interior(states[-1])
+    alone = amr.Batch([s.tree for s in solvers[:1]])
+    batch = amr.Batch([s.tree for s in solvers])
+    _, one = alone.autotune(10)
+    _, us = batch.autotune(10)
+    assert us > 2 * one  # 3.25 times the leaves
+    batch.scatter()
+    for s, u in zip(solvers, states):
+        assert np.array_equal(s.tree.get_interior().reshape(-1), u)
+    batch.advance(3)
+    batch.scatter()
+    for s, u in zip(solvers, states):
+        got = s.tree.get_interior()
+        s.tree.set_interior(u)
+        s.advance_batch_async(3)
+        s.finish_advance_batch()
+        assert np.array_equal(s.tree.get_interior().view(np.uint64), got.view(np.uint64))
