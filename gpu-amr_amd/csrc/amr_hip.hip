@@ -1581,8 +1581,27 @@ struct amr_tape
     uint64_t*                  scratch_keys    = nullptr;
     regrid_summary*            scratch_summary = nullptr;
     // Recomputed states of one segment and, where adjoint and forward steps
-    // share launches (adj_pair) and there is memory, of the one before it.
+    // share launches (shares_launches), of the one before it: an allocation
+    // each, cut up.
+    double*                    seg_mem[2]{};
     std::vector<double*>       seg[2];
+
+    // Up to here a gradient keeps a second segment's states, so that a
+    // segment's recomputation shares launches with the adjoint steps of the
+    // one after it.  It fills what a small tree leaves idle (us of an adjoint
+    // pass of 100 steps of 16^2, alone -> shared: 493 leaves 733 -> 528, 1753
+    // 871 -> 696, 4096 1189 -> 1074, 7816 2143 -> 1947, 16384 3509 -> 3800 and
+    // 3806 -> 3666), and the checkpoint interval is the caller's choice of
+    // memory, which a second segment may exceed by this much at most.  A tape
+    // that passes 64 MB with it, what the runtime keeps of freed memory, takes
+    // some 0.5 ms longer to record and free.
+    static constexpr uint64_t  kShareLeaves = 8192;
+    static constexpr uint64_t  kShareBytes  = 128ull << 20;
+    bool shares_launches() const
+    {
+        return op->adj_pair && variant == 0 && ckpt_every > 1 && steps > ckpt_every && max_n <= kShareLeaves &&
+               field_bytes(max_n) <= kShareBytes / (ckpt_every - 1);
+    }
     // The launch sequence of a recorded tape is fixed (steps, regrids,
     // buffers), so the forward replay and the adjoint pass are each captured
     // once into a hipGraph and replayed; the kernels read the velocity-
@@ -1601,11 +1620,10 @@ struct amr_tape
         for (pass_graph* g : { &g_forward, &g_adjoint })
             if (g->exec) (void)hipGraphExecDestroy(g->exec);
         std::vector<void*> ptrs = { lam[0], lam[1], work, vpart, step_sums, step_leaves, chunk, acc, scratch_keys,
-                                    scratch_summary, step_tab, adj_tab };
+                                    scratch_summary, step_tab, adj_tab, seg_mem[0], seg_mem[1] };
         for (auto& t : topos) ptrs.insert(ptrs.end(), { t.keys, t.links, t.metas });
         for (auto& r : regrids) ptrs.insert(ptrs.end(), { r.mark, r.head, r.counts, r.pos });
         for (double* c : ckpts) ptrs.push_back(c);
-        for (auto& set : seg) ptrs.insert(ptrs.end(), set.begin(), set.end());
         for (void* p : ptrs)
             if (p) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
@@ -1733,19 +1751,21 @@ struct amr_tape
         for (uint64_t k = 0; k < steps; ++k) h_leaves[k] = static_cast<uint32_t>(topo(k).n);
         AMR_HIP_CHECK(hipMemcpyAsync(step_leaves, h_leaves.data(), steps * sizeof(uint32_t), hipMemcpyHostToDevice,
                                      stream));
-        for (uint64_t j = 1; j < ckpt_every; ++j) seg[0].push_back(dev_alloc<double>(max_n * ni));
-        if (op->adj_pair && variant == 0 && ckpt_every > 1 && steps > ckpt_every)
+        // one allocation a segment (us to allocate and to free: 64 MB 11 and
+        // 12, 128 MB 146 and 354, 19 of 6.7 MB 449 and 2863)
+        for (int b = 0; b < (shares_launches() ? 2 : 1); ++b)
         {
             try
             {
-                for (uint64_t j = 1; j < ckpt_every; ++j) seg[1].push_back(dev_alloc<double>(max_n * ni));
+                seg_mem[b] = dev_alloc<double>((ckpt_every - 1) * max_n * ni);
             }
-            catch (amr_error const&) // no memory for a second segment: one after the other
+            catch (amr_error const&)
             {
-                for (double* b : seg[1]) (void)hipFree(b);
-                seg[1].clear();
-                (void)hipGetLastError();
+                if (b == 0) throw;
+                (void)hipGetLastError(); // no memory for a second segment: one after the other
+                break;
             }
+            for (uint64_t j = 0; j + 1 < ckpt_every; ++j) seg[b].push_back(seg_mem[b] + j * max_n * ni);
         }
         upload_constants();
     }

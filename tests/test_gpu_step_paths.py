@@ -367,3 +367,37 @@ def test_any_shape_adjoint(amr, rank, ext):
         hi[d] += h
         fd = (image(hi) - image(lo)) / (2 * h)
         assert abs(fd - gv[d]) <= 1e-13 * scale / h, (d, fd, gv[d])
+
+
+def test_tape_memory_follows_the_checkpoint_interval(amr):
+    """A tape of a large 2D 16^2 tree holds one segment of states besides its
+    checkpoints and work buffers, and its gradient is the same bits as with
+    every state kept."""
+    import torch
+
+    say("case: tape of 16384 leaves")
+    n, steps, keep = 16384, 24, 12
+    g = amr.NdTree(2, 7, 16, 1, n)
+    s = amr.AmrSolver(g, (1.0, 0.5), 0.4)
+    for _ in range(7):
+        g.refine_all()
+    assert g.size() == n
+    x = np.random.default_rng(2).standard_normal(n * g.ni)
+    u0, lam = torch.from_numpy(x).cuda(), torch.from_numpy(x[::-1].copy()).cuda()
+    uT, grad = torch.empty_like(u0), torch.empty_like(u0)
+    results = []
+    for every in (keep, steps):
+        g.set_interior(x)
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        tape = amr.Tape(s, steps, None, 0, every)
+        used = before - torch.cuda.mem_get_info()[0]
+        state = n * g.ni * 8
+        # the segment's states, the checkpoints, lambda twice and one more state
+        assert used < (every - 1 + -(-steps // every) + 3 + 2) * state, (every, used / state)
+        tape.forward(u0.data_ptr(), (0.9, -0.4), uT.data_ptr())
+        gv = tape.adjoint(lam.data_ptr(), grad.data_ptr())
+        results.append((uT.cpu().numpy(), grad.cpu().numpy(), gv))
+        tape.close()
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
