@@ -250,31 +250,6 @@ __device__ inline void ghost_values(const double* __restrict__ u, size_t fstride
     ghost_values<R, NV>(B, u, fstride, L, meta, dir, c, out);
 }
 
-// The NV values of the cell with layout coordinates c of `leaf`: interior
-// cells from the leaf, ghost cells (one coordinate just outside) through
-// the ghost rules.
-template <int R, class BX>
-__device__ inline void euler_cell(BX const& B, const double* __restrict__ u, size_t fstride, uint32_t leaf,
-                                  const face_link* __restrict__ links, const uint32_t* __restrict__ metas, const int* c,
-                                  double* U)
-{
-    constexpr int NV = R + 2;
-    int dir = -1;
-    for (int d = 0; d < R; ++d)
-    {
-        if (c[d] < 0) dir = 2 * d;
-        if (c[d] >= B.n(d)) dir = 2 * d + 1;
-    }
-    if (dir < 0)
-    {
-        const size_t at = static_cast<size_t>(leaf) * B.ni() + B.lin(c);
-        for (int v = 0; v < NV; ++v) U[v] = u[v * fstride + at];
-        return;
-    }
-    const size_t e = static_cast<size_t>(leaf) * box<R>::NDIR + dir;
-    ghost_values<R, NV>(B, u, fstride, links[e], metas[e], dir, c, U);
-}
-
 // Every field's (n+2)^R LDS tile of `leaf` (field v at tile + v * TS): the interior cells, then the
 // face-ghost cells with one decode of the face record per ghost cell for
 // all fields.
@@ -495,19 +470,18 @@ __device__ inline void euler_step_leaf(BX const& B, const double* __restrict__ u
             total[v] = 0.0;
         }
         const auto stc = euler_flux<R>::state_of(Uc, prm.gamma);
-        for (int d = 0; d < R; ++d)
-        {
-            const int j = R - 1 - d; // layout dim of physical axis d
-            double    UL[NV], UR[NV], fL[NV], fR[NV];
-            c[j] -= 1;
-            euler_cell<R>(B, u, fstride, leaf, links, metas, c, UL);
-            c[j] += 2;
-            euler_cell<R>(B, u, fstride, leaf, links, metas, c, UR);
-            c[j] -= 1;
+        auto along = [&](auto axis) {
+            constexpr int d = decltype(axis)::value, j = R - 1 - d; // layout dim of physical axis d
+            double        UL[NV], UR[NV], fL[NV], fR[NV];
+            neighbour_values<R, NV, j, 0>(B, u, fstride, leaf, links, metas, c, UL);
+            neighbour_values<R, NV, j, 1>(B, u, fstride, leaf, links, metas, c, UR);
             euler_flux<R>::rusanov(UL, euler_flux<R>::state_of(UL, prm.gamma), Uc, stc, fL, d);
             euler_flux<R>::rusanov(Uc, stc, UR, euler_flux<R>::state_of(UR, prm.gamma), fR, d);
             for (int k = 0; k < NV; ++k) total[k] -= dtdx[d] * (fR[k] - fL[k]);
-        }
+        };
+        along(std::integral_constant<int, 0>{});
+        along(std::integral_constant<int, 1>{});
+        if constexpr (R == 3) along(std::integral_constant<int, 2>{});
         double o[NV];
         for (int v = 0; v < NV; ++v)
         {
@@ -533,7 +507,11 @@ __global__ __launch_bounds__(NT) void k_euler_step(const double* __restrict__ u,
     euler_step_leaf<R, NT>(B, u, un, fstride, keys, links, metas, prm, sc, dt, leaf);
 }
 
-// k_euler_step for patches of any shape.
+// k_euler_step for patches of any shape (those that k_euler_step_layers does
+// not take).  Bound by the latency of the neighbours' loads: us per step on
+// adapted trees, a ghost's fine cells one by one -> together
+// (neighbour_values), 155 leaves of 20^3 256 -> 154, of 10x16x32 161 -> 97,
+// 1387 of 4x24x24 194 -> 149.
 template <int R, int NT>
 __global__ __launch_bounds__(NT) void k_euler_step_box(const double* __restrict__ u, double* __restrict__ un,
                                                        size_t fstride, const uint64_t* __restrict__ keys,

@@ -594,30 +594,6 @@ __host__ __device__ inline double padded_value(const double* __restrict__ u, uin
     return padded_value<R>(B, H, u, leaf, links, metas, i, kind);
 }
 
-// The upwind update of interior cell i of `leaf` with its neighbours read
-// from memory (interior cells, or ghost values at the patch boundary): the
-// same operands as upwind_cell on a staged tile, for patches of any shape.
-template <int R, class BX>
-__host__ __device__ inline double upwind_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
-                                                     const face_link* __restrict__ links,
-                                                     const uint32_t* __restrict__ metas, int i, const double* dtdx,
-                                                     const double* vel, const double* hs)
-{
-    int c[R];
-    B.coords(i, c);
-    double lo[R], hi[R];
-    for (int d = 0; d < R; ++d)
-    {
-        const int j = R - 1 - d; // layout dim of physical axis d
-        c[j] -= 1;
-        lo[d] = cell_or_ghost<R>(B, u, leaf, links, metas, c);
-        c[j] += 2;
-        hi[d] = cell_or_ghost<R>(B, u, leaf, links, metas, c);
-        c[j] -= 1;
-    }
-    return upwind_update<R>(u[static_cast<size_t>(leaf) * B.ni() + i], lo, hi, dtdx, vel, hs);
-}
-
 // gradient_cell with the neighbours read from memory (any patch shape).
 template <int R, class BX>
 __host__ __device__ inline double gradient_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
@@ -729,7 +705,7 @@ __host__ __device__ inline size_t face_source(BX const& B, int32_t nb, uint32_t 
 // finer neighbours ids (a vector, whose elements a select picks: an array
 // indexed by a lane's value would live in scratch memory).
 template <int R, int D, class BX>
-__device__ inline size_t face_fine_source(BX const& B, int4 ids, int side, const int* c)
+__host__ __device__ inline size_t face_fine_source(BX const& B, int4 ids, int side, const int* c)
 {
     int k = 0, bit = 0, cc[R];
     for (int d = 0; d < R; ++d)
@@ -746,7 +722,7 @@ __device__ inline size_t face_fine_source(BX const& B, int4 ids, int side, const
     return static_cast<size_t>(nb) * B.ni() + B.lin(cc);
 }
 
-__device__ inline int4 link_ids(const face_link* __restrict__ L) { return *reinterpret_cast<const int4*>(L); }
+__host__ __device__ inline int4 link_ids(const face_link* __restrict__ L) { return *reinterpret_cast<const int4*>(L); }
 
 // Offset of the o-th of those cells (row-major) from the first.
 template <int R, class BX>
@@ -780,6 +756,84 @@ __device__ inline void face_values(BX const& B, const double* __restrict__ u, si
         for (int v = 0; v < NV; ++v) sum[v] += u[v * fstride + first + fine_offset<R>(B, o)];
 #pragma unroll
     for (int v = 0; v < NV; ++v) out[v] = sum[v] / static_cast<double>(1 << R);
+}
+
+// The NV values (fields fstride apart) of the cell before (SIDE 0) or after
+// (SIDE 1) cell c of `leaf` along layout dim D: a cell of the patch or, past
+// its last one, the face's ghost.
+template <int R, int NV, int D, int SIDE, class BX>
+__host__ __device__ inline void neighbour_values(BX const& B, const double* __restrict__ u, size_t fstride,
+                                                 uint32_t leaf, const face_link* __restrict__ links,
+                                                 const uint32_t* __restrict__ metas, const int* c, double* out)
+{
+    if (SIDE ? c[D] + 1 < B.n(D) : c[D] > 0)
+    {
+        const size_t at = static_cast<size_t>(leaf) * B.ni() + (B.lin(c) + (SIDE ? B.stride(D) : -B.stride(D)));
+#pragma unroll
+        for (int v = 0; v < NV; ++v) out[v] = u[v * fstride + at];
+        return;
+    }
+    int g[R];
+    for (int d = 0; d < R; ++d) g[d] = c[d];
+    g[D]                = SIDE ? B.n(D) : -1;
+    const size_t   e    = static_cast<size_t>(leaf) * box<R>::NDIR + (2 * D + SIDE);
+    const uint32_t meta = metas[e];
+    const int4     L    = link_ids(links + e);
+    if (rel_of(meta) != REL_FINER)
+    {
+        const size_t at = face_source<R, D>(B, L.x, meta, SIDE, g);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) out[v] = u[v * fstride + at];
+        return;
+    }
+    // face_values' sums, the cells up to 20 at a time in flight: left to
+    // itself the compiler keeps registers by waiting for them one by one
+    constexpr int F = 1 << R, BATCH = NV * F <= 20 ? F : F / 2;
+    const size_t  first = face_fine_source<R, D>(B, L, SIDE, g);
+    double        sum[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) sum[v] = 0.0;
+#pragma unroll
+    for (int o0 = 0; o0 < F; o0 += BATCH)
+    {
+        double f[BATCH][NV];
+#pragma unroll
+        for (int o = 0; o < BATCH; ++o)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) f[o][v] = u[v * fstride + first + fine_offset<R>(B, o0 + o)];
+#ifdef __HIP_DEVICE_COMPILE__
+        __builtin_amdgcn_sched_barrier(0);
+#endif
+#pragma unroll
+        for (int o = 0; o < BATCH; ++o)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) sum[v] += f[o][v];
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) out[v] = sum[v] / static_cast<double>(F);
+}
+
+// The upwind update of interior cell i of `leaf` with its neighbours read
+// from memory (interior cells, or ghost values at the patch boundary): the
+// same operands as upwind_cell on a staged tile, for patches of any shape.
+template <int R, class BX>
+__host__ __device__ inline double upwind_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
+                                                     const face_link* __restrict__ links,
+                                                     const uint32_t* __restrict__ metas, int i, const double* dtdx,
+                                                     const double* vel, const double* hs)
+{
+    int c[R];
+    B.coords(i, c);
+    double lo[R], hi[R];
+    auto   along = [&](auto dim) {
+        constexpr int J = decltype(dim)::value; // layout dim of physical axis R - 1 - J
+        neighbour_values<R, 1, J, 0>(B, u, 0, leaf, links, metas, c, &lo[R - 1 - J]);
+        neighbour_values<R, 1, J, 1>(B, u, 0, leaf, links, metas, c, &hi[R - 1 - J]);
+    };
+    along(std::integral_constant<int, 0>{});
+    along(std::integral_constant<int, 1>{});
+    if constexpr (R == 3) along(std::integral_constant<int, 2>{});
+    return upwind_update<R>(u[static_cast<size_t>(leaf) * B.ni() + i], lo, hi, dtdx, vel, hs);
 }
 
 // How a workgroup of NT threads walks the cells of a patch: `layers` layers of
@@ -1476,7 +1530,11 @@ __global__ __launch_bounds__(NT) void k_step_box_tile(const double* __restrict__
                           upwind_tile_cell<R>(box_lds, T, col.t0 + k * col.dt, C.dtdx, C.vel, C.hs));
 }
 
-// Patches whose tile does not fit: neighbours from memory.
+// Patches whose tile does not fit: neighbours from memory, each through its
+// own dim's rule (neighbour_values), the fine cells of a ghost in flight
+// together.  Bound by the latency of those loads: us per step on adapted
+// trees, with one rule for every side -> by dim, 103 leaves of 90x88 53.2 ->
+// 37.9, 155 of 20^3 91.3 -> 59.6, 1387 of 4x24x24 50.0 -> 33.2.
 template <int R, int NT, int FROM>
 __global__ __launch_bounds__(NT) void k_step_box(const double* __restrict__ u, double* __restrict__ un,
                                                  const uint64_t* __restrict__ keys,
