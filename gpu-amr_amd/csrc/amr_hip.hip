@@ -159,13 +159,16 @@ constexpr size_t kBoxTileBytes = 64 * 1024; // largest LDS tile of the any-shape
 //  - at most 16 layers each,
 //  - a wave per SIMD (a chain of layers is latency: 32^2, 130 leaves, strips
 //    of 16 / 4 layers 19.4 / 14.7 us; 523 leaves 25.9 / 23.4; 1945 leaves
-//    42.5 / 44.5),
+//    42.5 / 44.5), but no shorter than four layers, or half a patch of fewer
+//    than eight (64 leaves of 6^3, six / three layers 20.7 / 15.3 us; of 4x6x8
+//    four / two 15 leaves 14.8 / 10.7, 155 16.8 / 13.5; of 4x48 103 leaves
+//    11.2 / 8.5; 7 of 2x128, two / one 9.4 / 7.3): a strip forms the states of
+//    one layer below and one above its own,
 //  - LDS for four (2D) or three (3D) waves per SIMD, what the registers allow
-//    (12^3, 1583 leaves, strips of 12 / 6 layers 126 / 92 us),
-// but not under four layers (three of patches with fewer than eight: 64 leaves
-// of 6^3, six / three layers 20.7 / 15.3 us) for these: a strip forms the states of one
-// layer below and one above its own.  0 where a layer has more than 512 cells or
-// its strip exceeds 64 KiB of LDS.
+//    (12^3, 1583 leaves, strips of 12 / 6 layers 126 / 92 us), but no shorter
+//    than four layers, or three of a patch of fewer than eight (11299 leaves
+//    of 4x8x8, four / two layers 94.5 / 103.9 us).
+// 0 where a layer has more than 512 cells or its strip exceeds 64 KiB of LDS.
 template <int R>
 int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
 {
@@ -180,17 +183,20 @@ int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
     const int    side_by_side = std::min(nt / cols, static_cast<int>(o.ext[0]));
     const size_t per_wave     = (160 * 1024 / 4) / (R == 2 ? 4 : 3);
     size_t       lds          = 0;
+    bool         waves        = false; // a wave per SIMD
     for (int g = 1;; ++g)
     {
         const int layers = (o.ext[0] + side_by_side * g - 1) / (side_by_side * g);
-        if (g > 1 && layers < (o.ext[0] < 8 ? 3 : 4)) break;
+        const int least  = waves ? (o.ext[0] < 8 ? 3 : 4) : std::min<int>(o.ext[0] / 2, 4);
+        if (g > 1 && (layers < least || W.layers == 1)) break;
         if (g > 1 && layers == W.layers) continue;
         const int strips = (o.ext[0] + layers - 1) / layers;
         W.layers         = layers;
         W.segs           = std::min(side_by_side, strips);
         W.groups         = static_cast<uint32_t>((strips + W.segs - 1) / W.segs);
         lds              = static_cast<size_t>(euler_layer_lds<R>(B, W)) * sizeof(double);
-        if (layers <= 16 && static_cast<uint64_t>(n) * W.groups * (nt / 64) >= 1024 && lds <= per_wave * (nt / 64)) break;
+        waves            = static_cast<uint64_t>(n) * W.groups * (nt / 64) >= 1024;
+        if (layers <= 16 && waves && lds <= per_wave * (nt / 64)) break;
     }
     W.group_quot = W.groups > 1 ? static_cast<uint32_t>(((uint64_t{ 1 } << 32) + W.groups - 1) / W.groups) : 0u;
     const bool divides = (static_cast<uint64_t>(n) * W.groups + kXcds) * W.groups < (uint64_t{ 1 } << 32);
