@@ -151,58 +151,6 @@ void for_source(const step_params* table, const uint32_t* inst, Fn&& f)
         f(std::integral_constant<int, PER_LEAF>{});
 }
 
-constexpr size_t kBoxTileBytes = 64 * 1024; // largest LDS tile of the any-shape kernels
-
-// The split of a leaf for k_euler_step_layers and its workgroup size: the
-// smallest workgroup that holds a layer, with as many strips side by side as
-// fit in it, and the fewest, hence longest, strips with
-//  - at most 16 layers each,
-//  - a wave per SIMD (a chain of layers is latency: 32^2, 130 leaves, strips
-//    of 16 / 4 layers 19.4 / 14.7 us; 523 leaves 25.9 / 23.4; 1945 leaves
-//    42.5 / 44.5), but no shorter than four layers, or half a patch of fewer
-//    than eight (64 leaves of 6^3, six / three layers 20.7 / 15.3 us; of 4x6x8
-//    four / two 15 leaves 14.8 / 10.7, 155 16.8 / 13.5; of 4x48 103 leaves
-//    11.2 / 8.5; 7 of 2x128, two / one 9.4 / 7.3): a strip forms the states of
-//    one layer below and one above its own,
-//  - LDS for four (2D) or three (3D) waves per SIMD, what the registers allow
-//    (12^3, 1583 leaves, strips of 12 / 6 layers 126 / 92 us), but no shorter
-//    than four layers, or three of a patch of fewer than eight (11299 leaves
-//    of 4x8x8, four / two layers 94.5 / 103.9 us).
-// 0 where a layer has more than 512 cells or its strip exceeds 64 KiB of LDS.
-template <int R>
-int euler_walk_for(ops const& o, uint32_t n, euler_walk& W)
-{
-    const launch_box<R> B    = launch_box<R>::of(o.ext);
-    const int           cols = B.face(0);
-    int                 nt   = 0;
-    for (int t : { 64, 128, 192, 256, 512 })
-        if (!nt && cols <= t) nt = t;
-    if (!nt) return 0;
-    for (int d = 1; d < R; ++d)
-        if (!B.m[d]) return 0; // too large for the divisions by multiplication
-    const int    side_by_side = std::min(nt / cols, static_cast<int>(o.ext[0]));
-    const size_t per_wave     = (160 * 1024 / 4) / (R == 2 ? 4 : 3);
-    size_t       lds          = 0;
-    bool         waves        = false; // a wave per SIMD
-    for (int g = 1;; ++g)
-    {
-        const int layers = (o.ext[0] + side_by_side * g - 1) / (side_by_side * g);
-        const int least  = waves ? (o.ext[0] < 8 ? 3 : 4) : std::min<int>(o.ext[0] / 2, 4);
-        if (g > 1 && (layers < least || W.layers == 1)) break;
-        if (g > 1 && layers == W.layers) continue;
-        const int strips = (o.ext[0] + layers - 1) / layers;
-        W.layers         = layers;
-        W.segs           = std::min(side_by_side, strips);
-        W.groups         = static_cast<uint32_t>((strips + W.segs - 1) / W.segs);
-        lds              = static_cast<size_t>(euler_layer_lds<R>(B, W)) * sizeof(double);
-        waves            = static_cast<uint64_t>(n) * W.groups * (nt / 64) >= 1024;
-        if (layers <= 16 && waves && lds <= per_wave * (nt / 64)) break;
-    }
-    W.group_quot = W.groups > 1 ? static_cast<uint32_t>(((uint64_t{ 1 } << 32) + W.groups - 1) / W.groups) : 0u;
-    const bool divides = (static_cast<uint64_t>(n) * W.groups + kXcds) * W.groups < (uint64_t{ 1 } << 32);
-    return divides && lds <= kBoxTileBytes ? nt : 0;
-}
-
 // One Euler step by k_euler_step_layers; false where the shape does not fit.
 template <int R>
 bool launch_euler_layers(ops const& o, const double* u, double* un, size_t fs, const uint64_t* keys,
@@ -210,7 +158,7 @@ bool launch_euler_layers(ops const& o, const double* u, double* un, size_t fs, c
                          uint32_t reverse, uint32_t n, hipStream_t s)
 {
     euler_walk W{};
-    const int  nt = euler_walk_for<R>(o, n, W);
+    const int  nt = euler_walk_for<R>(o.ext, n, W);
     auto       go = [&](auto threads) {
         constexpr int             NT    = decltype(threads)::value;
         const launch_box<R, true> B     = launch_box<R, true>::of(o.ext);
@@ -482,27 +430,6 @@ struct box_instance
     static char const* variant_name(int) { return "box"; }
     static int         variant_needs(int) { return 0; }
 
-    // The walk of a patch (box_walk) and its workgroup size: the one of 64,
-    // 128, 256 (512 from 2048 cells on) threads that spends the fewest thread
-    // slots in at most four passes, the smaller one of equals, else the
-    // largest.  0 when a layer has more cells than the largest workgroup.
-    static int walk_for(ops const& o, box_walk& W)
-    {
-        const int cols = o.ni() / o.ext[0], most = o.ni() >= 2048 ? 512 : 256;
-        int       best = 0, slots = 0;
-        for (int nt = 64; nt <= most; nt *= 2)
-        {
-            if (cols > nt) continue;
-            const int layers = std::min(nt / cols, static_cast<int>(o.ext[0]));
-            const int passes = (o.ext[0] + layers - 1) / layers;
-            if (best && (passes * nt >= slots) && !(W.passes > 4)) continue;
-            best  = nt;
-            slots = passes * nt;
-            W     = box_walk{ layers, passes };
-        }
-        return best;
-    }
-
     // LDS of one tile of nv fields
     static size_t tile_bytes(ops const& o, int nv)
     {
@@ -517,7 +444,7 @@ struct box_instance
         const dim3   grid(xcd_grid(n));
         const size_t lds = tile_bytes(o, 1);
         box_walk     W;
-        const int    nt  = lds <= kBoxTileBytes ? walk_for(o, W) : 0;
+        const int    nt  = lds <= kBoxTileBytes ? box_walk_for<R>(shape(o), W) : 0;
         for_source(table, inst, [&](auto source) {
             constexpr int FROM = decltype(source)::value;
             auto          go   = [&](auto threads) {

@@ -969,7 +969,7 @@ __global__ __launch_bounds__(NT) void k_adj_step_box_tile(const double* __restri
 {
     constexpr int NW = NT / 64;
     __shared__ double red[R][NW];
-    extern __shared__ double lds[];
+    HIP_DYNAMIC_SHARED(double, lds)
     const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
     const adjoint_params& prm = *prm_p;

@@ -590,6 +590,56 @@ __host__ __device__ inline int euler_layer_lds(BX const& B, euler_walk const& W)
     return euler_cell_slot<R> * (euler_layer_cells<R>(B, W) + euler_side_cells<R>(B, W)) + ((R + 2) | 1) * euler_layer_cells<R>(B, W);
 }
 
+// The split of a leaf for k_euler_step_layers and its workgroup size: the
+// smallest workgroup that holds a layer, with as many strips side by side as
+// fit in it, and the fewest, hence longest, strips with
+//  - at most 16 layers each,
+//  - a wave per SIMD (a chain of layers is latency: 32^2, 130 leaves, strips
+//    of 16 / 4 layers 19.4 / 14.7 us; 523 leaves 25.9 / 23.4; 1945 leaves
+//    42.5 / 44.5), but no shorter than four layers, or half a patch of fewer
+//    than eight (64 leaves of 6^3, six / three layers 20.7 / 15.3 us; of 4x6x8
+//    four / two 15 leaves 14.8 / 10.7, 155 16.8 / 13.5; of 4x48 103 leaves
+//    11.2 / 8.5; 7 of 2x128, two / one 9.4 / 7.3): a strip forms the states of
+//    one layer below and one above its own,
+//  - LDS for four (2D) or three (3D) waves per SIMD, what the registers allow
+//    (12^3, 1583 leaves, strips of 12 / 6 layers 126 / 92 us), but no shorter
+//    than four layers, or three of a patch of fewer than eight (11299 leaves
+//    of 4x8x8, four / two layers 94.5 / 103.9 us).
+// 0 where a layer has more than 512 cells or its strip exceeds 64 KiB of LDS.
+template <int R>
+int euler_walk_for(const int32_t* ext, uint32_t n, euler_walk& W)
+{
+    const launch_box<R> B    = launch_box<R>::of(ext);
+    const int           cols = B.face(0);
+    int                 nt   = 0;
+    for (int t : { 64, 128, 192, 256, 512 })
+        if (!nt && cols <= t) nt = t;
+    if (!nt) return 0;
+    for (int d = 1; d < R; ++d)
+        if (!B.m[d]) return 0; // too large for the divisions by multiplication
+    const int    side_by_side = ext[0] < nt / cols ? ext[0] : nt / cols;
+    const size_t per_wave     = (160 * 1024 / 4) / (R == 2 ? 4 : 3);
+    size_t       lds          = 0;
+    bool         waves        = false; // a wave per SIMD
+    for (int g = 1;; ++g)
+    {
+        const int layers = (ext[0] + side_by_side * g - 1) / (side_by_side * g);
+        const int least  = waves ? (ext[0] < 8 ? 3 : 4) : (ext[0] < 8 ? ext[0] / 2 : 4);
+        if (g > 1 && (layers < least || W.layers == 1)) break;
+        if (g > 1 && layers == W.layers) continue;
+        const int strips = (ext[0] + layers - 1) / layers;
+        W.layers         = layers;
+        W.segs           = strips < side_by_side ? strips : side_by_side;
+        W.groups         = static_cast<uint32_t>((strips + W.segs - 1) / W.segs);
+        lds              = static_cast<size_t>(euler_layer_lds<R>(B, W)) * sizeof(double);
+        waves            = static_cast<uint64_t>(n) * W.groups * (nt / 64) >= 1024;
+        if (layers <= 16 && waves && lds <= per_wave * (nt / 64)) break;
+    }
+    W.group_quot = W.groups > 1 ? static_cast<uint32_t>(((uint64_t{ 1 } << 32) + W.groups - 1) / W.groups) : 0u;
+    const bool divides = (static_cast<uint64_t>(n) * W.groups + kXcds) * W.groups < (uint64_t{ 1 } << 32);
+    return divides && lds <= kBoxTileBytes ? nt : 0;
+}
+
 // Euler step of patches of any shape whose layers (cells of one coordinate of
 // layout dim 0) fit a workgroup.  A strip of layers is walked along dim 0,
 // each thread keeping its column: the state of a cell is formed once, the
@@ -614,7 +664,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 :
 {
     constexpr int NV = R + 2;
     using EF         = euler_flux<R>;
-    extern __shared__ double lds[];
+    HIP_DYNAMIC_SHARED(double, lds)
     const uint32_t item = sweep_item(blockIdx.x, walk);
     const double   dt   = euler_step_dt(prm, sc);
     const uint32_t leaf = W.group_quot ? static_cast<uint32_t>((static_cast<uint64_t>(item) * W.group_quot) >> 32) : item;

@@ -7,8 +7,9 @@
 // from the neighbours' interiors through the device neighbour table, with the
 // reference's same / finer (mean) / coarser (injection) rules, into LDS.
 //
-// Every per-item body is __host__ __device__; the __global__ kernels only
-// distribute items over threads, so the same bodies can be run on the CPU.
+// Bodies that work on one item alone are __host__ __device__, so that they run
+// on the CPU item by item; kernels whose lanes share LDS or registers run there
+// as a whole, a launch lane by lane (the tests do both).
 #pragma once
 
 #include "device_common.hpp"
@@ -642,6 +643,8 @@ __device__ inline void stage_tile(double* tile, const double* __restrict__ u, ui
 // LDS tiles of patches whose extents are launch arguments: the patch plus one
 // ghost layer, (n(d) + 2) cells per dim, row-major.
 // ---------------------------------------------------------------------------
+constexpr size_t kBoxTileBytes = 64 * 1024; // largest of them
+
 template <int R>
 struct box_tile
 {
@@ -844,6 +847,28 @@ struct box_walk
 {
     int32_t layers, passes;
 };
+
+// The walk of a patch (box_walk) and its workgroup size: the one of 64,
+// 128, 256 (512 from 2048 cells on) threads that spends the fewest thread
+// slots in at most four passes, the smaller one of equals, else the
+// largest.  0 when a layer has more cells than the largest workgroup.
+template <int R>
+int box_walk_for(box<R> const& B, box_walk& W)
+{
+    const int cols = B.face(0), most = B.ni() >= 2048 ? 512 : 256;
+    int       best = 0, slots = 0;
+    for (int nt = 64; nt <= most; nt *= 2)
+    {
+        if (cols > nt) continue;
+        const int layers = B.n(0) < nt / cols ? B.n(0) : nt / cols;
+        const int passes = (B.n(0) + layers - 1) / layers;
+        if (best && (passes * nt >= slots) && !(W.passes > 4)) continue;
+        best  = nt;
+        slots = passes * nt;
+        W     = box_walk{ layers, passes };
+    }
+    return best;
+}
 
 // One thread's walk: active while k < passes and cell(k) is in the patch.
 template <int R>
@@ -1513,7 +1538,7 @@ __global__ __launch_bounds__(NT) void k_step_box_tile(const double* __restrict__
                                                       const uint32_t* __restrict__ metas, uint32_t nleaves, uint32_t walk, launch_box<R, true> B, box_walk W, step_params prm,
     const step_params* __restrict__ table, const uint32_t* __restrict__ inst)
 {
-    extern __shared__ double box_lds[];
+    HIP_DYNAMIC_SHARED(double, box_lds)
     const uint32_t leaf = sweep_item(blockIdx.x, walk);
     if (leaf >= nleaves) return;
     const uint32_t      who = leaf_instance<FROM>(inst, leaf);

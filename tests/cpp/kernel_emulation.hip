@@ -6,6 +6,7 @@
 #include "kernels_step.hpp"
 #include "kernels_tree.hpp"
 #include "kernels_adjoint.hpp"
+#include "kernels_euler.hpp"
 #include "kernels_fused.hpp"
 
 #include <algorithm>
@@ -585,6 +586,33 @@ int emu_adj_regrid_box(int rank, const int* ext, const double* lam_new, const ui
         adj_regrid_box<2>(ext, lam_new, maps, n_old, lam_old);
     else
         adj_regrid_box<3>(ext, lam_new, maps, n_old, lam_old);
+    return 0;
+}
+
+// The walks that the any-shape kernels take: out = layers, passes of a step and
+// its workgroup size; segs, layers, groups of an Euler step, its workgroup size
+// and bytes of LDS.
+int emu_walks(int rank, const int* ext, uint32_t n, int64_t* out)
+{
+    box_walk   S{};
+    euler_walk W{};
+    int        ns, ne, lds;
+    if (rank == 2)
+    {
+        const box<2> B = box_of<2>(ext);
+        ns             = box_walk_for<2>(B, S);
+        ne             = euler_walk_for<2>(B.e, n, W);
+        lds            = ne ? euler_layer_lds<2>(B, W) : 0;
+    }
+    else
+    {
+        const box<3> B = box_of<3>(ext);
+        ns             = box_walk_for<3>(B, S);
+        ne             = euler_walk_for<3>(B.e, n, W);
+        lds            = ne ? euler_layer_lds<3>(B, W) : 0;
+    }
+    const int64_t r[] = { S.layers, S.passes, ns, W.segs, W.layers, W.groups, ne, static_cast<int64_t>(lds) * 8 };
+    std::copy(std::begin(r), std::end(r), out);
     return 0;
 }
 

@@ -240,3 +240,11 @@ def batch_groups(sizes, most):
     fn.restype = ctypes.c_uint32
     count = fn(_p(sizes), ctypes.c_uint64(sizes.size), ctypes.c_uint64(int(most)), _p(first))
     return first[:count].astype(int).tolist()
+
+
+def walks(rank, ext, n):
+    """((layers, passes, threads) of an any-shape step, (segs, layers, groups,
+    threads, bytes of LDS) of an Euler step) for a tree of n leaves."""
+    out = np.zeros(8, dtype=np.int64)
+    load().emu_walks(rank, _ext(ext), ctypes.c_uint32(n), _p(out))
+    return tuple(out[:3].tolist()), tuple(out[3:].tolist())
