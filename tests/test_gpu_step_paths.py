@@ -401,3 +401,34 @@ def test_tape_memory_follows_the_checkpoint_interval(amr):
         tape.close()
     for a, b in zip(*results):
         assert np.array_equal(a, b)
+
+
+def test_euler_walk_16_adapted(amr):
+    """16^2 patches above the leaf count from which a wave walks a leaf, with
+    finer and coarser faces: a step against numpy, then a batch (which folds
+    each next dt) against single steps."""
+    say("case: Euler 16^2, 4102 leaves on two levels")
+    made = []
+    for _ in range(2):
+        s = amr.EulerSolver(2, 7, 16, 1, 4200, (1.0, 1.0), 1.4, 0.3)
+        t = s.tree
+        for _ in range(6):
+            t.refine_all()
+        flags = np.zeros(t.size(), dtype=np.int8)
+        flags[[0, 2741]] = amr.REFINE
+        assert t.reconstruct_tree(flags) and t.size() == 4102
+        rng = np.random.default_rng(16)
+        u0 = np.empty((4, t.size() * t.ni))
+        u0[0], u0[1:3], u0[3] = rng.uniform(0.5, 1.5, u0.shape[1]), rng.uniform(-0.5, 0.5, u0[1:3].shape), 3.0
+        t.set_interior(u0)
+        made.append(s)
+    single, batch = made
+    with np.errstate(all="ignore"):  # the corners of the padded patches are 0
+        exp = euler_step_of_padded(single.tree, 1.4, single.compute_dt())
+    time = single.advance()
+    assert_fields(single.tree.get_interior(), exp, "one step")
+    for _ in range(2):
+        time += single.advance()
+    batch.advance_batch_async(3)
+    assert batch.finish_advance_batch() == (time, 3)
+    assert_fields(batch.tree.get_interior(), single.tree.get_interior(), "batch of three")
