@@ -330,11 +330,14 @@ __host__ __device__ inline double restrict_value(const double* __restrict__ u, u
 // Trees of up to this many leaves: the table's binary searches and the
 // regrid's planning passes run on copies of the keys in LDS (32 KB).  Both are
 // chains of dependent reads, about ten per search, that cost an L2 round trip
-// each.  us a launch within adaptive solves on about 300 leaves of 16^2 / 700
-// of 64^2, before -> after (Morton arithmetic, records read together, the
-// deepest level formed by the plan instead of an atomic per emitted leaf):
-// table 4.9 -> 3.5 / 3.2 -> 2.8, planning 7.0 -> 6.6 / 7.1 -> 7.7 (bound by
-// one workgroup's barriers and integer work, LDS or not), emit 4.4 -> 3.3.
+// each.  us a launch, keys in memory and taken apart bit by bit -> in LDS and
+// Morton arithmetic (records read together, the deepest level formed by the
+// plan instead of an atomic per emitted leaf).  Planning: 256 leaves of 16^2,
+// some refined, 5.5 -> 4.4, their 364 coarsened back 10.6 -> 6.1; 512 of 8^3
+// 7.8 -> 6.2, their 981 back 32.6 -> 14.1; 4096 of 4^3 29.4 -> 13.0; nothing to
+// do on 319 of 16^2 4.5 -> 3.6, on 876 of 8^3 7.0 -> 4.6 (the 210 scalar
+// registers that the 3D plan spills are lanes of vector registers).  Table: 364
+// leaves of 16^2 8.4 -> 5.8, 981 of 8^3 13.5 -> 8.4.  Emit: 6.9 -> 4.4, 12.8 -> 7.7.
 constexpr uint32_t kLdsKeys = 4096;
 
 template <int R, bool SMALL>
@@ -574,7 +577,10 @@ __global__ __launch_bounds__(kPlanThreads) void k_regrid_plan(
     if (n_refine) atomicAdd(&sums[0], n_refine);
     if (n_coarsen) atomicAdd(&sums[1], n_coarsen);
     if (root_any) atomicOr(&sums[2], 2u);
-    if (deepest) atomicMax(&sums[3], deepest);
+    // the wave's deepest level, bit by bit: an atomic per leaf would queue up
+    uint32_t top = 0;
+    for (uint32_t bit = 16; bit > 0; bit >>= 1) top += __any(deepest >= top + bit) ? bit : 0u;
+    if (top && (t & 63u) == 0u) atomicMax(&sums[3], top);
     __syncthreads();
     if (t == 0) *summary = regrid_summary{ total, sums[0], sums[1], sums[2], sums[3], {} };
 }
