@@ -595,28 +595,6 @@ __host__ __device__ inline double padded_value(const double* __restrict__ u, uin
     return padded_value<R>(B, H, u, leaf, links, metas, i, kind);
 }
 
-// gradient_cell with the neighbours read from memory (any patch shape).
-template <int R, class BX>
-__host__ __device__ inline double gradient_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
-                                                       const face_link* __restrict__ links,
-                                                       const uint32_t* __restrict__ metas, int i)
-{
-    int c[R];
-    B.coords(i, c);
-    const double uc = u[static_cast<size_t>(leaf) * B.ni() + i];
-    double       g  = 0.0;
-    for (int j = 0; j < R; ++j)
-    {
-        c[j] += 1;
-        const double up = cell_or_ghost<R>(B, u, leaf, links, metas, c);
-        c[j] -= 2;
-        const double um = cell_or_ghost<R>(B, u, leaf, links, metas, c);
-        c[j] += 1;
-        g = fmax(g, fmax(fabs(up - uc), fabs(uc - um)));
-    }
-    return g;
-}
-
 __host__ __device__ inline int8_t decide(double value, int level, double rthr, double cthr, int min_level,
                                          int max_level)
 {
@@ -837,6 +815,29 @@ __host__ __device__ inline double upwind_cell_direct(BX const& B, const double* 
     along(std::integral_constant<int, 1>{});
     if constexpr (R == 3) along(std::integral_constant<int, 2>{});
     return upwind_update<R>(u[static_cast<size_t>(leaf) * B.ni() + i], lo, hi, dtdx, vel, hs);
+}
+
+// gradient_cell with the neighbours read from memory (any patch shape).
+template <int R, class BX>
+__host__ __device__ inline double gradient_cell_direct(BX const& B, const double* __restrict__ u, uint32_t leaf,
+                                                       const face_link* __restrict__ links,
+                                                       const uint32_t* __restrict__ metas, int i)
+{
+    int c[R];
+    B.coords(i, c);
+    const double uc = u[static_cast<size_t>(leaf) * B.ni() + i];
+    double       g  = 0.0;
+    auto         along = [&](auto dim) {
+        constexpr int J = decltype(dim)::value;
+        double        um, up;
+        neighbour_values<R, 1, J, 0>(B, u, 0, leaf, links, metas, c, &um);
+        neighbour_values<R, 1, J, 1>(B, u, 0, leaf, links, metas, c, &up);
+        g = fmax(g, fmax(fabs(up - uc), fabs(uc - um)));
+    };
+    along(std::integral_constant<int, 0>{});
+    along(std::integral_constant<int, 1>{});
+    if constexpr (R == 3) along(std::integral_constant<int, 2>{});
+    return g;
 }
 
 // How a workgroup of NT threads walks the cells of a patch: `layers` layers of
