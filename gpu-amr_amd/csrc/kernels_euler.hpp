@@ -650,12 +650,15 @@ int euler_walk_for(const int32_t* ext, uint32_t n, euler_walk& W)
 // the same bits.  Bound by FP64 issue and latency as they are (k_euler_step_box
 // formed 2 R + 1 states and 2 R fluxes per cell and read every neighbour from
 // memory).  us per step on adapted trees, from memory -> by layers: 1945
-// leaves of 32^2 64 -> 43 (32 MB read and written once: 9.2 at the copy
+// leaves of 32^2 64 -> 43 (64 MB read and written once: 18.3 at the copy
 // rate), 523 29 -> 22.5, 484 of 48^2 49 -> 36, 1583 of 6^3 35 -> 31, of
 // 12^3 158 -> 91, of 16^3 439 -> 204.  Cells one after another in LDS, the
 // leaf's fields by uniform pointers: with fields one after another in both,
 // the addresses alone took some 60 registers and 3D spilled (12^3: 192).  Five
-// (2D) or four (3D) waves per SIMD spill: 49 and 212.
+// (2D) or four (3D) waves per SIMD spill: 49 and 212.  In 3D dt / dx are in
+// scalar registers: in vector registers three waves spill six of them (1387
+// leaves of 12^3 84.4 -> 79.8 us, of 16^3 176 -> 163, of 6^3 23.4 -> 22.2; 2D
+// has registers to spare and does not change).
 template <int R, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 : 3))) void k_euler_step_layers(
     const double* __restrict__ u, double* __restrict__ un, size_t fstride, const uint64_t* __restrict__ keys,
@@ -717,7 +720,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 :
     double dtdx[R], smax[R];
     for (int d = 0; d < R; ++d)
     {
-        dtdx[d] = dt / prm.cs[lv][d];
+        dtdx[d] = R == 3 ? wave_uniform(dt / prm.cs[lv][d]) : dt / prm.cs[lv][d];
         smax[d] = 0.0;
     }
     constexpr int ST = euler_cell_slot<R>, TOP = NV | 1;
