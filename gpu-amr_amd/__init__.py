@@ -489,8 +489,9 @@ class EulerSolver:
 
 
 class Batch:
-    """Many independent trees stepped as one launch per step (optionally one
-    hipGraph launch for many steps); each keeps its own velocity and dt."""
+    """Many independent trees stepped together, a launch per step and group of
+    trees (optionally one hipGraph launch for many steps); each keeps its own
+    velocity and dt."""
 
     def __init__(self, trees):
         self.lib = load()

@@ -269,8 +269,9 @@ typedef struct amr_batch amr_batch;
 
 /* Concatenates the current state of `count` trees of the same rank, depth,
  * patch size and halo into one leaf list whose time steps run as one launch
- * over all leaves; every instance keeps its own velocity, cfl and dt (fixed
- * at creation from its finest level).  The trees are not modified until
+ * per group of instances (of up to 224 MiB of state; calls of one or two steps
+ * run over all leaves at once); every instance keeps its own velocity, cfl and
+ * dt (fixed at creation from its finest level).  The trees are not modified until
  * amr_batch_scatter. */
 int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out);
 int amr_batch_destroy(amr_batch* batch);
@@ -286,7 +287,8 @@ int amr_batch_synchronize(amr_batch* batch);
 int amr_batch_scatter(amr_batch* batch);
 int amr_batch_stream(amr_batch* batch, void** hip_stream);
 int amr_batch_set_step_variant(amr_batch* batch, int32_t variant);
-/* As amr_solver_autotune, over the whole batch. */
+/* As amr_solver_autotune, over the whole batch (every group is timed, best_us
+ * is the sum over the groups). */
 int amr_batch_autotune(amr_batch* batch, uint32_t trial_steps, int32_t* chosen, float* best_us);
 
 /* ---- discrete adjoint (no counterpart in the reference, which has no
@@ -315,7 +317,10 @@ typedef struct amr_tape_info
  * with k % regrid_every == 0 (criterion NULL or regrid_every 0: no regrid),
  * and records what the adjoint needs: each topology, the dt of every step,
  * every regrid's flags and leaf maps, and the state before every
- * checkpoint_every-th step.  The context ends at the final state. */
+ * checkpoint_every-th step.  An adjoint pass recomputes the states of one
+ * segment of checkpoint_every steps at a time, for which the tape holds
+ * checkpoint_every - 1 states (small trees of 2D 16^2 patches: twice as many, at
+ * most 128 MiB more).  The context ends at the final state. */
 int amr_tape_record(amr_ctx* ctx, const amr_criterion* criterion, uint64_t steps, uint64_t regrid_every,
                     uint64_t checkpoint_every, amr_tape** out);
 int amr_tape_destroy(amr_tape* tape);
