@@ -5,6 +5,7 @@ exact size: against the item bodies that the emulation tests pin to the oracle,
 and for the Euler equations a step in numpy, bit for bit (neither side
 contracts; the adjoint's velocity sums, whose order differs, to the rounding of
 a sum)."""
+import os
 import subprocess
 import types
 
@@ -46,7 +47,8 @@ def lanes(tmp_path, kind, rank, ext, table, arrays, reverse=0, count=None):
     with open(tmp_path / "in", "wb") as f:
         for a in (head, keys, links, metas, *(np.asarray(x, dtype=np.float64) for x in arrays)):
             f.write(np.ascontiguousarray(a).tobytes())
-    r = subprocess.run([str(BIN), str(tmp_path / "in"), str(tmp_path / "out")], capture_output=True, text=True)
+    r = subprocess.run([str(BIN), str(tmp_path / "in"), str(tmp_path / "out")], capture_output=True, text=True,
+                       env={**os.environ, "ASAN_OPTIONS": "verify_asan_link_order=0:detect_leaks=0"})
     assert r.returncode == 0, r.stderr[-3000:]
     return np.fromfile(tmp_path / "out", dtype=np.float64)
 
