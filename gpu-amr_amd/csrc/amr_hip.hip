@@ -1257,7 +1257,7 @@ struct amr_batch
     int                      variant = 0;
     uint64_t*                keys    = nullptr;
     face_link*               links   = nullptr; // neighbour slots count from the group's first leaf
-    face_link*               whole_links = nullptr; // from the batch's; with several groups only
+    face_link*               whole_links = nullptr; // from the batch's; where there is `whole`
     uint32_t*                metas   = nullptr;
     uint32_t*                inst    = nullptr;
     step_params*             table   = nullptr;
@@ -1278,7 +1278,7 @@ struct amr_batch
         run_lists        runs;
     };
     std::vector<std::unique_ptr<group>> groups;
-    group                               whole; // all leaves; with several groups only
+    std::unique_ptr<group>              whole; // all leaves, where there are several groups and memory
 
     // Calls of up to this many steps step the whole batch at once: a group
     // stepped once or twice finds little of itself in the cache, and one
@@ -1307,7 +1307,27 @@ struct amr_batch
         }
         for (size_t g = 0; g < groups.size(); ++g)
             groups[g]->leaves = (g + 1 < groups.size() ? groups[g + 1]->first : total) - groups[g]->first;
-        whole.leaves = total;
+    }
+
+    // Memory of the group of all leaves; without it, short calls step the
+    // groups too.
+    void allocate_whole()
+    {
+        if (groups.size() < 2) return;
+        auto w = std::make_unique<group>();
+        try
+        {
+            w->leaves = total;
+            w->links = whole_links = dev_alloc<face_link>(total * ndir);
+            if (run_lists::wanted(op)) w->runs.allocate(total);
+            whole = std::move(w);
+        }
+        catch (amr_error const&)
+        {
+            (void)hipGetLastError();
+            if (whole_links) (void)hipFree(whole_links);
+            whole_links = nullptr;
+        }
     }
     group& group_of(size_t instance)
     {
@@ -1358,8 +1378,8 @@ struct amr_batch
 
     void launch_steps(uint64_t steps)
     {
-        if (groups.size() > 1 && steps <= kWholeSteps)
-            launch_group(whole, steps);
+        if (whole && steps <= kWholeSteps)
+            launch_group(*whole, steps);
         else
             for (auto& g : groups) launch_group(*g, steps);
     }
@@ -2695,10 +2715,12 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
             b->keys  = dev_alloc<uint64_t>(b->total);
             b->links = dev_alloc<face_link>(b->total * b->ndir);
             b->metas = dev_alloc<uint32_t>(b->total * b->ndir);
-            if (b->groups.size() > 1) b->whole.links = b->whole_links = dev_alloc<face_link>(b->total * b->ndir);
             for (auto& g : b->groups) g->links = b->links + g->first * b->ndir;
             b->inst  = dev_alloc<uint32_t>(b->total);
             b->table = dev_alloc<step_params>(count);
+            if (run_lists::wanted(b->op))
+                for (auto& g : b->groups) g->runs.allocate(g->leaves);
+            b->allocate_whole();
             for (uint32_t i = 0; i < count; ++i)
             {
                 amr_ctx const* t = b->src[i];
@@ -2712,7 +2734,7 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
                 const uint64_t nl = t->n * b->ndir;
                 hipLaunchKernelGGL(k_offset_links, dim3(grid1d(nl, 256)), dim3(256), 0, b->stream, t->links,
                                    b->links + o * b->ndir, nl, static_cast<int32_t>(o - b->group_of(i).first));
-                if (b->whole_links)
+                if (b->whole)
                     hipLaunchKernelGGL(k_offset_links, dim3(grid1d(nl, 256)), dim3(256), 0, b->stream, t->links,
                                        b->whole_links + o * b->ndir, nl, static_cast<int32_t>(o));
                 hipLaunchKernelGGL(k_fill_instance, dim3(grid1d(t->n, 256)), dim3(256), 0, b->stream, b->inst + o, t->n,
@@ -2725,12 +2747,11 @@ int amr_batch_create(amr_ctx* const* trees, uint32_t count, amr_batch** out)
             if (run_lists::wanted(b->op))
             {
                 auto build_runs = [&](amr_batch::group& g) {
-                    g.runs.allocate(g.leaves);
                     g.runs.build(b->op->rank, b->keys + g.first, static_cast<uint32_t>(g.leaves), trees[0]->depth,
                                  g.links, b->metas + g.first * b->ndir, b->stream);
                 };
                 for (auto& g : b->groups) build_runs(*g);
-                if (b->whole_links) build_runs(b->whole);
+                if (b->whole) build_runs(*b->whole);
             }
             AMR_HIP_CHECK(hipStreamSynchronize(b->stream));
             *out = b.release();
